@@ -492,6 +492,25 @@ def _advect(case, f, mass):
     return 0.5 * (f + stage(stage(f)))
 
 
+class _BesselJ0:
+    """J0 on [0, top] by Taylor series about the multiples of 1/16, whose derivatives are Bessel's integral by the
+    trapezoid rule (torch's own is 4e-7 off near 5)."""
+
+    def __init__(self, top):
+        x = torch.arange(int(16 * top) + 2, dtype=torch.float64, device="cuda")[:, None] / 16
+        t = (torch.arange(512, dtype=torch.float64, device="cuda") + 0.5) * (2 * math.pi / 512)
+        s = torch.sin(t)[None]
+        self.d = [(s ** m * torch.cos(x * s + 0.5 * math.pi * m)).mean(1) / math.factorial(m) for m in range(9)]
+
+    def __call__(self, x):
+        i = (16 * x).round()
+        h, i = x - i / 16, i.long()
+        y = self.d[8][i]
+        for m in range(7, -1, -1):
+            y = y * h + self.d[m][i]
+        return y
+
+
 def _landau(case, seed):
     Lv = case["Lv"] * (1 + 0.05 * float(torch.rand(1, generator=torch.Generator().manual_seed(int(seed)))))
     e = torch.from_numpy(_grid(case, Lv)[1]).cuda()
@@ -503,6 +522,7 @@ def _landau(case, seed):
     n3 = E.shape[1]
     W = torch.zeros(n3, n3, dtype=torch.float64, device="cuda")
     z2 = E.square().sum(0)
+    j0 = _BesselJ0(Lv * math.sqrt(3) * float(e.abs().max()) + 1)
     step = max(1, (1 << 24) // n3)
     for a in range(0, n3, step):
         zz = z2[a:a + step, None]
@@ -516,7 +536,7 @@ def _landau(case, seed):
             for t in range(32):
                 s, c = math.sin(float(th[t])), math.cos(float(th[t]))
                 ph = r[i] * par * c
-                inner += tw[t] * s * torch.special.bessel_j0(r[i] * s * perp) * (-r[i] ** 2 * zz * s * s * torch.cos(ph) + 4 * r[i] * zl * c * torch.sin(ph))
+                inner += tw[t] * s * j0(r[i] * s * perp) * (-r[i] ** 2 * zz * s * s * torch.cos(ph) + 4 * r[i] * zl * c * torch.sin(ph))
             acc += rw[i] * inner
         W[a:a + step] = 2 * math.pi * acc
     return W
