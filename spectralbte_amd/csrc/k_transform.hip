@@ -137,7 +137,8 @@ __global__ void __launch_bounds__(XT) k_xform_a_cplx(int N, const double2 *__res
 // Pass B: x transform of the y-plane b; OUT = 0 double2, 1 float2, 2 real double.
 template <int OUT>
 __global__ void __launch_bounds__(XT) k_xform_b(int N, int ncell, const double2 *__restrict__ M, double pre,
-                                                const double2 *__restrict__ scratch, XformJobs jobs, void *out0) {
+                                                const double2 *__restrict__ scratch, XformJobs jobs, void *out0,
+                                                int npl) {
   extern __shared__ double2 sm[];
   const int n2 = N * N;
   const size_t n3 = (size_t)n2 * N;
@@ -146,7 +147,7 @@ __global__ void __launch_bounds__(XT) k_xform_b(int N, int ncell, const double2 
   double2 *P = sm;
   for (int e = threadIdx.x; e < n2; e += XT) {
     const int i = e / N, c = e - i * N;
-    P[e] = src[(size_t)i * n2 + b * N + c];
+    P[e] = i < npl ? src[(size_t)i * n2 + b * N + c] : make_double2(0.0, 0.0);
   }
   __syncthreads();
   void *dst = jobs.j[jb].dst ? jobs.j[jb].dst : out0;
@@ -429,7 +430,7 @@ template <int N, int OUT>
 __global__ void __launch_bounds__(XT) k_fft_b(int ncell, const double2 *__restrict__ tabs, double pre,
                                               const double2 *__restrict__ scratch, XformJobs jobs, void *out0,
                                               double dsgn, const double *__restrict__ v, const double *__restrict__ w,
-                                              double pm, double *__restrict__ ppart) {
+                                              double pm, double *__restrict__ ppart, int npl) {
   __shared__ double2 A[N * N], B[N * N];
   __shared__ FftTabs t;
   constexpr int n2 = N * N;
@@ -439,7 +440,7 @@ __global__ void __launch_bounds__(XT) k_fft_b(int ncell, const double2 *__restri
   const double2 *src = scratch + ((size_t)jb * ncell + cell) * n3;
   for (int e = threadIdx.x; e < n2; e += XT) {
     const int i = e / N, c = e - i * N;
-    A[e] = src[(size_t)i * n2 + b * N + c];
+    A[e] = i < npl ? src[(size_t)i * n2 + b * N + c] : make_double2(0.0, 0.0);
   }
   __syncthreads();
   double2 *r = fft_axis<N>(A, B, 1, N, t.tw, dsgn);        // x: sequences c, elements i (stride N)
@@ -779,7 +780,7 @@ template <int N, bool PROJ>
 __global__ void __launch_bounds__(XT) k_fft_cube_inv_x(int ncell, const double2 *__restrict__ tabs, double pre,
                                                        const double2 *__restrict__ scratch, double *__restrict__ q,
                                                        const double *__restrict__ v, const double *__restrict__ w,
-                                                       double pm, ProjArgs pa, spbte_epilogue ep) {
+                                                       double pm, ProjArgs pa, spbte_epilogue ep, int npl) {
   static_assert(N * N <= XT, "one line per thread");
   constexpr int n2 = N * N;
   constexpr size_t n3 = (size_t)n2 * N;
@@ -793,7 +794,7 @@ __global__ void __launch_bounds__(XT) k_fft_cube_inv_x(int ncell, const double2 
   load_tabs<N>(t, tabs);
   double2 x[N];
 #pragma unroll
-  for (int a = 0; a < N; ++a) x[a] = own ? scratch[cell * n3 + (size_t)a * n2 + tid] : make_double2(0.0, 0.0);
+  for (int a = 0; a < N; ++a) x[a] = own && a < npl ? scratch[cell * n3 + (size_t)a * n2 + tid] : make_double2(0.0, 0.0);
   // the update's a x + b y, loaded with the transform's input (every load
   // before the first store: out may alias x)
   double r[N];
@@ -857,29 +858,29 @@ void launch_fft_fwd(const spbte_grid_dev *g, const XformJobs &J, int njobs, int 
                      (const double *)g->d_w, (double2 *)scratch, -1.0, g->hv, g->mass, g->kb);
   if (out_fp32)
     hipLaunchKernelGGL((k_fft_b<N, 1>), dim3(N, ncell, njobs), dim3(XT), 0, s, ncell, tf, g->pre_fwd,
-                       (const double2 *)scratch, J, nullptr, -1.0, nullptr, nullptr, 0.0, nullptr);
+                       (const double2 *)scratch, J, nullptr, -1.0, nullptr, nullptr, 0.0, nullptr, N);
   else
     hipLaunchKernelGGL((k_fft_b<N, 0>), dim3(N, ncell, njobs), dim3(XT), 0, s, ncell, tf, g->pre_fwd,
-                       (const double2 *)scratch, J, nullptr, -1.0, nullptr, nullptr, 0.0, nullptr);
+                       (const double2 *)scratch, J, nullptr, -1.0, nullptr, nullptr, 0.0, nullptr, N);
 }
 
 // Complex cube transform (invert 0/1, OUT 0 = complex, 2 = real part, with
 // the projection's partials into ppart when it is not null).
 template <int N>
-void launch_fft_cplx(const spbte_grid_dev *g, const void *in, int nsl, void *out, int ncell, int invert, int real_out,
+void launch_fft_cplx(const spbte_grid_dev *g, const void *in, int nsl, int npl, void *out, int ncell, int invert, int real_out,
                      void *scratch, double *ppart, hipStream_t s) {
   const double2 *t = (const double2 *)g->d_fft + (invert ? 3 * N : 0);
   const double dsgn = invert ? 1.0 : -1.0, pre = invert ? g->pre_inv : g->pre_fwd;
   XformJobs J = {};
-  hipLaunchKernelGGL(k_fft_a_cplx<N>, dim3(N, ncell, 1), dim3(XT), 0, s, (const double2 *)in, nsl, ncell, t,
+  hipLaunchKernelGGL(k_fft_a_cplx<N>, dim3(npl, ncell, 1), dim3(XT), 0, s, (const double2 *)in, nsl, ncell, t,
                      (double2 *)scratch, dsgn);
   const double pm = g->hv * g->hv * g->hv * g->mass;
   if (real_out)
     hipLaunchKernelGGL((k_fft_b<N, 2>), dim3(N, ncell, 1), dim3(XT), 0, s, ncell, t, pre, (const double2 *)scratch, J,
-                       out, dsgn, (const double *)g->d_v, (const double *)g->d_w, pm, ppart);
+                       out, dsgn, (const double *)g->d_v, (const double *)g->d_w, pm, ppart, npl);
   else
     hipLaunchKernelGGL((k_fft_b<N, 0>), dim3(N, ncell, 1), dim3(XT), 0, s, ncell, t, pre, (const double2 *)scratch, J,
-                       out, dsgn, nullptr, nullptr, 0.0, nullptr);
+                       out, dsgn, nullptr, nullptr, 0.0, nullptr, npl);
 }
 
 // Grids with the whole-cube last pass (N^2 <= XT), used when a launch has at
@@ -901,18 +902,18 @@ bool with_cube_n(int N, F &&fn) {
 }
 
 template <int N>
-void launch_cube_inv(const spbte_grid_dev *g, const void *Qh, int nsl, double *q, int ncell, void *scratch,
+void launch_cube_inv(const spbte_grid_dev *g, const void *Qh, int nsl, int npl, double *q, int ncell, void *scratch,
                      const ProjArgs *pa, const spbte_epilogue &ep, hipStream_t s) {
   const double2 *t = (const double2 *)g->d_fft + 3 * N;  // inverse p, q, tw
-  hipLaunchKernelGGL(k_fft_a_cplx<N>, dim3(N, ncell, 1), dim3(XT), 0, s, (const double2 *)Qh, nsl, ncell, t,
+  hipLaunchKernelGGL(k_fft_a_cplx<N>, dim3(npl, ncell, 1), dim3(XT), 0, s, (const double2 *)Qh, nsl, ncell, t,
                      (double2 *)scratch, 1.0);
   const double *v = (const double *)g->d_v, *w = (const double *)g->d_w;
   if (pa)
     hipLaunchKernelGGL((k_fft_cube_inv_x<N, true>), dim3(ncell), dim3(XT), 0, s, ncell, t, g->pre_inv,
-                       (const double2 *)scratch, q, v, w, pa->pm[0], *pa, ep);
+                       (const double2 *)scratch, q, v, w, pa->pm[0], *pa, ep, npl);
   else
     hipLaunchKernelGGL((k_fft_cube_inv_x<N, false>), dim3(ncell), dim3(XT), 0, s, ncell, t, g->pre_inv,
-                       (const double2 *)scratch, q, v, w, 0.0, ProjArgs{}, ep);
+                       (const double2 *)scratch, q, v, w, 0.0, ProjArgs{}, ep, npl);
 }
 
 // Runs fn<N>() for the grid's N if it has FFT kernels; false otherwise.
@@ -973,17 +974,17 @@ extern "C" int spbte_launch_xform_fwd(const spbte_grid_dev *g, const spbte_xform
                      (const double2 *)g->d_mat_fwd, (const double *)g->d_v, (double2 *)scratch);
   if (out_fp32)
     hipLaunchKernelGGL(k_xform_b<1>, dim3(N, ncell, njobs), dim3(XT), lds_b, s, N, ncell, (const double2 *)g->d_mat_fwd,
-                       g->pre_fwd, (const double2 *)scratch, J, nullptr);
+                       g->pre_fwd, (const double2 *)scratch, J, nullptr, N);
   else
     hipLaunchKernelGGL(k_xform_b<0>, dim3(N, ncell, njobs), dim3(XT), lds_b, s, N, ncell, (const double2 *)g->d_mat_fwd,
-                       g->pre_fwd, (const double2 *)scratch, J, nullptr);
+                       g->pre_fwd, (const double2 *)scratch, J, nullptr, N);
   return (int)hipGetLastError();
 }
 
 extern "C" int spbte_launch_xform_fwd_complex(const spbte_grid_dev *g, const void *in, void *out, int ncell, int invert,
                                               void *scratch, hipStream_t s) {
   if (g->d_fft && with_fft_n(g->N, [&](auto n) {
-        launch_fft_cplx<decltype(n)::value>(g, in, 1, out, ncell, invert, 0, scratch, nullptr, s);
+        launch_fft_cplx<decltype(n)::value>(g, in, 1, g->N, out, ncell, invert, 0, scratch, nullptr, s);
       }))
     return (int)hipGetLastError();
   const int N = g->N;
@@ -993,25 +994,25 @@ extern "C" int spbte_launch_xform_fwd_complex(const spbte_grid_dev *g, const voi
   XformJobs J = {};
   hipLaunchKernelGGL(k_xform_a_cplx, dim3(N, ncell, 1), dim3(XT), lds_a, s, N, (const double2 *)in, ncell, M,
                      (double2 *)scratch);
-  hipLaunchKernelGGL(k_xform_b<0>, dim3(N, ncell, 1), dim3(XT), lds_b, s, N, ncell, M, pre, (const double2 *)scratch, J, out);
+  hipLaunchKernelGGL(k_xform_b<0>, dim3(N, ncell, 1), dim3(XT), lds_b, s, N, ncell, M, pre, (const double2 *)scratch, J, out, N);
   return (int)hipGetLastError();
 }
 
-extern "C" int spbte_launch_xform_inv_real(const spbte_grid_dev *g, const void *Qh, int nsl, double *q, int ncell,
+extern "C" int spbte_launch_xform_inv_real(const spbte_grid_dev *g, const void *Qh, int nsl, int npl, double *q, int ncell,
                                            void *scratch, double *proj_part, hipStream_t s) {
-  if (nsl < 1) return (int)hipErrorInvalidValue;
+  if (nsl < 1 || npl < 1 || npl > g->N) return (int)hipErrorInvalidValue;
   if (g->d_fft && with_fft_n(g->N, [&](auto n) {
-        launch_fft_cplx<decltype(n)::value>(g, Qh, nsl, q, ncell, 1, 1, scratch, proj_part, s);
+        launch_fft_cplx<decltype(n)::value>(g, Qh, nsl, npl, q, ncell, 1, 1, scratch, proj_part, s);
       }))
     return (int)hipGetLastError();
   if (proj_part || nsl != 1) return (int)hipErrorInvalidValue;  // the matrix form takes one set, writes no partials
   const int N = g->N;
   const size_t lds_a = 2 * (size_t)N * N * sizeof(double2), lds_b = (size_t)N * N * sizeof(double2);
   XformJobs J = {};
-  hipLaunchKernelGGL(k_xform_a_cplx, dim3(N, ncell, 1), dim3(XT), lds_a, s, N, (const double2 *)Qh, ncell,
+  hipLaunchKernelGGL(k_xform_a_cplx, dim3(npl, ncell, 1), dim3(XT), lds_a, s, N, (const double2 *)Qh, ncell,
                      (const double2 *)g->d_mat_inv, (double2 *)scratch);
   hipLaunchKernelGGL(k_xform_b<2>, dim3(N, ncell, 1), dim3(XT), lds_b, s, N, ncell, (const double2 *)g->d_mat_inv,
-                     g->pre_inv, (const double2 *)scratch, J, (void *)q);
+                     g->pre_inv, (const double2 *)scratch, J, (void *)q, npl);
   return (int)hipGetLastError();
 }
 
@@ -1087,14 +1088,14 @@ extern "C" int spbte_fft_cube(int N, int ncubes) {
   return ncubes >= 1 && ncubes <= kCubeMaxWg && with_cube_n(N, [](auto) {}) ? 1 : 0;
 }
 
-extern "C" int spbte_launch_xform_inv_real_cube(const spbte_grid_dev *g, const void *Qh, int nsl, double *q, int ncell,
+extern "C" int spbte_launch_xform_inv_real_cube(const spbte_grid_dev *g, const void *Qh, int nsl, int npl, double *q, int ncell,
                                                 void *scratch, const double *masses, const double *LU, const int *pivot,
                                                 const spbte_epilogue *epi, hipStream_t s) {
-  if (nsl < 1 || !g->d_fft || !spbte_fft_cube(g->N, ncell)) return (int)hipErrorInvalidValue;
+  if (nsl < 1 || npl < 1 || npl > g->N || !g->d_fft || !spbte_fft_cube(g->N, ncell)) return (int)hipErrorInvalidValue;
   const ProjArgs pa = masses ? proj_args(g, 1, masses, LU, pivot) : ProjArgs{};
   const spbte_epilogue ep = epi ? *epi : spbte_epilogue{};
   with_cube_n(g->N, [&](auto n) {
-    launch_cube_inv<decltype(n)::value>(g, Qh, nsl, q, ncell, scratch, masses ? &pa : nullptr, ep, s);
+    launch_cube_inv<decltype(n)::value>(g, Qh, nsl, npl, q, ncell, scratch, masses ? &pa : nullptr, ep, s);
   });
   return (int)hipGetLastError();
 }

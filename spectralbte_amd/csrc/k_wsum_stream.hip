@@ -23,10 +23,24 @@
 //    wave-wide load reads 1 KiB of contiguous HBM, in consumption order.
 // Precision forms: 0 FP64 W, 1 FP32 W, 2 FP16x2 W with FP64 arithmetic; 3 FP32 W
 // with FP32 F, G (8-byte LDS entries, half the LDS), FP32 products and FP32
-// partial sums added into FP64 accumulators every 32 steps in 8-step loop
-// bodies (N=32, N=16) and every 8 steps in longer ones (N=24).  Folding every
-// 4 steps cost 6% more time on the 512-problem N=32 batch for a largest
-// error against FP64 of 2.5e-7 instead of 2.9e-7.
+// partial sums added into FP64 accumulators every 8 steps.  Over 3 Heun steps of
+// 48 N=32 problems (lambda=1, L_v=8.5) the state is 1.30e-9 off the FP64 form's,
+// 1.64e-9 with 32-step partial sums, for 2% of the time (512 problems: 38650 us
+// against 37870); the sum over the whole table with 32 steps was 1.36e-9 off.
+//
+// Folded tables (k_fold_w below).  Cells are real and only the real part of the
+// inverse transform is kept, so half of the output modes determine Q, and in
+// Q(f, f) the modes c and s(r, c) enter alike, so half of the summed ones do: the
+// kernel then runs over N/2 + 1 of N x-planes of rows and N/2 or N/2 + 1
+// x-planes of columns (0.274 of the table at N=32, 0.293 at N=24, 0.299 at N=16),
+// or over the rows' half alone for two different cells.  The inner loop is the
+// same; every form gains by the smaller table (MI355X, one evaluation, before and
+// after): N=32 512 problems with FP32 products 140.7 -> 40.5 ms, 256 cells
+// ComputeQ FP64 67.8 -> 18.0, one cell FP64 (HBM-bound) 1.25 -> 0.44; N=24 37
+// cells FP64 2.94 -> 0.74; N=16 48 cells, two different arguments, 0.60 -> 0.19.
+// Whole planes are kept because every lane of a wave shares c and its G: the
+// self-paired planes (two of cx, in half of the row planes; rx = 0 and N/2) cost
+// 6-10% more than the exact half of each.
 #include <hip/hip_runtime.h>
 #include <type_traits>
 #include "spbte_internal.h"
@@ -41,7 +55,6 @@ struct SGeom {
   static constexpr int RW = 64 * TR;                 // rows per wave tile
   static constexpr int RWG = WAVES * RW;             // rows per workgroup
   static constexpr int N2 = N * N;
-  static constexpr int NC4 = N * N * N / 4;          // 4-column groups per row
   // x-planes of output rows a workgroup can touch: RWG / N2 when workgroups
   // tile whole planes, 1 when they tile within a plane, else the most planes a
   // run of RWG consecutive rows can straddle
@@ -112,11 +125,13 @@ template <int N, int TR, int WAVES, int TB, int NP, int FORM, bool NTW, int CPW>
 __global__ void __launch_bounds__(64 * WAVES * CPW) __attribute__((amdgpu_waves_per_eu(kWavesPerEU<TR, WAVES, TB, FORM>)))
 k_wsum_stream(const uint4 *__restrict__ Wp, const float *__restrict__ rowscale, const double2 *__restrict__ F0,
               const double2 *__restrict__ G0, const double2 *__restrict__ F1, const double2 *__restrict__ G1,
-              double2 *__restrict__ Qh, int ncell, int csplit, double2 *__restrict__ Qp) {
+              double2 *__restrict__ Qh, int ncell, int csplit, double2 *__restrict__ Qp, int npl, int fold) {
   using Gm = SGeom<N, TR, WAVES>;
-  constexpr int N2 = Gm::N2, P = Gm::P, RWG = Gm::RWG, NC4 = Gm::NC4;
+  constexpr int N2 = Gm::N2, P = Gm::P, RWG = Gm::RWG;
   constexpr size_t n3 = (size_t)N * N * N;
-  constexpr int NRT = (int)(n3 / RWG);                  // r-tiles
+  const int NRT = npl * N2 / RWG;                       // r-tiles
+  const int cfold = fold & 1;                           // fold: 0 whole table, 2 rows folded, 3 columns too
+  const int NC4 = (cfold ? N / 2 + 1 : N) * (N2 / 4);   // 4-column groups per table row
   constexpr int UPW = (FORM == 0) ? 2 : 1;              // 16-byte units per 4 weights
   // F, G elements: FP32 complex in the FP32-product form (products and
   // partial sums in FP32, folded into the FP64 accumulators), else FP64
@@ -156,12 +171,6 @@ k_wsum_stream(const uint4 *__restrict__ Wp, const float *__restrict__ rowscale, 
   if ((blockIdx.x >> 3) >= per || vid >= total) return;  // the few padding workgroups of the last slice
   const int rt = vid / (csplit * ncg), rem = vid - rt * (csplit * ncg);
   const int cs = rem / ncg, cg = rem - cs * ncg;
-  // slices: up to N take whole x-planes (N / csplit each); beyond N every
-  // x-plane's summed y-lines are split as well (csplit / N pieces of it)
-  const int ny = csplit > N ? csplit / N : 1;
-  const int cx0 = csplit > N ? cs / ny : cs * (N / csplit);
-  const int cx1 = csplit > N ? cx0 + 1 : cx0 + N / csplit;
-  const int cy0 = csplit > N ? (cs - cx0 * ny) * (N / ny) : 0, cy1 = cy0 + N / ny;
   // wave and cell group are wave-uniform: say so, so that the cell's G lines
   // stay scalar loads
   const int lane = threadIdx.x & 63;
@@ -173,6 +182,14 @@ k_wsum_stream(const uint4 *__restrict__ Wp, const float *__restrict__ rowscale, 
   const int rx = (int)(row0 / N2), ry = (int)((row0 / N) % N), rz0 = (int)(row0 % N);
   const int pl = rx - rx0;                               // this lane's plane in LDS
   const int k0 = (rz0 + N / 2) % N;                      // window start at cz = 0 (non-negative)
+  // summed x-planes: all N from 0, or, folded (one x-plane of rows per
+  // workgroup), one of every pair cx, rx + N/2 - cx (mod N); the slice's share
+  // of their z-lines is [l0, l1)
+  const int m = cfold ? (rx0 + N / 2) % N : 0;
+  const int ncx = cfold ? N / 2 + 1 - (m & 1) : N;
+  const int cxs = cfold ? (m + 1) / 2 + ncx - 1 : 0;     // the outermost first (k_fold_w)
+  const int nl = ncx * N;
+  const int l0 = (int)((long)cs * nl / csplit), l1 = (int)((long)(cs + 1) * nl / csplit);
   const size_t wt = (size_t)rt * WAVES + wave;           // wave tile of the permuted table
 
   const C *Fp[2] = {(const C *)F0, (const C *)F1};
@@ -212,12 +229,50 @@ k_wsum_stream(const uint4 *__restrict__ Wp, const float *__restrict__ rowscale, 
         else u[t][h] = *q;
       }
   };
+  // Adds the accumulators to the result (add: there is one already) and clears
+  // them.  With FP64 sums this is done after every x-plane: one accumulator over
+  // a whole slice rounds every small term at the full size of the gain and loss
+  // sums, 9-10e-13 of Q on a layer cell of the N=32 shock batch (1.2e-12 for the
+  // unfolded sum).  Together with the order of the folded table's z-lines
+  // (k_fold_w) it is 3.6e-13.  In the lines' natural order that took a store every
+  // 4 lines, whose 16-byte read-modify-writes cost 9% of the sum (256 cells
+  // ComputeQ: 19120 us against 17530).
+  int sums = 0;
+  auto store = [&](bool add) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < TB; ++b) {
+      const int cell = cg * KB + grp * TB + b;
+      if (cell < ncell) {
+        double2 *o = (csplit > 1 ? Qp + ((size_t)cs * ncell + cell) * n3 : Qh + (size_t)cell * n3) + row0;
+#pragma unroll
+        for (int t = 0; t < TR; ++t) {
+          double2 s = acc[b][t];
+          if constexpr (FORM == 2) {  // a power of two
+            const double sc = (double)rowscale[row0 + t];
+            s.x *= sc;
+            s.y *= sc;
+          }
+          if (add) {
+            const double2 q = o[t];
+            s.x += q.x;
+            s.y += q.y;
+          }
+          o[t] = s;
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < TR; ++t) acc[b][t] = make_double2(0.0, 0.0);
+    }
+  };
+
   // Two static register sets alternate over the 4-column chunks of W (a body
   // holds an even number of chunks), each loaded four cz steps before use.
   u32x4 wA[TR][UPW], wB[TR][UPW];
-  wload((cx0 * N + cy0) * (N / 4), wA);
+  wload(l0 * (N / 4), wA);
 
-  for (int cx = cx0; cx < cx1; ++cx) {
+  for (int ln0 = l0; ln0 < l1; ln0 = (ln0 / N + 1) * N) {  // z-lines ln0 .. of one x-plane
+    const int cx = cfold ? (cxs - ln0 / N) % N : ln0 / N;
+    const int cy0 = ln0 % N, cy1 = l1 - ln0 < N - cy0 ? cy0 + l1 - ln0 : N;
     __syncthreads();
     // ---- stage the shifted F x-planes of every cell, product and lane plane,
     // each z-line extended to LW values (entry m = F[(m - BS) mod N])
@@ -246,7 +301,9 @@ k_wsum_stream(const uint4 *__restrict__ Wp, const float *__restrict__ rowscale, 
       }
     __syncthreads();
 
-    for (int cy = cy0; cy < cy1; ++cy) {
+    for (int cl = cy0; cl < cy1; ++cl) {
+      // line slot -> cy: a folded table's lines go from the outermost to the middle
+      const int cy = fold ? ((cl & 1) ? N - 1 - cl / 2 : cl / 2) : cl;
       int sy = ry + N / 2 - cy;
       sy = sy < 0 ? sy + N : (sy > N - 1 ? sy - N : sy);
       const C *line[NP][TB];
@@ -273,8 +330,7 @@ k_wsum_stream(const uint4 *__restrict__ Wp, const float *__restrict__ rowscale, 
             buf[p][b][t] = line[p][b][Gm::pos(BS + ((k0 + t) % N))];
             if constexpr (GS) bufP[p][b][t] = lineP[p][b][Gm::pos(BS + ((k0 + t) % N))];
           }
-      const int c4base = (cx * N + cy) * (N / 4);
-      bool fold_body = true;
+      const int c4base = (ln0 + cl - cy0) * (N / 4);
       // One 4-step chunk at body offset jb (a compile-time constant after
       // unrolling): wc holds its weights, wn receives the next chunk's.  `fl`
       // points at the refill entry of body step 0: line + BS + (k0 - 1 - cz_body) mod N.
@@ -357,7 +413,7 @@ k_wsum_stream(const uint4 *__restrict__ Wp, const float *__restrict__ rowscale, 
           }
         }
         if constexpr (FORM == 3) {
-          if ((jb + 4) % 8 != 0 || !fold_body) return;  // 8 (32 in 8-step bodies) steps per FP32 partial sum
+          if ((jb + 4) % 8 != 0) return;  // 8 steps per FP32 partial sum
           // fold the FP32 partial sums into FP64
 #pragma unroll
           for (int b = 0; b < TB; ++b)
@@ -399,9 +455,6 @@ k_wsum_stream(const uint4 *__restrict__ Wp, const float *__restrict__ rowscale, 
             gz[p][b] = SG ? Gp[p] + go : sG + (size_t)(p * KB + grp * TB + b) * N2 + (size_t)cy * N + it * BS;
             gzs[p][b] = GS ? Gsum[p] + go : nullptr;
           }
-        // 8-step bodies fold every fourth body (32-term partial sums), longer
-        // bodies every 8 steps; the last body of a line always folds
-        fold_body = (BS >= 16) || ((it & 3) == 3) || (it == N / BS - 1);
 #pragma unroll
         for (int k = 0; k < BS / 4; k += 2) {
           const int c4 = c4base + it * (BS / 4) + k;
@@ -411,24 +464,11 @@ k_wsum_stream(const uint4 *__restrict__ Wp, const float *__restrict__ rowscale, 
         base = base - BS + N;
       }
     }
+    if constexpr (FORM != 3)
+      if (ln0 - cy0 + cy1 < l1) store(sums++ > 0);
   }
 
-#pragma unroll
-  for (int b = 0; b < TB; ++b) {
-    const int cell = cg * KB + grp * TB + b;
-    if (cell >= ncell) continue;
-#pragma unroll
-    for (int t = 0; t < TR; ++t) {
-      double2 s = acc[b][t];
-      if constexpr (FORM == 2) {
-        const double sc = (double)rowscale[row0 + t];
-        s.x *= sc;
-        s.y *= sc;
-      }
-      if (csplit > 1) Qp[((size_t)cs * ncell + cell) * n3 + row0 + t] = s;
-      else Qh[(size_t)cell * n3 + row0 + t] = s;
-    }
-  }
+  store(sums > 0);
 }
 
 // Qh[b][r] = sum over the csplit slices of Qp[s][b][r].
@@ -449,10 +489,12 @@ template <int N, int TR, int WAVES, int TB, int NP, int FORM, int CPW>
 int launch_s(const spbte_wsum_args *a, const void *Wp, const float *rowscale, int csplit, void *Qp, hipStream_t s) {
   using Gm = SGeom<N, TR, WAVES>;
   const int ncg = (a->ncell + TB * CPW - 1) / (TB * CPW);
-  const int nrt = (int)((size_t)N * N * N / Gm::RWG);
+  const int npl = a->npl ? a->npl : N, cfold = a->cfold;
+  if ((npl != N || cfold) && (N * N) % Gm::RWG != 0) return (int)hipErrorInvalidValue;  // one x-plane of rows per workgroup
+  const int nrt = npl * N * N / Gm::RWG;
   const int per = (nrt * csplit * ncg + 7) / 8;  // workgroups per XCD slice
-  constexpr size_t n3 = (size_t)N * N * N, kCacheResident = (size_t)160 << 20;
-  constexpr bool resident = n3 * n3 * (FORM == 0 ? 8 : 4) <= kCacheResident;
+  constexpr size_t n2 = (size_t)N * N, kCacheResident = (size_t)160 << 20;
+  const bool resident = npl * n2 * (cfold ? N / 2 + 1 : N) * n2 * (FORM == 0 ? 8 : 4) <= kCacheResident;
   bool nt = false;
   if constexpr (CPW == 1) nt = ncg == 1 && !resident;  // every W element read once: non-temporal loads
   if constexpr (CPW == 1)
@@ -460,12 +502,12 @@ int launch_s(const spbte_wsum_args *a, const void *Wp, const float *rowscale, in
       hipLaunchKernelGGL((k_wsum_stream<N, TR, WAVES, TB, NP, FORM, true, 1>), dim3(8 * per), dim3(64 * WAVES), 0, s,
                          (const uint4 *)Wp, rowscale, (const double2 *)a->F0, (const double2 *)a->G0,
                          (const double2 *)a->F1, (const double2 *)a->G1, (double2 *)a->Qh, a->ncell, csplit,
-                         (double2 *)Qp);
+                         (double2 *)Qp, npl, npl != N || cfold ? 2 + cfold : 0);
   if (!nt)
     hipLaunchKernelGGL((k_wsum_stream<N, TR, WAVES, TB, NP, FORM, false, CPW>), dim3(8 * per), dim3(64 * WAVES * CPW), 0,
                        s, (const uint4 *)Wp, rowscale, (const double2 *)a->F0, (const double2 *)a->G0,
                        (const double2 *)a->F1, (const double2 *)a->G1, (double2 *)a->Qh, a->ncell, csplit,
-                       (double2 *)Qp);
+                       (double2 *)Qp, npl, npl != N || cfold ? 2 + cfold : 0);
   if (csplit > 1 && !a->keep_slices) {
     const size_t n = (size_t)a->ncell * N * N * N;
     hipLaunchKernelGGL(k_slice_sum, dim3((unsigned)((n + 255) / 256 < 16384 ? (n + 255) / 256 : 16384)), dim3(256), 0,
@@ -551,6 +593,77 @@ __global__ void __launch_bounds__(256) k_permute_w(const double *__restrict__ W,
   }
 }
 
+// Natural FP64 table -> folded permuted copy (form 0: FP64, else FP32), units
+// as in k_permute_w over the kept rows (x-planes rx < npl) and the kept columns.
+//  * Row fold (mr.on): the inverse transform keeps the real part, and the
+//    operands are transforms of real cells, X[k'] = S(k) conj X[k] with
+//    k' = (2 (N/2) - k) mod N per axis.  The rows r and r' then enter as
+//    Qhat[r] + R(r) conj Qhat[r'], whose second term is the sum over the same
+//    (c, s(r, c)) with W[r'][c'] R(r) S(c) S(s): one row of
+//    W[r][c] + R(r) S(c) S(s) W[r'][c'] serves both.  Kept are rx <= N/2; a
+//    plane that is its own mirror image keeps its rows as they are.
+//  * Column fold (cfold): where the summed products are symmetric under
+//    c <-> s(r, c), the column c carries the weight of both.  With
+//    m = (rx + N/2) mod N (even N) the kept planes are cx = ceil(m/2) to
+//    ceil(m/2) + N/2 - (m odd), mod N, the last of them first.  Planes with
+//    2 cx = m (mod N) are their own partners and stay whole.
+// The z-lines of a plane go from the outermost cy to the middle ones, as the
+// planes do: the operands decay away from the middle of the grid, so the large
+// terms of a plane are added last and few additions round at its full size.
+// Both identities hold for any table; nothing is assumed of W.
+__global__ void __launch_bounds__(256) k_fold_w(const double *__restrict__ W, void *__restrict__ out, int form, int TR,
+                                                int N, int npl, int cfold, spbte_mirror mr) {
+  const int n2 = N * N, h = N / 2, ncp = cfold ? N / 2 + 1 : N;
+  const size_t n3 = (size_t)n2 * N, nc4 = (size_t)ncp * n2 / 4;
+  const size_t total = (size_t)npl * n2 * nc4;
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
+    const size_t lane = i % 64, q1 = i / 64;
+    const size_t t = q1 % TR, q2 = q1 / TR;
+    const size_t c4 = q2 % nc4, wtile = q2 / nc4;
+    const size_t row = (wtile * 64 + lane) * TR + t;
+    const int rx = (int)(row / n2), ry = (int)(row / N % N), rz = (int)(row % N);
+    const int j = (int)(c4 * 4 / n2), cl = (int)(c4 * 4 / N % N), cz0 = (int)(c4 * 4 % N);
+    const int cy = (cl & 1) ? N - 1 - cl / 2 : cl / 2;
+    const int m = (rx + h) % N;
+    const int ncx = cfold ? N / 2 + 1 - (m & 1) : N;
+    const bool used = j < ncx;
+    const int cx = cfold && used ? ((m + 1) / 2 + ncx - 1 - j) % N : j % N;
+    const int sx = (rx + h - cx + N) % N, sy = (ry + h - cy + N) % N;
+    const bool pair = cfold && sx != cx;
+    const int a2 = 2 * h;
+    const int mx = (a2 - rx + N) % N, my = (a2 - ry + N) % N, mz = (a2 - rz + N) % N;
+    const bool mir = mr.on && mx != rx;
+    const size_t rowm = ((size_t)mx * N + my) * N + mz;
+    const double R = mir ? mr.r[rx] * mr.r[ry] * mr.r[rz] : 0.0;
+    double w[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int cz = cz0 + k, sz = (rz + h - cz + N) % N;
+      double x = 0.0;
+      if (used) {
+        const size_t c = ((size_t)cx * N + cy) * N + cz, s = ((size_t)sx * N + sy) * N + sz;
+        x = W[row * n3 + c];
+        if (pair) x += W[row * n3 + s];
+        if (mir) {
+          const double sg = R * mr.s[cx] * mr.s[cy] * mr.s[cz] * mr.s[sx] * mr.s[sy] * mr.s[sz];
+          const size_t cm = ((size_t)((a2 - cx + N) % N) * N + (a2 - cy + N) % N) * N + (a2 - cz + N) % N;
+          double y = W[rowm * n3 + cm];
+          if (pair) y += W[rowm * n3 + ((size_t)((a2 - sx + N) % N) * N + (a2 - sy + N) % N) * N + (a2 - sz + N) % N];
+          x += sg * y;
+        }
+      }
+      w[k] = x;
+    }
+    if (form == 0) {
+      double2 *o = (double2 *)out;
+      o[((wtile * nc4 + c4) * TR + t) * 128 + lane] = make_double2(w[0], w[1]);
+      o[((wtile * nc4 + c4) * TR + t) * 128 + 64 + lane] = make_double2(w[2], w[3]);
+    } else {
+      ((float4 *)out)[i] = make_float4((float)w[0], (float)w[1], (float)w[2], (float)w[3]);
+    }
+  }
+}
+
 }  // namespace
 
 extern "C" int spbte_csplit_valid(int N, int csplit) {
@@ -570,7 +683,7 @@ extern "C" int spbte_stream_tile_supported(int N, int form, int nprod, int tr, i
 extern "C" int spbte_launch_wsum_stream(int N, int form, int tr, int waves, int tb, const spbte_wsum_args *a, const void *Wp,
                                         const float *rowscale, int csplit, void *Qp, hipStream_t s) {
   const SEntry *e = sfind(N, form, a->nprod, tr, waves, tb);
-  if (!e || !spbte_csplit_valid(N, csplit) || (csplit > 1 && !Qp)) return (int)hipErrorInvalidValue;
+  if (!e || csplit < 1 || (csplit > 1 && !Qp)) return (int)hipErrorInvalidValue;
   return e->fn(a, Wp, rowscale, csplit, Qp, s);
 }
 
@@ -579,5 +692,20 @@ extern "C" int spbte_launch_permute_weights(const double *W64, void *dst, const 
                                             hipStream_t s) {
   if (TR < 1 || n3 % (64 * (size_t)TR) || n3 % 4) return (int)hipErrorInvalidValue;
   hipLaunchKernelGGL(k_permute_w, dim3(8192), dim3(256), 0, s, W64, dst, rowscale, form, TR, n3);
+  return (int)hipGetLastError();
+}
+
+// 1 if the tile's workgroups each stay within one x-plane of output rows, as
+// folded tables need.
+extern "C" int spbte_stream_tile_folds(int N, int tr, int waves) {
+  const int w = waves == 16 ? 4 : waves;  // the 16-wave tile: four groups on the rows of one 4-wave tile
+  return N % 2 == 0 && (N * N) % (64 * tr * w) == 0;
+}
+
+// Folded table for tiles of TR rows per lane: form 0 FP64, 1 FP32.
+extern "C" int spbte_launch_fold_weights(const double *W64, void *dst, int form, int TR, int N, int npl, int cfold,
+                                         const spbte_mirror *mr, hipStream_t s) {
+  if (TR < 1 || N % 4 || (N * N) % (64 * TR) || form < 0 || form > 1) return (int)hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_fold_w, dim3(8192), dim3(256), 0, s, W64, dst, form, TR, N, npl, cfold, *mr);
   return (int)hipGetLastError();
 }

@@ -68,6 +68,7 @@ struct spbte_op {
     double *dW64;      /* FP64 master copy */
     void *dWf[NFORMS]; /* [0] aliases dW64; [1] float (forms 1, 3); [2] (hi,lo) pairs + row scales */
     void *dWp[3][9];   /* tables permuted for the streaming kernel, per storage form and rows per lane */
+    void *dWh[2][2][9]; /* the same folded (k_fold_w): [columns folded too][storage form FP64, FP32][rows per lane] */
     int have_w;
   } tab[SPBTE_MAX_NS * SPBTE_MAX_NS], *t;
   /* conservation */
@@ -93,6 +94,9 @@ struct spbte_op {
   void *nac;
   size_t nac_bytes;
   int nac_err; /* hipError_t of resolving it */
+  spbte_mirror mirror; /* of the transforms on this grid (on: folded tables hold half the rows) */
+  double *d_tab;       /* the grid's device tables (pointers into it in g) */
+  double *d_sym;       /* of them, mirror.on: build_mirror's factors and matrices */
   /* bumped whenever a device buffer, the table, the species or a tile changes:
    * launch sequences captured in a graph are valid for one generation */
   unsigned gen;
@@ -176,6 +180,77 @@ static void build_fft_factors(int N, const double *a, double delta, double Lstar
     out[2 * (2 * N + j)] = (double)cosl(th);
     out[2 * (2 * N + j) + 1] = (double)sinl(th);
   }
+}
+
+/* The transforms with the mirror symmetry of real cells exact to the last bit:
+ * with k' = (2h - k) mod N, h = N/2 (rounded down), conj Mf[k][j] = s(k) Mf[k'][j]
+ * and conj Mi[j][k] / w_k = t(k) Mi[j][k'] / w_k', signs s, t (-1 at the mode
+ * -N/2 of an even N, which is its own mirror image).  The reference's phases
+ * keep it to about 1e-13 only: its factor exp(i j L_eta h_v) is (-1)^j times
+ * exp(i j eps), eps the rounding of L_eta h_v.  Here the part of each phase that
+ * is odd under k <-> k' is kept as it is and the even part is the exact one.
+ * That turns f into f exp(i eps j), so Q by i eps times a real function, which
+ * the real part drops: the results agree to eps^2.  Taken instead with the
+ * reference's phases, the folded sums were 3.6e-14 off (relative, N=16) where
+ * the unfolded ones are 2.8e-15.
+ * out: forward p, q, twiddles, inverse p, q, twiddles (N complex each), then
+ * both matrices.  Returns 1 if the grid has the symmetry: the matrices within
+ * 1e-12 of the given ones (the 1D grids of odd N and a caller's own may not). */
+static int build_mirror(int N, const double *eta, double Lv, double heta, const double *w, const double *Mf,
+                        const double *Mi, double *out /* 2 (6N + 2N^2) */, spbte_mirror *mr) {
+  const long double pi = 3.141592653589793238462643383279502884L;
+  const int h = N / 2;
+  double *p = out, *q = out + 2 * N, *pi_ = out + 6 * N, *qi = out + 8 * N, *mf = out + 12 * N, *mi = mf + 2 * N * N;
+  long double a[SPBTE_MAX_N], c[SPBTE_MAX_N];
+  for (int k = 0; k < N; k++) {
+    const int km = (2 * h - k + N) % N;
+    a[k] = (long double)Lv * ((long double)eta[k] - (long double)eta[km]) / 2;
+    c[k] = -(long double)(k - h) * (long double)Lv * heta;
+    mr->s[k] = mr->r[k] = 1.0;
+    if (km == k) { /* its own image: the phase is a quarter turn's multiple */
+      const long na = lroundl((long double)Lv * eta[k] / (pi / 2)), nc = lroundl(c[k] / (pi / 2));
+      a[k] = na * (pi / 2);
+      c[k] = nc * (pi / 2);
+      mr->s[k] = na % 2 ? -1.0 : 1.0;
+      mr->r[k] = nc % 2 ? -1.0 : 1.0;
+    }
+    mr->r[k] *= w[km] / w[k];
+  }
+  long double f[SPBTE_MAX_N][8], tw[SPBTE_MAX_N][2]; /* p, q forward, p, q inverse; exp(2 pi i j / N) */
+  for (int j = 0; j < N; j++) {
+    const long double b = 2.0L * pi * ((j * h) % N) / N, t = 2.0L * pi * j / N;
+    tw[j][0] = cosl(t);
+    tw[j][1] = sinl(t);
+    f[j][0] = cosl(b) * w[j];
+    f[j][1] = sinl(b) * w[j];
+    f[j][2] = cosl(a[j]);
+    f[j][3] = sinl(a[j]);
+    f[j][4] = cosl(c[j]) * w[j];
+    f[j][5] = sinl(c[j]) * w[j];
+    f[j][6] = cosl(b);
+    f[j][7] = -sinl(b);
+    for (int z = 0; z < 2; z++) {
+      p[2 * j + z] = (double)f[j][z];
+      q[2 * j + z] = (double)f[j][2 + z];
+      pi_[2 * j + z] = (double)f[j][4 + z];
+      qi[2 * j + z] = (double)f[j][6 + z];
+      out[10 * N + 2 * j + z] = (double)tw[j][z];
+      out[4 * N + 2 * j + z] = (double)(z ? -tw[j][1] : tw[j][0]);
+    }
+  }
+  double dev = 0.0;
+  for (int d = 0; d < 2; d++) /* M[r][s] = q[r] exp(-+2 pi i r s / N) p[s] */
+    for (int r = 0; r < N; r++)
+      for (int s = 0; s < N; s++) {
+        const long double *q1 = f[r] + 4 * d + 2, *p1 = f[s] + 4 * d, *t = tw[(r * s) % N], ti = d ? t[1] : -t[1];
+        const long double x = q1[0] * p1[0] - q1[1] * p1[1], y = q1[0] * p1[1] + q1[1] * p1[0];
+        double *m = (d ? mi : mf) + 2 * (r * N + s);
+        const double *g = (d ? Mi : Mf) + 2 * (r * N + s);
+        m[0] = (double)(x * t[0] - y * ti);
+        m[1] = (double)(x * ti + y * t[0]);
+        dev = fmax(dev, fmax(fabs(m[0] - g[0]), fabs(m[1] - g[1])));
+      }
+  return dev <= 1e-12; /* false for NaN */
 }
 
 /* ---------------------------------------------- LU (src/conserve.c:89-168) */
@@ -292,35 +367,35 @@ int spbte_op_create(spbte_op **out, int N, double L_v, const double *v, const do
   const double scale3 = pow(1.0 / sqrt(2.0 * M_PI), 3.0); /* src/collisions.c:46 */
   g->pre_fwd = scale3 * g->hv * g->hv * g->hv;
   g->pre_inv = scale3 * g->heta * g->heta * g->heta;
-  double *Mf = malloc(sizeof(double) * 2 * N * N), *Mi = malloc(sizeof(double) * 2 * N * N), w[SPBTE_MAX_N];
-  if (!Mf || !Mi) {
-    free(Mf);
-    free(Mi);
+  /* one device buffer: both matrices, FFT factors, the mirror-symmetric set of
+   * all of these, v, w */
+  const size_t n2 = (size_t)N * N, nset = 2 * (6 * N + 2 * n2), ntab = 2 * nset + 2 * N;
+  double *tab = malloc(sizeof(double) * ntab);
+  if (!tab) {
     spbte_op_destroy(op);
     return fail(SPBTE_ERR_ARG, "out of host memory");
   }
+  double *ff = tab, *Mf = tab + 12 * N, *Mi = Mf + 2 * n2, *sym = tab + nset, *hv = tab + 2 * nset, *w = hv + N;
   const double Leta = -eta[0];
   build_matrix(N, eta, g->hv, Leta, L_v, 1.0, -1.0, Mf);
   build_matrix(N, v, g->heta, L_v, Leta, -1.0, 1.0, Mi);
+  build_fft_factors(N, eta, g->hv, Leta, L_v, 1.0, -1.0, ff);
+  build_fft_factors(N, v, g->heta, L_v, Leta, -1.0, 1.0, ff + 6 * N);
   for (int i = 0; i < N; i++) w[i] = (i == 0 || i == N - 1) ? 0.5 : 1.0;
+  memcpy(hv, v, sizeof(double) * N);
+  op->mirror.on = build_mirror(N, eta, L_v, g->heta, w, Mf, Mi, sym, &op->mirror);
   int rc = SPBTE_OK;
-  if (hipStreamCreate(&op->s) != hipSuccess || hipMalloc(&g->d_mat_fwd, sizeof(double) * 2 * N * N) != hipSuccess ||
-      hipMalloc(&g->d_mat_inv, sizeof(double) * 2 * N * N) != hipSuccess ||
-      hipMalloc(&g->d_v, sizeof(double) * N) != hipSuccess || hipMalloc(&g->d_w, sizeof(double) * N) != hipSuccess ||
-      hipMemcpy(g->d_mat_fwd, Mf, sizeof(double) * 2 * N * N, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(g->d_mat_inv, Mi, sizeof(double) * 2 * N * N, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(g->d_v, v, sizeof(double) * N, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(g->d_w, w, sizeof(double) * N, hipMemcpyHostToDevice) != hipSuccess)
+  if (hipStreamCreate(&op->s) != hipSuccess || hipMalloc((void **)&op->d_tab, sizeof(double) * ntab) != hipSuccess ||
+      hipMemcpy(op->d_tab, tab, sizeof(double) * ntab, hipMemcpyHostToDevice) != hipSuccess)
     rc = fail(SPBTE_ERR_HIP, "device setup failed: %s", hipGetErrorString(hipGetLastError()));
-  free(Mf);
-  free(Mi);
-  if (rc == SPBTE_OK && spbte_fft_supported(N)) {
-    double ff[2 * 6 * SPBTE_MAX_N];
-    build_fft_factors(N, eta, g->hv, Leta, L_v, 1.0, -1.0, ff);
-    build_fft_factors(N, v, g->heta, L_v, Leta, -1.0, 1.0, ff + 6 * N);
-    if (hipMalloc(&g->d_fft, sizeof(double) * 12 * N) != hipSuccess ||
-        hipMemcpy(g->d_fft, ff, sizeof(double) * 12 * N, hipMemcpyHostToDevice) != hipSuccess)
-      rc = fail(SPBTE_ERR_HIP, "device setup failed: %s", hipGetErrorString(hipGetLastError()));
+  free(tab);
+  if (rc == SPBTE_OK) {
+    g->d_mat_fwd = op->d_tab + 12 * N;
+    g->d_mat_inv = op->d_tab + 12 * N + 2 * n2;
+    g->d_v = op->d_tab + 2 * nset;
+    g->d_w = op->d_tab + 2 * nset + N;
+    if (spbte_fft_supported(N)) g->d_fft = op->d_tab;
+    op->d_sym = op->d_tab + nset;
   }
   if (rc != SPBTE_OK) {
     spbte_op_destroy(op);
@@ -339,6 +414,15 @@ int spbte_op_create(spbte_op **out, int N, double L_v, const double *v, const do
   return SPBTE_OK;
 }
 
+static void free_folded(struct wtable *w) {
+  for (int c = 0; c < 2; c++)
+    for (int f = 0; f < 2; f++)
+      for (int t = 0; t < 9; t++) {
+        if (w->dWh[c][f][t]) hipFree(w->dWh[c][f][t]);
+        w->dWh[c][f][t] = NULL;
+      }
+}
+
 static void free_weights(spbte_op *op) {
   for (int k = 0; k < SPBTE_MAX_NS * SPBTE_MAX_NS; k++) {
     struct wtable *w = &op->tab[k];
@@ -352,6 +436,7 @@ static void free_weights(spbte_op *op) {
         if (w->dWp[f][t]) hipFree(w->dWp[f][t]);
         w->dWp[f][t] = NULL;
       }
+    free_folded(w);
     w->have_w = 0;
   }
 }
@@ -383,11 +468,7 @@ void spbte_op_destroy(spbte_op *op) {
   if (op->d_Qp) hipFree(op->d_Qp);
   free_weights(op);
   free_scratch(op);
-  if (op->g.d_mat_fwd) hipFree(op->g.d_mat_fwd);
-  if (op->g.d_mat_inv) hipFree(op->g.d_mat_inv);
-  if (op->g.d_v) hipFree(op->g.d_v);
-  if (op->g.d_w) hipFree(op->g.d_w);
-  if (op->g.d_fft) hipFree(op->g.d_fft);
+  if (op->d_tab) hipFree(op->d_tab);
   if (op->s) hipStreamDestroy(op->s);
   free(op->v);
   free(op->eta);
@@ -434,10 +515,11 @@ typedef struct {
   void *Qp;    /* partial sums of the split streaming kernel (fixed sets only) */
   size_t qp_bytes;
   int fixed;   /* 1: allocate nothing */
+  int kind;    /* fixed sets: slices of the split streaming kernel (0: the tile's own) */
 } scratch_set;
 
 static scratch_set own_scratch(const spbte_op *op) {
-  scratch_set ss = {op->d_mom, op->d_part, op->d_xs, op->d_FG, op->d_Qh, NULL, 0, 0};
+  scratch_set ss = {op->d_mom, op->d_part, op->d_xs, op->d_FG, op->d_Qh, NULL, 0, 0, 0};
   return ss;
 }
 
@@ -451,6 +533,7 @@ static int alloc_w64(spbte_op *op) {
     for (int f = 0; f < 3; f++)
       for (int t = 0; t < 9; t++)
         if (op->t->dWp[f][t]) { hipFree(op->t->dWp[f][t]); op->t->dWp[f][t] = NULL; }
+    free_folded(op->t);
     return SPBTE_OK;
   }
   HIPCHK(hipMalloc((void **)&op->t->dW64, sizeof(double) * op->n3 * op->n3));
@@ -659,6 +742,48 @@ static int weights_permuted(spbte_op *op, int form, int tr, int build, const voi
   return SPBTE_OK;
 }
 
+/* How a weighted sum may use the symmetries of its operands. */
+enum {
+  SUM_ANY = 0,  /* operands arbitrary, or every mode of the result wanted: the whole table */
+  SUM_REAL = 1, /* operands transforms of real cells, result for the inverse's real part: half the rows */
+  SUM_SELF = 2  /* and the products symmetric under c <-> s(r, c) (Q(f, f)): half the columns as well */
+};
+
+/* The fold of a sum on a streaming tile: row planes and column fold of its
+ * table (k_wsum_stream.hip), 0 where it takes the whole one. */
+static int fold_of(const spbte_op *op, int form, const spbte_tile *t, int sum, int *npl, int *cfold) {
+  if (sum == SUM_ANY || t->kind < 1 || form == SPBTE_FORM_FP16X2 || !spbte_stream_tile_folds(op->N, t->tr, t->lines) ||
+      (sum == SUM_REAL && !op->mirror.on))
+    return 0;
+  *npl = op->mirror.on ? op->N / 2 + 1 : op->N;
+  *cfold = sum == SUM_SELF;
+  return 1;
+}
+
+/* The folded tables of a form for tr rows per lane.  Building makes both of them
+ * resident (without the mirror symmetry the whole table in place of the
+ * row-folded one) and the natural table of the form, so that what one evaluation
+ * built serves every later allocation-free one with rows of that tile.  Without
+ * build, *Wp is NULL where the one asked for is not resident. */
+static int weights_folded(spbte_op *op, int form, int tr, int npl, int cfold, int build, const void **Wp) {
+  const int st = storage_of(form) == SPBTE_FORM_FP64 ? 0 : 1, N = op->N;
+  for (int c = 0; c < 2 && build; c++) {
+    void **p = &op->t->dWh[c][st][tr];
+    if (*p) continue;
+    const void *w;
+    const float *rs;
+    int rc = !c && !op->mirror.on ? weights_permuted(op, form, tr, 1, &w, &rs) : weights_form(op, form, 1, &w, &rs);
+    if (rc) return rc;
+    if (!c && !op->mirror.on) continue;
+    const size_t rows = (size_t)npl * N * N, cols = (size_t)(c ? N / 2 + 1 : N) * N * N;
+    HIPCHK(hipMalloc(p, rows * cols * (st ? 4 : 8)));
+    op->gen++;
+    LCHK(spbte_launch_fold_weights(op->t->dW64, *p, st, tr, N, npl, c, &op->mirror, op->s));
+  }
+  *Wp = op->t->dWh[cfold][st][tr];
+  return SPBTE_OK;
+}
+
 /* ------------------------------------------------------------------ tiles */
 static int bucket(int ncell) {
   int b = 0;
@@ -702,60 +827,68 @@ static int default_tile(int N, int form, int nprod, int ncell, spbte_tile *t) {
   return 0;
 }
 
-/* Workgroups of a streaming tile without the x-plane split. */
+/* Workgroups of a streaming tile without the split, on a folded table where the
+ * tile has one (N/2 + 1 x-planes of output rows). */
 static long stream_wgs(int N, int ncell, const spbte_tile *t) {
-  return (long)N * N * N / (64L * t->lines * t->tr) * ((ncell + t->tb - 1) / t->tb);
+  const long rows = (long)(spbte_stream_tile_folds(N, t->tr, t->lines) ? N / 2 + 1 : N) * N * N;
+  return rows / (64L * t->lines * t->tr) * ((ncell + t->tb - 1) / t->tb);
 }
 
-/* Streaming kernel defaults (measured on 256-512 cells, MI355X): FP64 weights
- * favour 8 rows per lane for the two-product sum, FP32 weights 4 rows and 4
- * waves; the one-product (ComputeQ) sum at N=32 four cells per workgroup when
- * the batch has them; the FP32-product maxPreserve sum at N=24 takes 3 rows x 3 waves with
- * two problems per lane (31.7 ms for 512 problems against 44.2 ms on the tiled
- * kernel).  The 16-wave tile of the FP32-product maxPreserve sum at N=32 (four
- * cells per workgroup: half the W refetch) is left to the autotuner: on 512
- * problems it ran 5.8% faster than the 4-wave tile on one MI355X and 4.7%
- * slower on another.  Unsupported candidates are skipped.
- * Batches too small to give 2048 workgroups split the summed x-planes into up
- * to 8 slices; at N=16, where one to four cells take one row per lane, into
- * as many as give 2048 workgroups, cutting x-planes into y-line ranges if
- * need be (one cell: 32 slices of half an x-plane, its FP64 table streamed in
- * 41.6 us against 48.3 with 16 whole planes and 99 with 8 slices of 4 rows;
- * 64 slices took 56.8 us, the F staging outweighing the extra waves; with the
- * later kernel, two one-row waves a workgroup over the same 32 slices took
- * 26.8 us against 29.5 with one). */
+/* Streaming kernel defaults on folded tables, measured on an MI355X (us per
+ * evaluation, best of the tiles and splits tried):
+ *  N=32 two products: 4 rows x 4 waves (FP64, one cell: 444 against 472 with 8
+ *    rows x 2 waves); two cells per lane from 32 cells on with FP64 arithmetic
+ *    (128 cells: 16390 against 17440), never with FP32 products (512 cells:
+ *    41870 against 43880).  One product: as many cells per lane as the batch has,
+ *    to 4 (256 cells, 4 and 2: 17960, 19840).
+ *  N=24: 3 rows x 3 waves, the tile that keeps to one x-plane of rows; two cells
+ *    per lane with one product (37 cells: 735 against 807) and with FP32 products
+ *    (512 cells: 8390 against 8680).
+ *  N=16: one row per lane, 4 waves, up to 4 cells (one cell: 40 against 46 with
+ *    one wave, 47 with 4 rows); then 4 rows, with one cell per lane for two
+ *    products (600 cells: 1715 against 1920) and two for one.
+ * The summed lines are split into at least 8 slices (16 with FP32 products at
+ * N=32) and into as many as give 2400 workgroups, at most 32 (N=32), 48 (N=24),
+ * 64 (N=16): a last round of workgroups that is nearly empty costs less, and the
+ * slices of one r-tile keep nearer each other in the table (N=32, 512 cells with
+ * FP32 products: 43930 us with one slice, 42060 with 4, 40000 with 16; 256 cells
+ * ComputeQ in FP64: 22770 with one, 17910 with 4, 17530 with 8, 17910 with 16;
+ * one cell, FP64: 553 with 8, 413 with 60).  The inverse transform adds them. */
 static int default_stream_tile(int N, int form, int nprod, int ncell, spbte_tile *t) {
-  static const spbte_tile s32[] = {{4, 4, 4, 1}, {4, 4, 2, 1}, {4, 4, 1, 1}}, s32m[] = {{4, 4, 1, 1}},
-                         s32m64[] = {{8, 2, 1, 1}};
-  static const spbte_tile s24[] = {{4, 2, 2, 1}, {4, 2, 1, 1}}, s24m[] = {{4, 2, 1, 1}};
-  static const spbte_tile s24ma[] = {{3, 3, 2, 1}, {3, 3, 1, 1}};
-  static const spbte_tile s16[] = {{4, 1, 2, 1}, {4, 1, 1, 1}}, s16m[] = {{4, 1, 2, 1}, {4, 1, 1, 1}};
-  static const spbte_tile s16one[] = {{1, 2, 1, 1}};
+  static const spbte_tile s32[] = {{4, 4, 4, 1}, {4, 4, 2, 1}, {4, 4, 1, 1}}, s32m[] = {{4, 4, 2, 1}, {4, 4, 1, 1}};
+  static const spbte_tile s24[] = {{3, 3, 2, 1}, {3, 3, 1, 1}};
+  static const spbte_tile s16[] = {{4, 1, 2, 1}, {4, 1, 1, 1}};
+  static const spbte_tile s16few[] = {{1, 4, 1, 1}, {4, 1, 2, 1}};
   const spbte_tile *c = NULL;
-  int nc = 0;
+  int nc = 0, kmin = 8, kmax = 0;
   if (N == 32) {
+    kmax = 32;
     if (nprod == 1) { c = s32; nc = 3; }
-    else if (form == SPBTE_FORM_FP64) { c = s32m64; nc = 1; }
-    else { c = s32m; nc = 1; }
+    else {
+      const int one = form == SPBTE_FORM_FP32A || ncell < 32;
+      c = s32m + one;
+      nc = 2 - one;
+    }
+    if (form == SPBTE_FORM_FP32A) kmin = 16;
   } else if (N == 24) {
-    if (nprod == 2 && form == SPBTE_FORM_FP32A) { c = s24ma; nc = 2; }
-    else { c = nprod == 2 ? s24m : s24; nc = nprod == 2 ? 1 : 2; }
-  }
-  else if (N == 16) {
-    if (ncell <= 4 && spbte_stream_tile_supported(N, form, nprod, 1, 2, 1)) { c = s16one; nc = 1; }
-    else { c = nprod == 2 ? s16m : s16; nc = 2; }
-  }
-  else return 0;
+    kmax = 48;
+    const int one = nprod == 2 && form != SPBTE_FORM_FP32A;
+    c = s24 + one;
+    nc = 2 - one;
+  } else if (N == 16) {
+    kmax = 64;
+    const int one = nprod == 2 && form != SPBTE_FORM_FP32A;
+    if (ncell <= 4) { c = s16few; nc = 2; }
+    else { c = s16 + one; nc = 2 - one; }
+  } else return 0;
   for (int i = 0; i < nc; i++) {
     if (!spbte_stream_tile_supported(N, form, nprod, c[i].tr, c[i].lines, c[i].tb)) continue;
     if (c[i].tb > ncell && i + 1 < nc) continue;
     *t = c[i];
     const long wgs = stream_wgs(N, ncell, t);
-    int k = 1;
-    /* N <= 16 counts waves, not workgroups (its one-row tiles run 2 waves a workgroup) */
-    while ((N <= 16 ? wgs * k * t->lines : wgs * k) < 2048 && spbte_csplit_valid(N, 2 * k) && (N <= 16 || 2 * k <= 8))
-      k *= 2;
-    t->kind = k;
+    t->kind = kmin;
+    for (int k = kmin; k <= kmax && wgs * t->kind < 2400; k++)
+      if (spbte_csplit_valid(N, k)) t->kind = k;
     return 1;
   }
   return 0;
@@ -810,20 +943,37 @@ int spbte_get_tile(spbte_op *op, int ncell, int form, int maxpreserve, int *kind
 }
 
 /* ---------------------------------------------------------- the operator */
-/* The weighted sum's result is left at *qsrc as *nsl sets to add: Qh (one set),
+typedef struct {
+  const void *q; /* where the weighted sum's result is */
+  int nsl;       /* sets to add */
+  int npl;       /* x-planes of each cube that hold it (the others are zero, not written) */
+} wsum_result;
+
+/* The weighted sum's result is left as res->nsl sets to add: Qh (one set),
  * or, with a->keep_slices, a split tile's unsummed slices in Qp. */
-static int launch_tile(spbte_op *op, int form, const spbte_tile *t, const spbte_wsum_args *a, const scratch_set *ss,
-                       const void **qsrc, int *nsl) {
-  const float *rs;
-  *qsrc = a->Qh;
-  *nsl = 1;
+static int launch_tile(spbte_op *op, int form, const spbte_tile *t, const spbte_wsum_args *a0, int sum,
+                       const scratch_set *ss, wsum_result *res) {
+  const float *rs = NULL;
+  spbte_wsum_args b = *a0;
+  const spbte_wsum_args *a = &b;
+  res->q = a->Qh;
+  res->nsl = 1;
+  res->npl = op->N;
   if (t && t->kind >= 1) {
     const void *Wp = NULL;
-    int rc = weights_permuted(op, form, t->tr, !ss->fixed, &Wp, &rs);
+    int rc = SPBTE_OK;
+    if (fold_of(op, form, t, sum, &b.npl, &b.cfold)) {
+      rc = weights_folded(op, form, t->tr, b.npl, b.cfold, !ss->fixed, &Wp);
+      if (rc) return rc;
+      if (Wp) res->npl = b.npl;
+      else b.npl = b.cfold = 0;
+    }
+    if (!Wp) rc = weights_permuted(op, form, t->tr, !ss->fixed, &Wp, &rs);
     if (rc) return rc;
     void *Qp = NULL;
-    if (t->kind > 1) {
-      const size_t need = (size_t)t->kind * a->ncell * op->n3 * 16;
+    const int k = ss->fixed && ss->kind ? ss->kind : t->kind;
+    if (k > 1) {
+      const size_t need = (size_t)k * a->ncell * op->n3 * 16;
       if (ss->fixed) {
         if (need > ss->qp_bytes) return fail(SPBTE_ERR_ARG, "partial sums need %zu bytes of workspace", need);
         Qp = ss->Qp;
@@ -833,36 +983,35 @@ static int launch_tile(spbte_op *op, int form, const spbte_tile *t, const spbte_
         Qp = op->d_Qp;
       }
     }
-    LCHK(spbte_launch_wsum_stream(op->N, form, t->tr, t->lines, t->tb, a, Wp, rs, t->kind, Qp, op->s));
-    if (a->keep_slices && t->kind > 1) {
-      *qsrc = Qp;
-      *nsl = t->kind;
+    LCHK(spbte_launch_wsum_stream(op->N, form, t->tr, t->lines, t->tb, a, Wp, rs, k, Qp, op->s));
+    if (a->keep_slices && k > 1) {
+      res->q = Qp;
+      res->nsl = k;
     }
     return SPBTE_OK;
   }
   const void *W;
   int rc = weights_form(op, form, !ss->fixed, &W, &rs);
   if (rc) return rc;
-  spbte_wsum_args b = *a;
   b.W = W;
   LCHK(spbte_launch_wsum_scaled(op->N, form, t, &b, rs, op->s));
   return SPBTE_OK;
 }
 
-/* keep_slices: a split tile may leave its slices unsummed (see launch_tile);
- * qsrc/nsl (NULL unless keep_slices) say where the result is. */
+/* keep_slices: a split tile may leave its slices unsummed (see launch_tile). */
 static int run_wsum(spbte_op *op, int form, int nprod, const void *F0, const void *G0, const void *F1, const void *G1,
-                    int ncell, const scratch_set *ss, int keep_slices, const void **qsrc, int *nsl) {
+                    int ncell, int sum, const scratch_set *ss, int keep_slices, wsum_result *res) {
   if (!op->t->have_w) return fail(SPBTE_ERR_NOWEIGHTS, "no weight table set");
   spbte_tile t;
   int have = pick_tile(op, ncell, form, nprod, &t);
   if (!have && form != SPBTE_FORM_FP64)
     return fail(SPBTE_ERR_UNSUPPORTED, "no reduced-precision weighted-sum kernel for N=%d", op->N);
-  spbte_wsum_args a = {NULL, F0, G0, F1, G1, ss->Qh, ncell, nprod, keep_slices};
-  const void *q;
-  int n;
-  return launch_tile(op, form, have ? &t : NULL, &a, ss, qsrc ? qsrc : &q, nsl ? nsl : &n);
+  spbte_wsum_args a = {NULL, F0, G0, F1, G1, ss->Qh, ncell, nprod, keep_slices, 0, 0};
+  return launch_tile(op, form, have ? &t : NULL, &a, sum, ss, res);
 }
+
+/* Flag beside the public ones: every mode of Qhat is left in ss->Qh. */
+#define FULL_QHAT (1 << 30)
 
 /* One chunk of spbte_compute_q.  ev_a/ev_b (optional) bracket the weighted-sum
  * launch so its duration can be timed on the operator's stream. */
@@ -879,10 +1028,17 @@ static int compute_chunk(spbte_op *op, const double *d_f, const double *d_g, dou
   int nj = 0;
   const void *F0, *G0, *F1 = NULL, *G1 = NULL;
   double *mom_f = ss->mom, *mom_g = ss->mom + (size_t)ncell * SPBTE_MOM_STRIDE;
+  const int sum = (flags & FULL_QHAT) ? SUM_ANY : (self ? SUM_SELF : SUM_REAL);
+  spbte_grid_dev g = op->g;
+  if (sum != SUM_ANY && op->mirror.on) {
+    g.d_mat_fwd = op->d_sym + 12 * op->N;
+    g.d_mat_inv = op->d_sym + 12 * op->N + 2 * op->n3 / op->N;
+    if (g.d_fft) g.d_fft = op->d_sym;
+  }
   /* FFT grids: the forward transform computes the Maxwellians' moments itself
    * from per-plane partial sums (f's, then g's, in ss->part), and the inverse
    * transform writes the projection's partial sums (over f's, dead by then) */
-  const int fused = op->g.d_fft != NULL && spbte_fft_supported(op->N);
+  const int fused = g.d_fft != NULL && spbte_fft_supported(op->N);
   /* small grids: for a few cells the forward transform's workgroups take the
    * Maxwellians' moments from the cells themselves (every Maxwellian
    * workgroup reads its whole cell, 1 MB per cell at N=16, against a launch
@@ -902,13 +1058,13 @@ static int compute_chunk(spbte_op *op, const double *d_f, const double *d_g, dou
     /* Q = sum W [ T(g - M_f)[c] T(f)[s] + T(M_g)[c] T(f - M_f)[s] ] */
     if (fused) {
       if (!mom_inl) {
-        LCHK(spbte_launch_moment_partials(&op->g, d_f, ncell, (double *)part_f, op->s));
-        if (!self) LCHK(spbte_launch_moment_partials(&op->g, d_g, ncell, (double *)part_g, op->s));
+        LCHK(spbte_launch_moment_partials(&g, d_f, ncell, (double *)part_f, op->s));
+        if (!self) LCHK(spbte_launch_moment_partials(&g, d_g, ncell, (double *)part_g, op->s));
       }
       mom_f = mom_g = NULL;
     } else {
-      LCHK(spbte_launch_moments(&op->g, d_f, mom_f, ncell, ss->part, op->s));
-      if (!self) LCHK(spbte_launch_moments(&op->g, d_g, mom_g, ncell, ss->part, op->s));
+      LCHK(spbte_launch_moments(&g, d_f, mom_f, ncell, ss->part, op->s));
+      if (!self) LCHK(spbte_launch_moments(&g, d_g, mom_g, ncell, ss->part, op->s));
     }
     jobs[nj++] = (spbte_xform_job){d_f, NULL, 0, B[0], NULL, NULL};           /* F0 = T(f)        */
     jobs[nj++] = (spbte_xform_job){d_f, mom_f, 1, B[1], part_f, msrc_f};      /* F1 = T(f - M_f)  */
@@ -925,29 +1081,38 @@ static int compute_chunk(spbte_op *op, const double *d_f, const double *d_g, dou
       G1 = B[3];
     }
   }
-  LCHK(spbte_launch_xform_fwd(&op->g, jobs, nj, ncell, fg_bytes(form) == 8, ss->xs, op->s));
+  LCHK(spbte_launch_xform_fwd(&g, jobs, nj, ncell, fg_bytes(form) == 8, ss->xs, op->s));
   if (ev_a) HIPCHK(hipEventRecord(ev_a, op->s));
   /* FFT grids: the inverse transform adds the split sum's slices itself */
-  const void *qsrc;
-  int nsl;
-  int rc = run_wsum(op, form, mp ? 2 : 1, F0, G0, F1, G1, ncell, ss, fused, &qsrc, &nsl);
+  wsum_result r;
+  int rc = run_wsum(op, form, mp ? 2 : 1, F0, G0, F1, G1, ncell, sum, ss, fused && !(flags & FULL_QHAT), &r);
   if (ev_b) HIPCHK(hipEventRecord(ev_b, op->s));
   if (rc) return rc;
   const int cons = (flags & SPBTE_CONSERVE) != 0;
   if (cons && op->Ns != 1) return fail(SPBTE_ERR_UNSUPPORTED, "per-cell projection needs one species (Ns=%d)", op->Ns);
   if (cube_i) {
-    LCHK(spbte_launch_xform_inv_real_cube(&op->g, qsrc, nsl, d_Q, ncell, ss->xs, cons ? op->masses : NULL, op->LU,
+    LCHK(spbte_launch_xform_inv_real_cube(&g, r.q, r.nsl, r.npl, d_Q, ncell, ss->xs, cons ? op->masses : NULL, op->LU,
                                           op->pivot, epi, op->s));
     return SPBTE_OK;
   }
   if (epi) return fail(SPBTE_ERR_UNSUPPORTED, "no fused update on this grid and batch");
-  LCHK(spbte_launch_xform_inv_real(&op->g, qsrc, nsl, d_Q, ncell, ss->xs, cons && fused ? ss->part : NULL, op->s));
-  if (cons && fused) LCHK(spbte_launch_project_apply(&op->g, op->masses, op->LU, op->pivot, d_Q, ncell, ss->part, op->s));
-  else if (cons) LCHK(spbte_launch_project(&op->g, 1, op->masses, op->LU, op->pivot, d_Q, ncell, ss->part, op->s));
+  LCHK(spbte_launch_xform_inv_real(&g, r.q, r.nsl, r.npl, d_Q, ncell, ss->xs, cons && fused ? ss->part : NULL, op->s));
+  if (cons && fused) LCHK(spbte_launch_project_apply(&g, op->masses, op->LU, op->pivot, d_Q, ncell, ss->part, op->s));
+  else if (cons) LCHK(spbte_launch_project(&g, 1, op->masses, op->LU, op->pivot, d_Q, ncell, ss->part, op->s));
   return SPBTE_OK;
 }
 
+static int compute_q(spbte_op *op, const double *d_f, const double *d_g, double *d_Q, int ncell, int form, int flags);
+
 int spbte_compute_q(spbte_op *op, const double *d_f, const double *d_g, double *d_Q, int ncell, int form, int flags) {
+  return compute_q(op, d_f, d_g, d_Q, ncell, form, flags & ~FULL_QHAT);
+}
+
+int spbte_compute_q_qhat(spbte_op *op, const double *d_f, double *d_Q, int ncell, int form, int flags) {
+  return compute_q(op, d_f, NULL, d_Q, ncell, form, flags | FULL_QHAT);
+}
+
+static int compute_q(spbte_op *op, const double *d_f, const double *d_g, double *d_Q, int ncell, int form, int flags) {
   if (!op || ncell < 0 || form < 0 || form >= NFORMS) return fail(SPBTE_ERR_ARG, "bad arguments");
   if (ncell == 0) return SPBTE_OK;
   if (!d_f || !d_Q) return fail(SPBTE_ERR_ARG, "null buffer");
@@ -996,6 +1161,7 @@ int spbte_compute_q_noalloc(spbte_op *op, const double *d_f, const double *d_g, 
     return fail(SPBTE_ERR_HIP, "no fixed workspace on this GPU: %s", hipGetErrorString((hipError_t)op->nac_err));
   if ((flags & SPBTE_CONSERVE) && op->Ns != 1)
     return fail(SPBTE_ERR_UNSUPPORTED, "per-cell projection needs one species (Ns=%d)", op->Ns);
+  flags &= ~FULL_QHAT;
   if (!d_g) flags |= SPBTE_SELF;
   const int self = (flags & SPBTE_SELF) != 0 || d_g == d_f;
   const int mp = (flags & SPBTE_MAXPRESERVE) != 0;
@@ -1004,9 +1170,13 @@ int spbte_compute_q_noalloc(spbte_op *op, const double *d_f, const double *d_g, 
   const int have = pick_tile(op, ncell, form, mp ? 2 : 1, &t);
   if (!have && form != SPBTE_FORM_FP64)
     return fail(SPBTE_ERR_UNSUPPORTED, "no reduced-precision weighted-sum kernel for N=%d", op->N);
-  const void *W;
+  const void *W = NULL;
   const float *rs;
-  int rc = (have && t.kind >= 1) ? weights_permuted(op, form, t.tr, 0, &W, &rs) : weights_form(op, form, 0, &W, &rs);
+  int rc = SPBTE_OK, npl, cfold;
+  if (have && fold_of(op, form, &t, self ? SUM_SELF : SUM_REAL, &npl, &cfold))
+    rc = weights_folded(op, form, t.tr, npl, cfold, 0, &W);
+  if (!rc && !W)
+    rc = (have && t.kind >= 1) ? weights_permuted(op, form, t.tr, 0, &W, &rs) : weights_form(op, form, 0, &W, &rs);
   if (rc) return rc;
   /* workspace: moments | partial sums | transformed operands | Qhat | transform scratch,
    * which also holds the split sum's partial sums (they are dead by the time
@@ -1016,9 +1186,16 @@ int spbte_compute_q_noalloc(spbte_op *op, const double *d_f, const double *d_g, 
   const size_t b_mom = al256(sizeof(double) * 2 * (size_t)ncell * SPBTE_MOM_STRIDE);
   const size_t b_part = al256(sizeof(double) * 10 * (size_t)op->N * ncell);
   const size_t b_fg = al256((size_t)nj * fg_stride(form, n)), b_qh = al256(16 * n);
-  const size_t b_xs = 16 * n * (size_t)nj, b_qp = (have && t.kind > 1) ? 16 * n * (size_t)t.kind : 0;
+  const size_t b_xs = 16 * n * (size_t)nj, b_fix = b_mom + b_part + b_fg + b_qh;
+  /* a tile that was not pinned or tuned takes fewer slices where the workspace
+   * does not hold its own number (the sums then differ by rounding) */
+  int kind = have ? t.kind : 0;
+  spbte_tile dt;
+  const int is_default = have && default_stream_tile(op->N, form, mp ? 2 : 1, ncell, &dt) && !memcmp(&dt, &t, sizeof t);
+  while (is_default && kind > 1 && b_fix + al256(16 * n * (size_t)kind) > op->nac_bytes) kind--;
+  const size_t b_qp = kind > 1 ? 16 * n * (size_t)kind : 0;
   const size_t b_x = al256(b_xs > b_qp ? b_xs : b_qp);
-  const size_t need = b_mom + b_part + b_fg + b_qh + b_x;
+  const size_t need = b_fix + b_x;
   if (need > op->nac_bytes)
     return fail(SPBTE_ERR_ARG, "a batch of %d cells at N=%d needs %zu bytes of workspace, more than the %zu of the "
                 "fixed workspace (SPBTE_NOALLOC_SCRATCH_BYTES)", ncell, op->N, need, op->nac_bytes);
@@ -1033,6 +1210,7 @@ int spbte_compute_q_noalloc(spbte_op *op, const double *d_f, const double *d_g, 
   ss.Qp = ss.xs;
   ss.qp_bytes = b_x;
   ss.fixed = 1;
+  ss.kind = kind;
   return compute_chunk(op, d_f, d_g, d_Q, ncell, form, flags, NULL, NULL, &ss, NULL);
 }
 
@@ -1110,7 +1288,8 @@ int spbte_qhat(spbte_op *op, const double *d_Fhat, const double *d_Ghat, double 
     G = FG + stride;
   }
   const scratch_set ss = own_scratch(op);
-  rc = run_wsum(op, form, 1, F, G, NULL, NULL, ncell, &ss, 0, NULL, NULL);
+  wsum_result r;
+  rc = run_wsum(op, form, 1, F, G, NULL, NULL, ncell, SUM_ANY, &ss, 0, &r);
   if (rc) return rc;
   HIPCHK(hipMemcpyAsync(d_Qhat, op->d_Qh, 16 * n, hipMemcpyDeviceToDevice, op->s));
   return SPBTE_OK;
@@ -1168,7 +1347,7 @@ static const spbte_tile k_cand[] = {
     {3, 3, 2, 1}, {4, 2, 1, 1}, {8, 1, 1, 1}, {4, 1, 1, 1}, {4, 1, 2, 1}, {4, 9, 1, 1}, {4, 16, 1, 1},
     /* streaming with the summed x-planes split in 2-8 slices, for small batches */
     {4, 4, 1, 2}, {4, 4, 1, 4}, {4, 4, 1, 8}, {4, 4, 2, 2}, {4, 4, 2, 4}, {4, 4, 2, 8}, {4, 2, 1, 4}, {4, 2, 1, 8},
-    {4, 2, 2, 4}, {8, 2, 1, 4}, {8, 2, 1, 8}, {4, 2, 1, 2}, {4, 9, 1, 2}, {4, 9, 1, 4},
+    {4, 2, 2, 4}, {8, 2, 1, 4}, {8, 2, 1, 8}, {4, 2, 1, 2}, {4, 9, 1, 2}, {4, 9, 1, 4}, {3, 3, 1, 8}, {3, 3, 1, 24},
     /* one or a few cells at N=16: narrower rows, up to one x-plane per slice */
     {4, 1, 1, 8}, {4, 1, 1, 16}, {2, 1, 1, 8}, {2, 1, 1, 16}, {1, 1, 1, 8}, {1, 1, 1, 16}, {8, 2, 1, 16},
     /* and x-planes cut into y-line ranges */
@@ -1190,24 +1369,25 @@ int spbte_autotune(spbte_op *op, int ncell, int form, int maxpreserve, int *kind
   char *FG = (char *)op->d_FG;
   LCHK(spbte_launch_fill_pattern(FG, 4 * stride / (single ? 4 : 8), single, op->s));
   spbte_wsum_args args = {NULL, FG, FG + stride, np == 2 ? FG + 2 * stride : NULL, np == 2 ? FG + 3 * stride : NULL,
-                          op->d_Qh, ncell, np, 0};
+                          op->d_Qh, ncell, np, 0, 0, 0};
   const scratch_set ss = own_scratch(op);
   spbte_tile best = {0, 0, 0, 0};
   float best_ms = 1e30f;
-  const void *qsrc;
-  int nsl;
+  wsum_result res;
   hipEvent_t a, b;
   HIPCHK(hipEventCreate(&a));
   HIPCHK(hipEventCreate(&b));
-  for (size_t i = 0; i < sizeof k_cand / sizeof k_cand[0]; i++) {
-    const spbte_tile *t = &k_cand[i];
+  spbte_tile dt = {0, 0, 0, 0};
+  const int have_dt = default_stream_tile(op->N, form, np, ncell, &dt);
+  for (size_t i = 0; i < sizeof k_cand / sizeof k_cand[0] + (size_t)have_dt; i++) {
+    const spbte_tile *t = have_dt ? (i ? &k_cand[i - 1] : &dt) : &k_cand[i]; /* the default tile first */
     if (!tile_supported(op->N, form, np, t)) continue;
     if (t->tb > 2 * ncell) continue;
     if (t->kind > 1 && stream_wgs(op->N, ncell, t) >= 2048) continue; /* the chip is full without a split */
     /* warm-up (builds the table layout it needs); a tile whose warm-up alone
      * takes twice the best time so far is not timed further */
     HIPCHK(hipEventRecord(a, op->s));
-    rc = launch_tile(op, form, t, &args, &ss, &qsrc, &nsl);
+    rc = launch_tile(op, form, t, &args, SUM_SELF, &ss, &res);
     HIPCHK(hipEventRecord(b, op->s));
     HIPCHK(hipEventSynchronize(b));
     if (rc) break;
@@ -1216,7 +1396,7 @@ int spbte_autotune(spbte_op *op, int ncell, int form, int maxpreserve, int *kind
     if (warm > 2.0f * best_ms) continue;
     HIPCHK(hipEventRecord(a, op->s));
     const int reps = 2;
-    for (int r = 0; r < reps && rc == SPBTE_OK; r++) rc = launch_tile(op, form, t, &args, &ss, &qsrc, &nsl);
+    for (int r = 0; r < reps && rc == SPBTE_OK; r++) rc = launch_tile(op, form, t, &args, SUM_SELF, &ss, &res);
     HIPCHK(hipEventRecord(b, op->s));
     HIPCHK(hipEventSynchronize(b));
     if (rc) break;

@@ -58,7 +58,19 @@ typedef struct {
   int nprod;          /* 1: ComputeQ, 2: fused maxPreserve */
   int keep_slices;    /* split streaming tiles: leave the slices' partial sums in
                          Qp for the consumer to add (Qh is then not written) */
+  int npl, cfold;     /* streaming kernel on a folded table: x-planes of output rows
+                         it holds (0: all N; the others of Qh are not written), and
+                         whether its columns are folded too */
 } spbte_wsum_args;
+
+/* Mirror symmetry of the transforms of real cells on one grid: with
+ * k' = (2 (N/2) - k) mod N, X[k'] = s(k) conj X[k] for the forward transform,
+ * and the inverse's real part takes Qhat[k'] as r(k) conj Qhat[k'] at k (both
+ * are products over the three axes). */
+typedef struct {
+  int on;
+  double s[SPBTE_MAX_N], r[SPBTE_MAX_N];
+} spbte_mirror;
 
 /* Tile of a weighted-sum kernel.  kind 0: k_wsum.hip (lines = z-lines of output
  * modes per workgroup); kind 1: k_wsum_stream.hip (lines = waves per workgroup). */
@@ -81,7 +93,8 @@ int spbte_launch_xform_fwd(const spbte_grid_dev *g, const spbte_xform_job *jobs,
 int spbte_launch_xform_fwd_complex(const spbte_grid_dev *g, const void *in, void *out, int ncell, int invert,
                                    void *scratch, hipStream_t s);
 /* Qh: nsl sets of ncell * N^3 double2, ncell * N^3 apart, whose sum is
- * transformed (nsl > 1 on FFT grids only: the split weighted sum's slices; Qh
+ * transformed, the first npl of each cube's N x-planes only (the others are
+ * taken as zero and not read) (nsl > 1 on FFT grids only: the split weighted sum's slices; Qh
  * may then alias scratch).  proj_part (FFT grids only, else NULL): also writes
  * the one-species projection's per-plane partial sums of q (5 N per cell) for
  * spbte_launch_project_apply. */
@@ -106,11 +119,11 @@ int spbte_compute_q_update(struct spbte_op *op, const double *d_f, double *d_Q, 
 /* Inverse transform of the sum of nsl sets to the real part on whole-cube
  * grids, projected per cell (one species) when masses is not NULL, then the
  * update epi when it is not NULL. */
-int spbte_launch_xform_inv_real_cube(const spbte_grid_dev *g, const void *Qh, int nsl, double *q, int ncell,
+int spbte_launch_xform_inv_real_cube(const spbte_grid_dev *g, const void *Qh, int nsl, int npl, double *q, int ncell,
                                      void *scratch, const double *masses, const double *LU, const int *pivot,
                                      const spbte_epilogue *epi, hipStream_t s);
-int spbte_launch_xform_inv_real(const spbte_grid_dev *g, const void *Qh, int nsl, double *q, int ncell, void *scratch,
-                                double *proj_part, hipStream_t s);
+int spbte_launch_xform_inv_real(const spbte_grid_dev *g, const void *Qh, int nsl, int npl, double *q, int ncell,
+                                void *scratch, double *proj_part, hipStream_t s);
 /* The first pass of spbte_launch_moments alone (part: 5 N per cell), whose
  * partials FFT transform jobs read in place of the moments. */
 int spbte_launch_moment_partials(const spbte_grid_dev *g, const double *f, int ncell, double *part, hipStream_t s);
@@ -133,6 +146,9 @@ int spbte_stream_tile_supported(int N, int form, int nprod, int tr, int waves, i
 int spbte_csplit_valid(int N, int csplit);
 int spbte_launch_wsum_stream(int N, int form, int tr, int waves, int tb, const spbte_wsum_args *a, const void *Wp,
                              const float *rowscale, int csplit, void *Qp, hipStream_t s);
+int spbte_stream_tile_folds(int N, int tr, int waves);
+int spbte_launch_fold_weights(const double *W64, void *dst, int form, int TR, int N, int npl, int cfold,
+                              const spbte_mirror *mr, hipStream_t s);
 int spbte_launch_permute_weights(const double *W64, void *dst, const float *rowscale, int form, int TR, size_t n3,
                                  hipStream_t s);
 /* Projection of ncell groups of Ns*Ns arrays (group-major).  part: (Ns+4) N
@@ -217,6 +233,9 @@ hipStream_t spbte_op_stream(struct spbte_op *op);
 const spbte_grid_dev *spbte_op_grid(struct spbte_op *op);
 int spbte_op_get_weights_rows(struct spbte_op *op, double **rows);
 unsigned spbte_op_generation(struct spbte_op *op);
+/* spbte_compute_q (f alone) that leaves every mode of Qhat of its last chunk in
+ * spbte_op_qhat_buffer. */
+int spbte_compute_q_qhat(struct spbte_op *op, const double *d_f, double *d_Q, int ncell, int form, int flags);
 const void *spbte_op_qhat_buffer(struct spbte_op *op);
 int spbte_op_chunk_cells(struct spbte_op *op);
 int spbte_op_n(struct spbte_op *op);

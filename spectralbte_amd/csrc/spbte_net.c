@@ -345,7 +345,7 @@ static int moments_and_features(spbte_net *n, const double *d_f, int B) {
 /* Exact Qhat of the operator (ComputeQ or fused maxPreserve, FP64 weights) -> n->T. */
 static int exact_targets(spbte_net *n, const double *d_f, double *d_Qscratch, int B) {
   const int flags = SPBTE_SELF | (n->maxpreserve ? SPBTE_MAXPRESERVE : 0);
-  CHK(spbte_compute_q(n->op, d_f, NULL, d_Qscratch, B, SPBTE_FORM_FP64, flags));
+  CHK(spbte_compute_q_qhat(n->op, d_f, d_Qscratch, B, SPBTE_FORM_FP64, flags));
   LCHK(spbte_net_targets(n->N, n->Kb, B, spbte_op_qhat_buffer(n->op), n->mom, n->tscale, n->T, n->s));
   return SPBTE_OK;
 }
@@ -516,7 +516,7 @@ int spbte_net_predict(spbte_net *n, const double *d_f, double *d_Q, int ncell, i
     CHK(moments_and_features(n, d_f + c0 * n3, B));
     CHK(forward(n, B));
     LCHK(spbte_net_scatter(n->N, n->Kb, B, n->Y, n->mom, n->tscale, n->Qh, n->s));
-    LCHK(spbte_launch_xform_inv_real(g, n->Qh, 1, d_Q + c0 * n3, B, n->xs, NULL, n->s));
+    LCHK(spbte_launch_xform_inv_real(g, n->Qh, 1, n->N, d_Q + c0 * n3, B, n->xs, NULL, n->s));
   }
   if (conserve) CHK(spbte_conserve(n->op, d_Q, ncell));
   return SPBTE_OK;
