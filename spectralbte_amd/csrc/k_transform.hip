@@ -122,14 +122,24 @@ __global__ void __launch_bounds__(XT) k_xform_a_real(int N, XformJobs jobs, int 
 }
 
 // Pass A for complex FP64 inputs.
-__global__ void __launch_bounds__(XT) k_xform_a_cplx(int N, const double2 *__restrict__ in, int ncell,
-                                                     const double2 *__restrict__ M, double2 *__restrict__ scratch) {
+// the sum of nsl sets, as in k_fft_a_cplx (in may alias scratch)
+__global__ void __launch_bounds__(XT) k_xform_a_cplx(int N, const double2 *in, int nsl, int ncell,
+                                                     const double2 *__restrict__ M, double2 *scratch) {
   extern __shared__ double2 sm[];
   const int n2 = N * N;
-  const size_t n3 = (size_t)n2 * N;
+  const size_t n3 = (size_t)n2 * N, sstride = (size_t)ncell * n3;
   const int i = blockIdx.x, cell = blockIdx.y;
   double2 *X = sm, *T1 = sm + n2;
-  for (int e = threadIdx.x; e < n2; e += XT) X[e] = in[cell * n3 + (size_t)i * n2 + e];
+  for (int e = threadIdx.x; e < n2; e += XT) {
+    const size_t o = cell * n3 + (size_t)i * n2 + e;
+    double2 x = in[o];
+    for (int sl = 1; sl < nsl; ++sl) {
+      const double2 y = in[(size_t)sl * sstride + o];
+      x.x += y.x;
+      x.y += y.y;
+    }
+    X[e] = x;
+  }
   __syncthreads();
   plane_zy(N, M, X, T1, scratch + (size_t)cell * n3 + (size_t)i * n2);
 }
@@ -992,7 +1002,7 @@ extern "C" int spbte_launch_xform_fwd_complex(const spbte_grid_dev *g, const voi
   const double2 *M = (const double2 *)(invert ? g->d_mat_inv : g->d_mat_fwd);
   const double pre = invert ? g->pre_inv : g->pre_fwd;
   XformJobs J = {};
-  hipLaunchKernelGGL(k_xform_a_cplx, dim3(N, ncell, 1), dim3(XT), lds_a, s, N, (const double2 *)in, ncell, M,
+  hipLaunchKernelGGL(k_xform_a_cplx, dim3(N, ncell, 1), dim3(XT), lds_a, s, N, (const double2 *)in, 1, ncell, M,
                      (double2 *)scratch);
   hipLaunchKernelGGL(k_xform_b<0>, dim3(N, ncell, 1), dim3(XT), lds_b, s, N, ncell, M, pre, (const double2 *)scratch, J, out, N);
   return (int)hipGetLastError();
@@ -1005,11 +1015,11 @@ extern "C" int spbte_launch_xform_inv_real(const spbte_grid_dev *g, const void *
         launch_fft_cplx<decltype(n)::value>(g, Qh, nsl, npl, q, ncell, 1, 1, scratch, proj_part, s);
       }))
     return (int)hipGetLastError();
-  if (proj_part || nsl != 1) return (int)hipErrorInvalidValue;  // the matrix form takes one set, writes no partials
+  if (proj_part) return (int)hipErrorInvalidValue;  // the matrix form writes no partials
   const int N = g->N;
   const size_t lds_a = 2 * (size_t)N * N * sizeof(double2), lds_b = (size_t)N * N * sizeof(double2);
   XformJobs J = {};
-  hipLaunchKernelGGL(k_xform_a_cplx, dim3(npl, ncell, 1), dim3(XT), lds_a, s, N, (const double2 *)Qh, ncell,
+  hipLaunchKernelGGL(k_xform_a_cplx, dim3(npl, ncell, 1), dim3(XT), lds_a, s, N, (const double2 *)Qh, nsl, ncell,
                      (const double2 *)g->d_mat_inv, (double2 *)scratch);
   hipLaunchKernelGGL(k_xform_b<2>, dim3(N, ncell, 1), dim3(XT), lds_b, s, N, ncell, (const double2 *)g->d_mat_inv,
                      g->pre_inv, (const double2 *)scratch, J, (void *)q, npl);

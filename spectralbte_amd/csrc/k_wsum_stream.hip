@@ -508,11 +508,7 @@ int launch_s(const spbte_wsum_args *a, const void *Wp, const float *rowscale, in
                        s, (const uint4 *)Wp, rowscale, (const double2 *)a->F0, (const double2 *)a->G0,
                        (const double2 *)a->F1, (const double2 *)a->G1, (double2 *)a->Qh, a->ncell, csplit,
                        (double2 *)Qp, npl, npl != N || cfold ? 2 + cfold : 0);
-  if (csplit > 1 && !a->keep_slices) {
-    const size_t n = (size_t)a->ncell * N * N * N;
-    hipLaunchKernelGGL(k_slice_sum, dim3((unsigned)((n + 255) / 256 < 16384 ? (n + 255) / 256 : 16384)), dim3(256), 0,
-                       s, n, csplit, (const double2 *)Qp, (double2 *)a->Qh);
-  }
+  if (csplit > 1 && !a->keep_slices) return spbte_launch_slice_sum(N, a->ncell, csplit, Qp, a->Qh, s);
   return (int)hipGetLastError();
 }
 
@@ -670,6 +666,13 @@ extern "C" int spbte_csplit_valid(int N, int csplit) {
   if (csplit < 1) return 0;
   if (csplit <= N) return N % csplit == 0;
   return csplit % N == 0 && N % (csplit / N) == 0;
+}
+
+extern "C" int spbte_launch_slice_sum(int N, int ncell, int csplit, const void *Qp, void *Qh, hipStream_t s) {
+  const size_t n = (size_t)ncell * N * N * N;
+  hipLaunchKernelGGL(k_slice_sum, dim3((unsigned)((n + 255) / 256 < 16384 ? (n + 255) / 256 : 16384)), dim3(256), 0, s, n,
+                     csplit, (const double2 *)Qp, (double2 *)Qh);
+  return (int)hipGetLastError();
 }
 
 extern "C" int spbte_stream_tile_supported(int N, int form, int nprod, int tr, int waves, int tb) {

@@ -70,6 +70,7 @@ struct spbte_op {
     void *dWp[3][9];   /* tables permuted for the streaming kernel, per storage form and rows per lane */
     void *dWh[2][2][9]; /* the same folded (k_fold_w): [columns folded too][storage form FP64, FP32][rows per lane] */
     int have_w;
+    void *dWa[2];      /* folded for k_wsum_any.hip: rows, rows and columns */
   } tab[SPBTE_MAX_NS * SPBTE_MAX_NS], *t;
   /* conservation */
   int Ns;
@@ -415,6 +416,10 @@ int spbte_op_create(spbte_op **out, int N, double L_v, const double *v, const do
 }
 
 static void free_folded(struct wtable *w) {
+  for (int c = 0; c < 2; c++) {
+    if (w->dWa[c]) hipFree(w->dWa[c]);
+    w->dWa[c] = NULL;
+  }
   for (int c = 0; c < 2; c++)
     for (int f = 0; f < 2; f++)
       for (int t = 0; t < 9; t++) {
@@ -990,6 +995,37 @@ static int launch_tile(spbte_op *op, int form, const spbte_tile *t, const spbte_
     }
     return SPBTE_OK;
   }
+  if (!t && sum != SUM_ANY && spbte_any_supported(op->N) && (sum == SUM_SELF || op->mirror.on)) {
+    void **Wa = &op->t->dWa[sum == SUM_SELF];
+    b.npl = op->mirror.on ? op->N / 2 + 1 : op->N;
+    b.cfold = sum == SUM_SELF;
+    if (!*Wa && !ss->fixed) {
+      HIPCHK(hipMalloc(Wa, spbte_any_table_bytes(op->N, b.npl, b.cfold)));
+      op->gen++;
+      LCHK(spbte_launch_fold_any(op->t->dW64, *Wa, op->N, b.npl, b.cfold, &op->mirror, op->s));
+    }
+    if (*Wa) { /* else an allocation-free call before the first of its kind: the whole table, which is always there */
+      int k = spbte_any_slices(op->N, b.npl, b.cfold, a->nprod, a->ncell);
+      void *Qp = NULL;
+      const size_t one = (size_t)a->ncell * op->n3 * 16;
+      if (ss->fixed) {
+        k = ss->kind;
+        Qp = ss->Qp;
+      } else if (k > 1) {
+        int rc = ensure_partials(op, one * k);
+        if (rc) return rc;
+        Qp = op->d_Qp;
+      }
+      LCHK(spbte_launch_wsum_any(op->N, a, *Wa, k, Qp, op->s));
+      res->npl = b.npl;
+      if (a->keep_slices && k > 1) {
+        res->q = Qp;
+        res->nsl = k;
+      }
+      return SPBTE_OK;
+    }
+    b.npl = b.cfold = 0;
+  }
   const void *W;
   int rc = weights_form(op, form, !ss->fixed, &W, &rs);
   if (rc) return rc;
@@ -1083,9 +1119,9 @@ static int compute_chunk(spbte_op *op, const double *d_f, const double *d_g, dou
   }
   LCHK(spbte_launch_xform_fwd(&g, jobs, nj, ncell, fg_bytes(form) == 8, ss->xs, op->s));
   if (ev_a) HIPCHK(hipEventRecord(ev_a, op->s));
-  /* FFT grids: the inverse transform adds the split sum's slices itself */
+  /* the inverse transform adds the split sum's slices itself */
   wsum_result r;
-  int rc = run_wsum(op, form, mp ? 2 : 1, F0, G0, F1, G1, ncell, sum, ss, fused && !(flags & FULL_QHAT), &r);
+  int rc = run_wsum(op, form, mp ? 2 : 1, F0, G0, F1, G1, ncell, sum, ss, !(flags & FULL_QHAT), &r);
   if (ev_b) HIPCHK(hipEventRecord(ev_b, op->s));
   if (rc) return rc;
   const int cons = (flags & SPBTE_CONSERVE) != 0;
@@ -1193,6 +1229,10 @@ int spbte_compute_q_noalloc(spbte_op *op, const double *d_f, const double *d_g, 
   spbte_tile dt;
   const int is_default = have && default_stream_tile(op->N, form, mp ? 2 : 1, ncell, &dt) && !memcmp(&dt, &t, sizeof t);
   while (is_default && kind > 1 && b_fix + al256(16 * n * (size_t)kind) > op->nac_bytes) kind--;
+  if (!have && spbte_any_supported(op->N) && (self || op->mirror.on)) { /* likewise */
+    kind = spbte_any_slices(op->N, op->mirror.on ? op->N / 2 + 1 : op->N, self, mp ? 2 : 1, ncell);
+    while (kind > 1 && b_fix + al256(16 * n * (size_t)kind) > op->nac_bytes) kind--;
+  }
   const size_t b_qp = kind > 1 ? 16 * n * (size_t)kind : 0;
   const size_t b_x = al256(b_xs > b_qp ? b_xs : b_qp);
   const size_t need = b_fix + b_x;

@@ -73,6 +73,39 @@ def test_folded_sum_against_whole_sum(spb, orc, N, mp, pair):
     op.close()
 
 
+@pytest.mark.parametrize("N,grid,n", [(2, "0d", 3), (3, "0d", 2), (6, "0d", 5), (8, "1d", 64), (9, "0d", 3), (9, "1d", 3),
+                                      (10, "0d", 7), (10, "shifted", 2), (12, "0d", 1), (14, "0d", 33), (15, "0d", 2),
+                                      (15, "1d", 2), (18, "0d", 2), (20, "1d", 1), (23, "0d", 2)])
+def test_folded_sum_other_grids_against_oracle(spb, orc, N, grid, n):
+    """Grids without streaming tiles: even and odd, with the mirror symmetry and without (the 1D grid of
+    odd N), one and two cells a workgroup, planes of one to nine waves."""
+    op, v, eta, W = _op(spb, orc, N, grid, 10)
+    f, g = _cells(N, n, 11), _cells(N, n, 12)
+    some = sorted({0, n // 2, n - 1})
+    for mp in (False, True):
+        q = orc.compute_q_maxpreserve if mp else orc.compute_q
+        for h in (f, g):
+            got = op.compute_q(f, None if h is f else g, maxpreserve=mp)
+            ref = np.stack([q(N, v, eta, W, f[b], h[b]).ravel() for b in some])
+            assert rel_l2(got[some], ref) < 1e-12, (mp, h is g)
+    op.close()
+
+
+def test_noalloc_before_the_folded_table(spb, orc):
+    """An allocation-free call on a grid without streaming tiles needs nothing resident: it sums the whole table then."""
+    N = 10
+    op, v, eta, W = _op(spb, orc, N, "0d", 13)
+    f = _cells(N, 3, 14)
+    d_f, d_Q = spb.DeviceArray.from_host(f), spb.DeviceArray(f.shape)
+    ref = np.stack([orc.compute_q(N, v, eta, W, x, x).ravel() for x in f])
+    for _ in range(2):   # before and after the table is there
+        assert spb.lib().spbte_compute_q_noalloc(op.h, d_f.ptr, None, d_Q.ptr, 3, 0, spb.SELF) == 0
+        op.sync()
+        assert rel_l2(d_Q.download(), ref) < 1e-12
+        assert rel_l2(op.compute_q(f), ref) < 1e-12
+    op.close()
+
+
 def test_qhat_of_complex_operands_is_whole(spb, orc):
     """spbte_qhat takes any operands and returns every mode: it never folds, whatever compute_q built before."""
     N = 16
