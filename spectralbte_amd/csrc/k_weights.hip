@@ -11,15 +11,162 @@
 // The reference integrates every entry with GSL QAG (GAUSS21, 1e-8/1e-8): CPU-
 // days at N=32 (1.07e9 entries).  Here lam = 0 and lam = 1 use the closed forms
 // of the integral (gain - loss), one thread per entry; any other lam uses a
-// composite 64-panel x 20-point Gauss-Legendre rule per entry.
+// composite 64-panel x 20-point Gauss-Legendre rule per distinct entry.
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include <algorithm>
+#include <cmath>
+#include <new>
 #include <vector>
 
 #include "spbte_internal.h"
 
 namespace {
+
+// ---- Entries and their images.  The integrals of every table depend on the row
+// mode zeta and the column mode xi through |zeta|, |xi| and zeta.xi alone, so they
+// are the same for both modes with one permutation and one choice of signs of the
+// three axes applied to both.  Where the N modes of an axis are fewer absolute
+// values (na of them), the quadrature kernels compute only the rows
+// a >= b >= c >= 0 (R = na (na + 1) (na + 2) / 6) against all signed columns (E^3,
+// E = 2 na less one if zero is a mode: one more than N for even N, whose mode -N/2
+// has no mirror image), and k_expand writes every entry from its image: 1/21 of the
+// entries at N = 16, 1/31 at N = 32.  Generation on an MI355X, before and after:
+// Landau N = 16 160.7 -> 9.1 ms, N = 32 10.67 -> 0.356 s; glance 69.2 -> 11.9 ms, 4.61
+// -> 0.190 s; isotropic with lambda = 0.5 247.5 -> 13.0 ms, 15.8 -> 0.522 s.  (A table
+// of lambda = 0 or 1 in closed form takes 0.4 ms and 19 ms either way and stays as it is.)  Modes of equal absolute value to 1e-12 of the
+// largest count as equal (they differ by the rounding of -L_eta + i h_eta).
+struct AxisClasses {
+  int na, zero;                       // absolute values; 1 if zero is the first
+  int E;                              // signed values
+  unsigned char cls[SPBTE_MAX_N];     // class of mode i
+  signed char sgn[SPBTE_MAX_N];       // its sign (+1 for zero)
+};
+__host__ __device__ inline int axis_slot(const AxisClasses &a, int c, int s) {
+  return a.zero ? a.na - 1 + s * c : (s > 0 ? a.na + c : a.na - 1 - c);
+}
+__host__ __device__ inline long row_rank(int a, int b, int c) { return (long)a * (a + 1) * (a + 2) / 6 + b * (b + 1) / 2 + c; }
+
+// The isotropic table's factors of an entry: the trapezoid weights of its column, dfac and P.
+__device__ __forceinline__ double iso_entry(int N, int l, int m, int n, double dfac, double P, double I) {
+  const double wl = (l == 0 || l == N - 1) ? 0.5 : 1.0, wm = (m == 0 || m == N - 1) ? 0.5 : 1.0,
+               wn = (n == 0 || n == N - 1) ? 0.5 : 1.0;
+  return wl * wm * wn * dfac * (P * I);
+}
+
+// One row r per blockIdx.x: W[r][c] = U[image of r][image of c] (iso: times iso_entry's factors).
+__global__ void __launch_bounds__(256) k_expand(int N, AxisClasses ax, const double *__restrict__ U, bool iso, double dfac,
+                                                double P, double *__restrict__ W) {
+  const int n2 = N * N, n3 = n2 * N;
+  const int r = blockIdx.x, q[3] = {r / n2, r / N % N, r % N};
+  int p[3] = {0, 1, 2};  // axes by descending class
+  if (ax.cls[q[p[0]]] < ax.cls[q[p[1]]]) { const int t = p[0]; p[0] = p[1]; p[1] = t; }
+  if (ax.cls[q[p[1]]] < ax.cls[q[p[2]]]) { const int t = p[1]; p[1] = p[2]; p[2] = t; }
+  if (ax.cls[q[p[0]]] < ax.cls[q[p[1]]]) { const int t = p[0]; p[0] = p[1]; p[1] = t; }
+  const int E = ax.E;
+  const double *Ur = U + row_rank(ax.cls[q[p[0]]], ax.cls[q[p[1]]], ax.cls[q[p[2]]]) * E * E * E;
+  // slot of every mode on each sorted axis
+  __shared__ int slot[3][SPBTE_MAX_N];
+  for (int e = threadIdx.x; e < 3 * N; e += 256) {
+    const int d = e / N, i = e - d * N;
+    slot[d][i] = axis_slot(ax, ax.cls[i], ax.sgn[q[p[d]]] * ax.sgn[i]);
+  }
+  __syncthreads();
+  for (int c = threadIdx.x; c < n3; c += 256) {
+    const int x[3] = {c / n2, c / N % N, c % N};
+    int s[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) s[d] = slot[d][p[d] == 0 ? x[0] : (p[d] == 1 ? x[1] : x[2])];
+    double w = Ur[((long)s[0] * E + s[1]) * E + s[2]];
+    if (iso) w = iso_entry(N, x[0], x[1], x[2], dfac, P, w);
+    W[(size_t)r * n3 + c] = w;
+  }
+}
+
+// What a quadrature kernel computes: R rows zeta (3 values each) against E^3
+// columns with the axis values ex, into out.
+struct Entries {
+  long R;
+  int E;
+  double *rows, *ex, *out;  // device
+  bool direct;              // out is the table itself
+};
+
+// Runs compute(Entries) over the distinct entries and writes the table; over the
+// whole table itself (direct: rows and columns are the modes in their order) where
+// the modes are not symmetric (no fewer entries) or there is no room for the rest.
+template <class F>
+int with_entries(int N, const double *eta, bool iso, double dfac, double P, double *W, hipStream_t s, F compute) {
+  const long n3 = (long)N * N * N;
+  AxisClasses ax = {};
+  std::vector<double> A, ex, rows;
+  double *buf = nullptr;
+  Entries en = {};
+  try {
+    double emax = 0.0;
+    bool finite = true;
+    for (int i = 0; i < N; ++i) {
+      emax = fmax(emax, fabs(eta[i]));
+      finite = finite && std::isfinite(eta[i]);
+    }
+    for (int i = 0; i < N && finite; ++i) ex.push_back(fabs(eta[i]));
+    std::sort(ex.begin(), ex.end());
+    for (double x : ex)
+      if (A.empty() || x - A.back() > 1e-12 * emax) A.push_back(x);
+    ax.na = (int)A.size();
+    ax.zero = finite && A[0] <= 1e-12 * emax;
+    for (int i = 0; i < N && finite; ++i) {
+      int k = 0;
+      while (k + 1 < ax.na && fabs(eta[i]) - A[k] > 1e-12 * emax) ++k;
+      ax.cls[i] = (unsigned char)k;
+      ax.sgn[i] = eta[i] < 0 && !(ax.zero && k == 0) ? -1 : 1;
+    }
+    ax.E = 2 * ax.na - ax.zero;
+    en = {(long)ax.na * (ax.na + 1) * (ax.na + 2) / 6, ax.E, nullptr, nullptr, nullptr, !finite};
+    en.direct = en.direct || (double)en.R * ax.E * ax.E * ax.E >= (double)n3 * n3;
+    for (;;) {
+      rows.clear();
+      if (en.direct) {
+        en.R = n3;
+        en.E = N;
+        ex.assign(eta, eta + N);
+        for (long r = 0; r < n3; ++r)
+          for (long v : {r / ((long)N * N), r / N % N, r % N}) rows.push_back(eta[v]);
+      } else {
+        ex.assign(ax.E, 0.0);
+        for (int k = 0; k < ax.na; ++k) {
+          if (k || !ax.zero) ex[axis_slot(ax, k, -1)] = -A[k];
+          ex[axis_slot(ax, k, 1)] = A[k];
+        }
+        for (int a = 0; a < ax.na; ++a)
+          for (int b = 0; b <= a; ++b)
+            for (int c = 0; c <= b; ++c)
+              for (int k : {a, b, c}) rows.push_back(A[k]);
+      }
+      rows.insert(rows.end(), ex.begin(), ex.end());
+      const size_t nu = en.direct ? 0 : (size_t)en.R * en.E * en.E * en.E;
+      const hipError_t e = hipMalloc((void **)&buf, sizeof(double) * (rows.size() + nu));
+      if (e == hipSuccess) break;
+      if (en.direct) return (int)e;
+      (void)hipGetLastError();
+      en.direct = true;
+    }
+  } catch (const std::bad_alloc &) {
+    return (int)hipErrorOutOfMemory;
+  }
+  en.rows = buf;
+  en.ex = buf + 3 * en.R;
+  en.out = en.direct ? W : buf + rows.size();
+  hipError_t e = hipMemcpyAsync(buf, rows.data(), sizeof(double) * rows.size(), hipMemcpyHostToDevice, s);
+  if (e == hipSuccess) e = (hipError_t)compute(en);
+  if (e == hipSuccess && !en.direct) {
+    hipLaunchKernelGGL(k_expand, dim3((unsigned)n3), dim3(256), 0, s, N, ax, en.out, iso, dfac, P, W);
+    e = hipGetLastError();
+  }
+  const hipError_t e2 = hipStreamSynchronize(s), e3 = hipFree(buf);
+  return e != hipSuccess ? (int)e : (e2 != hipSuccess ? (int)e2 : (int)e3);
+}
 
 __device__ __forceinline__ double sinc(double x) { return (x != 0.0) ? sin(x) / x : 1.0; }
 __device__ __forceinline__ double fcos(double x) { return (fabs(x) > 1e-12) ? (cos(x) - 1.0) / (x * x) : -0.5 + x * x / 24.0; }
@@ -80,8 +227,25 @@ __device__ double integral_gl(double a0, double a1, double a2, double L, double 
   return sum;
 }
 
+// Any other lam: the quadrature alone, over distinct entries.
+__global__ void __launch_bounds__(256) k_weights_iso_gl(int E, const double *__restrict__ rows,
+                                                        const double *__restrict__ ex, long r0, long nrows, double L,
+                                                        double lam, double mu, GL20 q, bool direct, double dfac,
+                                                        double P, double *__restrict__ out) {
+  const long n3 = (long)E * E * E;
+  const long e = (long)blockIdx.x * 256 + threadIdx.x;
+  if (e >= nrows * n3) return;
+  const long r = r0 + e / n3, c = e % n3;
+  const double z1 = rows[3 * r], z2 = rows[3 * r + 1], z3 = rows[3 * r + 2];
+  const double k1 = ex[c / ((long)E * E)], k2 = ex[(c / E) % E], k3 = ex[c % E];
+  const double a0 = mu * sqrt(z1 * z1 + z2 * z2 + z3 * z3), a1 = sqrt(k1 * k1 + k2 * k2 + k3 * k3);
+  const double d1 = k1 - mu * z1, d2 = k2 - mu * z2, d3 = k3 - mu * z3;
+  const double I = integral_gl(a0, a1, sqrt(d1 * d1 + d2 * d2 + d3 * d3), L, lam, q);
+  out[e] = direct ? iso_entry(E, (int)(c / ((long)E * E)), (int)((c / E) % E), (int)(c % E), dfac, P, I) : I;
+}
+
 __global__ void __launch_bounds__(256) k_weights_iso(int N, const double *__restrict__ eta, double L, double lam, double P,
-                                                     double dfac, double mu, GL20 q, unsigned chunks,
+                                                     double dfac, double mu, unsigned chunks,
                                                      double *__restrict__ W) {
   const size_t n3 = (size_t)N * N * N;
   const size_t r = blockIdx.x / chunks;                 // one row per `chunks` workgroups
@@ -97,11 +261,8 @@ __global__ void __launch_bounds__(256) k_weights_iso(int N, const double *__rest
     const double a2 = sqrt(d1 * d1 + d2 * d2 + d3 * d3);
     double I;
     if (lam == 0.0) I = gain0(a0, a2, L) - loss0(a1, L);
-    else if (lam == 1.0) I = gain1(a0, a2, L) - loss1(a1, L);
-    else I = integral_gl(a0, a1, a2, L, lam, q);
-    const double wl = (l == 0 || l == N - 1) ? 0.5 : 1.0, wm = (m == 0 || m == N - 1) ? 0.5 : 1.0,
-                 wn = (n == 0 || n == N - 1) ? 0.5 : 1.0;
-    W[r * n3 + c] = wl * wm * wn * dfac * (P * I);
+    else I = gain1(a0, a2, L) - loss1(a1, L);
+    W[r * n3 + c] = iso_entry(N, l, m, n, dfac, P, I);
   }
 }
 
@@ -154,13 +315,14 @@ __device__ __forceinline__ double landau_g(double r, double a0, double a1, doubl
   return st * j0(r * a0 * st) * (-r * r * a1 * st * st * cv + 4 * r * a3 * sv * ct);
 }
 
-__global__ void __launch_bounds__(256) k_weights_landau(int N, const double *__restrict__ eta, long r0, long nrows,
+__global__ void __launch_bounds__(256) k_weights_landau(int N, const double *__restrict__ rows,
+                                                        const double *__restrict__ eta, long r0, long nrows,
                                                         LandauRule q, double *__restrict__ W) {
   const long n3 = (long)N * N * N;
   const long e = (long)blockIdx.x * 256 + threadIdx.x;
   if (e >= nrows * n3) return;
   const long r = r0 + e / n3, c = e % n3;
-  const double z1 = eta[r / ((long)N * N)], z2 = eta[(r / N) % N], z3 = eta[r % N];
+  const double z1 = rows[3 * r], z2 = rows[3 * r + 1], z3 = rows[3 * r + 2];
   const double x1 = eta[c / ((long)N * N)], x2 = eta[(c / N) % N], x3 = eta[c % N];
   const double zetalen2 = z3 * z3 + z2 * z2 + z1 * z1;
   const double xilen2 = x1 * x1 + x2 * x2 + x3 * x3;
@@ -208,10 +370,8 @@ void gauss_legendre_half(int n, double *x, double *w) {
 
 }  // namespace
 
-extern "C" int spbte_launch_weights_landau(const spbte_grid_dev *g, const double *eta, double lam, double *W,
+extern "C" int spbte_launch_weights_landau(const spbte_grid_dev *g, const double *eta_host, double lam, double *W,
                                            hipStream_t s) {
-  const int N = g->N;
-  const long n3 = (long)N * N * N;
   LandauRule q;
   double x[32];
   gauss_legendre_half(64, x, q.w);
@@ -227,16 +387,19 @@ extern "C" int spbte_launch_weights_landau(const spbte_grid_dev *g, const double
     q.rl_p[k] = pow(q.r_p[k], lam + 2);
     q.rl_m[k] = pow(q.r_m[k], lam + 2);
   }
-  // rows per launch: about 8M entries (a fraction of a second each at N = 32)
-  const long rows = n3 >= (8L << 20) ? 1 : (8L << 20) / n3;
-  for (long r0 = 0; r0 < n3; r0 += rows) {
-    const long nr = r0 + rows <= n3 ? rows : n3 - r0;
-    const unsigned blocks = (unsigned)((nr * n3 + 255) / 256);
-    hipLaunchKernelGGL(k_weights_landau, dim3(blocks), dim3(256), 0, s, N, eta, r0, nr, q, W + r0 * n3);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return (int)e;
-  }
-  return 0;
+  return with_entries(g->N, eta_host, false, 0.0, 0.0, W, s, [&](const Entries &en) {
+    const long n3 = (long)en.E * en.E * en.E;
+    // rows per launch: about 8M entries
+    const long rows = n3 >= (8L << 20) ? 1 : (8L << 20) / n3;
+    for (long r0 = 0; r0 < en.R; r0 += rows) {
+      const long nr = r0 + rows <= en.R ? rows : en.R - r0;
+      const unsigned blocks = (unsigned)((nr * n3 + 255) / 256);
+      hipLaunchKernelGGL(k_weights_landau, dim3(blocks), dim3(256), 0, s, en.E, en.rows, en.ex, r0, nr, q, en.out + r0 * n3);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return (int)e;
+    }
+    return 0;
+  });
 }
 
 // ---- Glancing-collision table (glance g > 0): gHat3 of
@@ -334,7 +497,8 @@ __host__ __device__ inline int glance_pofs(int k) { return 8 * k * (k - 1) + 2 *
 // table (nD panels) at dofs: the first nlds doubles, copied to LDS; then the
 // E1, E2, E3 tables (nE panels each), read in place.
 constexpr int kGlanceThreads = 256;
-__global__ void __launch_bounds__(kGlanceThreads) k_weights_glance(int N, const double *__restrict__ eta, long r0, long nrows,
+__global__ void __launch_bounds__(kGlanceThreads) k_weights_glance(int N, const double *__restrict__ rows,
+                                                        const double *__restrict__ eta, long r0, long nrows,
                                                         const double *__restrict__ rule, GlanceDims d,
                                                         double *__restrict__ W) {
   extern __shared__ double sm[];
@@ -346,7 +510,7 @@ __global__ void __launch_bounds__(kGlanceThreads) k_weights_glance(int N, const 
   const long e = (long)blockIdx.x * kGlanceThreads + threadIdx.x;
   if (e >= nrows * n3) return;
   const long r = r0 + e / n3, c = e % n3;
-  const double z1 = eta[r / ((long)N * N)], z2 = eta[(r / N) % N], z3 = eta[r % N];
+  const double z1 = rows[3 * r], z2 = rows[3 * r + 1], z3 = rows[3 * r + 2];
   const double x1 = eta[c / ((long)N * N)], x2 = eta[(c / N) % N], x3 = eta[c % N];
   // geometry as gHat3 (:165-183)
   const double zetalen2 = z1 * z1 + z2 * z2 + z3 * z3;
@@ -491,10 +655,9 @@ void poly_table(int P, double h, F f, std::vector<double> &out) {
 }  // namespace
 
 // The glance table: 0 < g < pi (log sin(g/2) < 0), checked by the caller.
-extern "C" int spbte_launch_weights_glance(const spbte_grid_dev *g, const double *eta_host, const double *eta,
-                                           double lam, double glance, double *W, hipStream_t s) {
+extern "C" int spbte_launch_weights_glance(const spbte_grid_dev *g, const double *eta_host, double lam, double glance,
+                                           double *W, hipStream_t s) {
   const int N = g->N;
-  const long n3 = (long)N * N * N;
   const double L = g->Lv;
   double emax = 0.0;
   for (int i = 0; i < N; ++i) emax = fmax(emax, fabs(eta_host[i]));
@@ -560,28 +723,46 @@ extern "C" int spbte_launch_weights_glance(const spbte_grid_dev *g, const double
   hipError_t e = hipMalloc((void **)&drule, bytes);
   if (e != hipSuccess) return (int)e;
   e = hipMemcpy(drule, buf.data(), bytes, hipMemcpyHostToDevice);
-  // rows per launch: about 4M entries
-  const long rows = n3 >= (4L << 20) ? 1 : (4L << 20) / n3;
-  for (long r0 = 0; e == hipSuccess && r0 < n3; r0 += rows) {
-    const long nr = r0 + rows <= n3 ? rows : n3 - r0;
-    const unsigned blocks = (unsigned)((nr * n3 + kGlanceThreads - 1) / kGlanceThreads);
-    hipLaunchKernelGGL(k_weights_glance, dim3(blocks), dim3(kGlanceThreads), lds, s, N, eta, r0, nr, drule, d,
-                       W + r0 * n3);
-    e = hipGetLastError();
-  }
+  if (e == hipSuccess)
+    e = (hipError_t)with_entries(N, eta_host, false, 0.0, 0.0, W, s, [&](const Entries &en) {
+      // rows per launch: about 4M entries
+      const long n3 = (long)en.E * en.E * en.E, rows = n3 >= (4L << 20) ? 1 : (4L << 20) / n3;
+      for (long r0 = 0; r0 < en.R; r0 += rows) {
+        const long nr = r0 + rows <= en.R ? rows : en.R - r0;
+        const unsigned blocks = (unsigned)((nr * n3 + kGlanceThreads - 1) / kGlanceThreads);
+        hipLaunchKernelGGL(k_weights_glance, dim3(blocks), dim3(kGlanceThreads), lds, s, en.E, en.rows, en.ex, r0, nr,
+                           drule, d, en.out + r0 * n3);
+        const hipError_t el = hipGetLastError();
+        if (el != hipSuccess) return (int)el;
+      }
+      return 0;
+    });
   const hipError_t e2 = hipStreamSynchronize(s), e3 = hipFree(drule);
   return e != hipSuccess ? (int)e : (e2 != hipSuccess ? (int)e2 : (int)e3);
 }
 
-extern "C" int spbte_launch_weights_iso(const spbte_grid_dev *g, const double *eta, double lam, double dfac, double mu,
+extern "C" int spbte_launch_weights_iso(const spbte_grid_dev *g, const double *eta_host, const double *eta, double lam, double dfac, double mu,
                                         double *W, hipStream_t s) {
   const int N = g->N;
   const size_t n3 = (size_t)N * N * N;
   const double P = 16.0 * M_PI * M_PI * g->heta * g->heta * g->heta / pow(2.0 * M_PI, 1.5) / (4.0 * M_PI);
-  GL20 q;
-  gauss_legendre20(q);
+  if (lam != 0.0 && lam != 1.0) {
+    GL20 q;
+    gauss_legendre20(q);
+    return with_entries(N, eta_host, true, dfac, P, W, s, [&](const Entries &en) {
+      const long m3 = (long)en.E * en.E * en.E, rows = m3 >= (8L << 20) ? 1 : (8L << 20) / m3;
+      for (long r0 = 0; r0 < en.R; r0 += rows) {
+        const long nr = r0 + rows <= en.R ? rows : en.R - r0;
+        hipLaunchKernelGGL(k_weights_iso_gl, dim3((unsigned)((nr * m3 + 255) / 256)), dim3(256), 0, s, en.E, en.rows,
+                           en.ex, r0, nr, g->Lv, lam, mu, q, en.direct, dfac, P, en.out + r0 * m3);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return (int)e;
+      }
+      return 0;
+    });
+  }
   const unsigned chunks = (unsigned)((n3 + 255) / 256 < 64 ? (n3 + 255) / 256 : 64);
-  hipLaunchKernelGGL(k_weights_iso, dim3((unsigned)(n3 * chunks)), dim3(256), 0, s, N, eta, g->Lv, lam, P, dfac, mu, q, chunks,
+  hipLaunchKernelGGL(k_weights_iso, dim3((unsigned)(n3 * chunks)), dim3(256), 0, s, N, eta, g->Lv, lam, P, dfac, mu, chunks,
                      W);
   return (int)hipGetLastError();
 }

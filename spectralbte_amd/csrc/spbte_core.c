@@ -613,7 +613,7 @@ int spbte_op_generate_weights_iso(spbte_op *op, double lambda, double d_i, doubl
   HIPCHK(hipMemcpy(d_eta, op->eta, sizeof(double) * op->N, hipMemcpyHostToDevice));
   const double dfac = 0.25 * pow(0.5 * (d_i + d_j), 2); /* src/weights.c:277 */
   const double mu = m_j / (m_i + m_j);                  /* src/weights.c:190 */
-  int e = spbte_launch_weights_iso(&op->g, d_eta, lambda, dfac, mu, op->t->dW64, op->s);
+  int e = spbte_launch_weights_iso(&op->g, op->eta, d_eta, lambda, dfac, mu, op->t->dW64, op->s);
   hipError_t e2 = hipStreamSynchronize(op->s);
   hipFree(d_eta);
   if (e != 0 || e2 != hipSuccess)
@@ -626,12 +626,8 @@ int spbte_op_generate_weights_landau(spbte_op *op, double lambda) {
   if (!op || !isfinite(lambda)) return fail(SPBTE_ERR_ARG, "bad arguments");
   int rc = alloc_w64(op);
   if (rc) return rc;
-  double *d_eta = NULL;
-  HIPCHK(hipMalloc((void **)&d_eta, sizeof(double) * op->N));
-  HIPCHK(hipMemcpy(d_eta, op->eta, sizeof(double) * op->N, hipMemcpyHostToDevice));
-  int e = spbte_launch_weights_landau(&op->g, d_eta, lambda, op->t->dW64, op->s);
+  int e = spbte_launch_weights_landau(&op->g, op->eta, lambda, op->t->dW64, op->s);
   hipError_t e2 = hipStreamSynchronize(op->s);
-  hipFree(d_eta);
   if (e != 0 || e2 != hipSuccess)
     return fail(SPBTE_ERR_HIP, "Landau weight generation: %s", hipGetErrorString(e ? (hipError_t)e : e2));
   op->t->have_w = 1;
@@ -644,12 +640,8 @@ int spbte_op_generate_weights_glance(spbte_op *op, double lambda, double glance)
     return fail(SPBTE_ERR_ARG, "glance %g outside (0, pi), where log(sin(glance/2)) < 0", glance);
   int rc = alloc_w64(op);
   if (rc) return rc;
-  double *d_eta = NULL;
-  HIPCHK(hipMalloc((void **)&d_eta, sizeof(double) * op->N));
-  HIPCHK(hipMemcpy(d_eta, op->eta, sizeof(double) * op->N, hipMemcpyHostToDevice));
-  int e = spbte_launch_weights_glance(&op->g, op->eta, d_eta, lambda, glance, op->t->dW64, op->s);
+  int e = spbte_launch_weights_glance(&op->g, op->eta, lambda, glance, op->t->dW64, op->s);
   hipError_t e2 = hipStreamSynchronize(op->s);
-  hipFree(d_eta);
   if (e != 0 || e2 != hipSuccess)
     return fail(SPBTE_ERR_HIP, "glancing-collision weight generation: %s", hipGetErrorString(e ? (hipError_t)e : e2));
   op->t->have_w = 1;
