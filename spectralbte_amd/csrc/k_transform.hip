@@ -44,6 +44,30 @@ struct XformJobs {
   spbte_xform_job j[4];
 };
 
+// x += the sets from..nsl-1, sstride apart, in set order, U loads in flight.
+template <int U>
+__device__ __forceinline__ void add_slices(double2 &x, const double2 *in, int from, int nsl, size_t sstride) {
+  for (int sl = from; sl < nsl; sl += U) {
+    double2 y[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) y[u] = sl + u < nsl ? in[(size_t)(sl + u) * sstride] : make_double2(0.0, 0.0);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (sl + u < nsl) {
+        x.x += y[u].x;
+        x.y += y[u].y;
+      }
+  }
+}
+// One element of the sum of nsl sets: 8 loads in flight for a batch's few slices, 32
+// for one cell's many (64 at N = 16, read by the 9 workgroups of its kept planes).
+__device__ __forceinline__ double2 sum_slices(const double2 *in, int nsl, size_t sstride) {
+  double2 x = in[0];
+  if (nsl <= 17) add_slices<8>(x, in, 1, nsl, sstride);
+  else add_slices<32>(x, in, 1, nsl, sstride);
+  return x;
+}
+
 // Maxwellian of src/collisions.c:98-103 at grid point (i, j, k).
 __device__ __forceinline__ double maxwellian_at(const double *mom, const double *v, int i, int j, int k) {
   const double ux = mom[1], uy = mom[2], uz = mom[3], T = mom[4], pre = mom[5];
@@ -132,13 +156,7 @@ __global__ void __launch_bounds__(XT) k_xform_a_cplx(int N, const double2 *in, i
   double2 *X = sm, *T1 = sm + n2;
   for (int e = threadIdx.x; e < n2; e += XT) {
     const size_t o = cell * n3 + (size_t)i * n2 + e;
-    double2 x = in[o];
-    for (int sl = 1; sl < nsl; ++sl) {
-      const double2 y = in[(size_t)sl * sstride + o];
-      x.x += y.x;
-      x.y += y.y;
-    }
-    X[e] = x;
+    X[e] = sum_slices(in + o, nsl, sstride);
   }
   __syncthreads();
   plane_zy(N, M, X, T1, scratch + (size_t)cell * n3 + (size_t)i * n2);
@@ -412,18 +430,7 @@ __global__ void __launch_bounds__(XT) k_fft_a_cplx(const double2 *in, int nsl, i
   for (int e = threadIdx.x; e < n2; e += XT) {
     const int j = e / N, k = e - j * N;
     const size_t o = cell * n3 + (size_t)i * n2 + e;
-    double2 x = in[o];
-    for (int sl = 1; sl < nsl; sl += 8) {  // up to eight loads in flight, added in set order
-      double2 y[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) y[u] = sl + u < nsl ? in[(size_t)(sl + u) * sstride + o] : make_double2(0.0, 0.0);
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (sl + u < nsl) {
-          x.x += y[u].x;
-          x.y += y[u].y;
-        }
-    }
+    const double2 x = sum_slices(in + o, nsl, sstride);
     A[e] = cmul(x, cmul(cmul(pi_, t.p[j]), t.p[k]));
   }
   __syncthreads();

@@ -12,8 +12,10 @@
 //    time, so G_b[c] is wave-uniform: it is read straight from global memory
 //    with scalar loads (no LDS traffic, no vector registers; staging the G
 //    x-planes in LDS held 32 KiB per workgroup and twice the LDS reads), except
-//    with FP64 weights and one product, where the G lines passing through L2
-//    crowd out the 8-byte W stream and the x-plane is staged in LDS instead;
+//    at N = 32 with FP64 weights and one product, where the G lines passing
+//    through L2 crowd out the 8-byte W stream and the x-plane is staged in LDS
+//    instead (N = 24, 37 cells: 735 us an evaluation staged, 665 with scalar
+//    loads, which leave LDS for twice the workgroups);
 //  * along cz the shifted operand F_b[sy][rz + N/2 - cz] of a lane's TR rows is a
 //    window sliding by one element per cz step: it lives in registers and takes
 //    one LDS load per step, shared by TR rows (the F x-planes of the cells sit in
@@ -156,7 +158,7 @@ k_wsum_stream(const uint4 *__restrict__ Wp, const float *__restrict__ rowscale, 
   // 39.4 ms against 30.1 ms in the plain form).
   constexpr bool GS = FORM == 3 && NP == 2 && TB == 1;
   __shared__ float sP[GS ? NP * KB * P * N * LW : 1];
-  constexpr bool SG = FORM != 0 || NP == 2 || TB >= 4;  // G by scalar loads (else staged in LDS)
+  constexpr bool SG = FORM != 0 || NP == 2 || TB >= 4 || N < 32;  // G by scalar loads (else staged in LDS)
   __shared__ __attribute__((aligned(16))) C sG[SG ? 1 : NP * KB * N2];  // [p][k][cy][cz]
 
   // ---- workgroup -> (r-tile, cx slice, cell group), XCD-aware: workgroups are

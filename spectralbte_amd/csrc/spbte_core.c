@@ -845,12 +845,14 @@ static long stream_wgs(int N, int ncell, const spbte_tile *t) {
  *    one wave, 47 with 4 rows); then 4 rows, with one cell per lane for two
  *    products (600 cells: 1715 against 1920) and two for one.
  * The summed lines are split into at least 8 slices (16 with FP32 products at
- * N=32) and into as many as give 2400 workgroups, at most 32 (N=32), 48 (N=24),
- * 64 (N=16): a last round of workgroups that is nearly empty costs less, and the
- * slices of one r-tile keep nearer each other in the table (N=32, 512 cells with
- * FP32 products: 43930 us with one slice, 42060 with 4, 40000 with 16; 256 cells
- * ComputeQ in FP64: 22770 with one, 17910 with 4, 17530 with 8, 17910 with 16;
- * one cell, FP64: 553 with 8, 413 with 60).  The inverse transform adds them. */
+ * N=32 and one product at N=16, 12 with one product at N=24) and into as many as
+ * give 4000 workgroups, at most 32 (N=32), 48 (N=24), 64 (N=16): a last round of
+ * workgroups that is nearly empty costs less, and the slices of one r-tile keep
+ * nearer each other in the table (N=32, 512 cells with FP32 products: 43930 us
+ * with one slice, 42060 with 4, 40000 with 16; 256 cells ComputeQ in FP64: 22770
+ * with one, 17910 with 4, 17530 with 8, 17910 with 16; N=24, 37 cells ComputeQ: 756
+ * with 8, 693 with 12, 665 with 24; N=16, 48 cells, two arguments: 206 with 8, 183
+ * with 16, 172 with 32).  The inverse transform adds them. */
 static int default_stream_tile(int N, int form, int nprod, int ncell, spbte_tile *t) {
   static const spbte_tile s32[] = {{4, 4, 4, 1}, {4, 4, 2, 1}, {4, 4, 1, 1}}, s32m[] = {{4, 4, 2, 1}, {4, 4, 1, 1}};
   static const spbte_tile s24[] = {{3, 3, 2, 1}, {3, 3, 1, 1}};
@@ -869,11 +871,13 @@ static int default_stream_tile(int N, int form, int nprod, int ncell, spbte_tile
     if (form == SPBTE_FORM_FP32A) kmin = 16;
   } else if (N == 24) {
     kmax = 48;
+    if (nprod == 1) kmin = 12;
     const int one = nprod == 2 && form != SPBTE_FORM_FP32A;
     c = s24 + one;
     nc = 2 - one;
   } else if (N == 16) {
     kmax = 64;
+    if (nprod == 1) kmin = 16;
     const int one = nprod == 2 && form != SPBTE_FORM_FP32A;
     if (ncell <= 4) { c = s16few; nc = 2; }
     else { c = s16 + one; nc = 2 - one; }
@@ -884,11 +888,21 @@ static int default_stream_tile(int N, int form, int nprod, int ncell, spbte_tile
     *t = c[i];
     const long wgs = stream_wgs(N, ncell, t);
     t->kind = kmin;
-    for (int k = kmin; k <= kmax && wgs * t->kind < 2400; k++)
+    for (int k = kmin; k <= kmax && wgs * t->kind < 4000; k++)
       if (spbte_csplit_valid(N, k)) t->kind = k;
     return 1;
   }
   return 0;
+}
+
+/* Slices a tile's launch takes: its kind; where one cell group streams a table from
+ * HBM (N >= 24), the next number that fills whole rounds of the 256 CUs (one N=32
+ * cell, 17 workgroups a slice: 425 us with 32 slices, 404 with 30, 392 with 45). */
+static int tile_slices(int N, int ncell, const spbte_tile *t) {
+  const long wgs = stream_wgs(N, ncell, t);
+  if (t->kind < 16 || N < 24 || ncell > t->tb) return t->kind;
+  const long k = (wgs * t->kind + 255) / 256 * 256 / wgs;
+  return (int)(k > t->kind ? k : t->kind);
 }
 
 static int pick_tile(spbte_op *op, int ncell, int form, int nprod, spbte_tile *t) {
@@ -968,7 +982,7 @@ static int launch_tile(spbte_op *op, int form, const spbte_tile *t, const spbte_
     if (!Wp) rc = weights_permuted(op, form, t->tr, !ss->fixed, &Wp, &rs);
     if (rc) return rc;
     void *Qp = NULL;
-    const int k = ss->fixed && ss->kind ? ss->kind : t->kind;
+    const int k = ss->fixed && ss->kind ? ss->kind : tile_slices(op->N, a->ncell, t);
     if (k > 1) {
       const size_t need = (size_t)k * a->ncell * op->n3 * 16;
       if (ss->fixed) {
@@ -1217,7 +1231,7 @@ int spbte_compute_q_noalloc(spbte_op *op, const double *d_f, const double *d_g, 
   const size_t b_xs = 16 * n * (size_t)nj, b_fix = b_mom + b_part + b_fg + b_qh;
   /* a tile that was not pinned or tuned takes fewer slices where the workspace
    * does not hold its own number (the sums then differ by rounding) */
-  int kind = have ? t.kind : 0;
+  int kind = have ? (t.kind > 1 ? tile_slices(op->N, ncell, &t) : t.kind) : 0;
   spbte_tile dt;
   const int is_default = have && default_stream_tile(op->N, form, mp ? 2 : 1, ncell, &dt) && !memcmp(&dt, &t, sizeof t);
   while (is_default && kind > 1 && b_fix + al256(16 * n * (size_t)kind) > op->nac_bytes) kind--;
