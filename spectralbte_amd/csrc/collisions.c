@@ -3,9 +3,11 @@
  * Replaces src/collisions.c.  Module state stays file-static and one grid per
  * process, as in the reference (src/collisions.c:11-30), but the operator runs
  * on the GPU: each call uploads f and g, evaluates the operator with the
- * batched path of spbte_core.c for one cell and downloads Q.  The copies go
- * through a pinned host buffer as asynchronous copies on the operator's
- * stream, so a call waits for the GPU once.  Weight tables
+ * batched path of spbte_core.c for one cell and downloads Q, through a pinned
+ * host buffer on the operator's stream, so a call waits for the GPU once.  Up to
+ * SPBTE_PINNED_DIRECT a kernel fetches f and g from that buffer and the
+ * evaluation's last pass writes Q into it (an N=16 ComputeQ_maxPreserve and its
+ * projection: see conserve.c); beyond, they are asynchronous copies.  Weight tables
  * are cached in HBM keyed by the conv_weights pointer (the reference passes the
  * same pointer every step, exec/boltz.c:196,288), so an N=32 table (8.6 GB)
  * crosses PCIe once.
@@ -172,12 +174,22 @@ static void run_q(double *f, double *g, double *Q, double **conv_weights, int fl
   spbte_op *op = op_for(conv_weights);
   hipStream_t s = spbte_op_stream(op);
   const size_t n3 = (size_t)N * N * N, b = sizeof(double) * n3;
-  double *df = d_buf, *dg = d_buf + n3, *dQ = d_buf + 2 * n3;
-  stage_in(df, h_buf, f, b, s, "ComputeQ");
-  if (g != f) stage_in(dg, h_buf + n3, g, b, s, "ComputeQ");
+  const int direct = b <= SPBTE_PINNED_DIRECT, two = g != f;
+  double *df = d_buf, *dg = d_buf + n3, *dQ = direct ? h_buf + 2 * n3 : d_buf + 2 * n3;
+  if (direct) {
+    memcpy(h_buf, f, b);
+    if (two) memcpy(h_buf + n3, g, b);
+    hip_ok((hipError_t)spbte_launch_copy_cell(h_buf, d_buf, two ? 2 * n3 : n3, s), "ComputeQ");
+  } else {
+    stage_in(df, h_buf, f, b, s, "ComputeQ");
+    if (two) stage_in(dg, h_buf + n3, g, b, s, "ComputeQ");
+  }
   if (spbte_compute_q(op, df, g == f ? df : dg, dQ, 1, form_from_env(), flags | (g == f ? SPBTE_SELF : 0)) != SPBTE_OK)
     die("ComputeQ");
-  finish_out(Q, h_buf + 2 * n3, dQ, b, s, "ComputeQ");
+  if (direct) {
+    hip_ok(hipStreamSynchronize(s), "ComputeQ");
+    memcpy(Q, dQ, b);
+  } else finish_out(Q, h_buf + 2 * n3, dQ, b, s, "ComputeQ");
 }
 
 void ComputeQ(double *f, double *g, double *Q, double **conv_weights) { run_q(f, g, Q, conv_weights, 0); }

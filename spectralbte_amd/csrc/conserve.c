@@ -129,11 +129,13 @@ void conserveAllMoments(double **Q) {
   const size_t n3 = (size_t)N * N * N, na = (size_t)Ns * Ns;
   hipError_t e;
   for (size_t a = 0; a < na; a++) memcpy(h_Q + a * n3, Q[a], sizeof(double) * n3);
-  if ((e = hipMemcpyAsync(d_Q, h_Q, sizeof(double) * na * n3, hipMemcpyHostToDevice, stream)) != hipSuccess)
+  /* small arrays: both passes work on the pinned copy itself */
+  const int direct = sizeof(double) * na * n3 <= SPBTE_PINNED_DIRECT;
+  if (!direct && (e = hipMemcpyAsync(d_Q, h_Q, sizeof(double) * na * n3, hipMemcpyHostToDevice, stream)) != hipSuccess)
     die("conserveAllMoments", e);
-  int le = spbte_launch_project(&grid, Ns, masses, CCt, pivot, d_Q, 1, d_part, stream);
+  int le = spbte_launch_project(&grid, Ns, masses, CCt, pivot, direct ? h_Q : d_Q, 1, d_part, stream);
   if (le != 0) die("conserveAllMoments", (hipError_t)le);
-  if ((e = hipMemcpyAsync(h_Q, d_Q, sizeof(double) * na * n3, hipMemcpyDeviceToHost, stream)) != hipSuccess)
+  if (!direct && (e = hipMemcpyAsync(h_Q, d_Q, sizeof(double) * na * n3, hipMemcpyDeviceToHost, stream)) != hipSuccess)
     die("conserveAllMoments", e);
   if ((e = hipStreamSynchronize(stream)) != hipSuccess) die("conserveAllMoments", e);
   for (size_t a = 0; a < na; a++) memcpy(Q[a], h_Q + a * n3, sizeof(double) * n3);

@@ -488,7 +488,18 @@ __global__ void __launch_bounds__(256) k_copy16(const uint4 *__restrict__ in, ui
   for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n16; i += (size_t)gridDim.x * blockDim.x)
     out[i] = in[i];
 }
+__global__ void __launch_bounds__(256) k_copy8(const double *__restrict__ in, double *__restrict__ out, size_t n) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n) out[i] = in[i];
+}
 }  // namespace
+
+// n doubles (up to a cell or two), from or to pinned host memory: a launch in place of
+// a queued copy, whose engine takes longer to start than 32 KiB take to cross.
+extern "C" int spbte_launch_copy_cell(const double *in, double *out, size_t n, hipStream_t s) {
+  hipLaunchKernelGGL(k_copy8, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, in, out, n);
+  return (int)hipGetLastError();
+}
 
 extern "C" int spbte_launch_copy(const void *in, void *out, size_t bytes, hipStream_t s) {
   if (bytes % 16 || ((uintptr_t)in | (uintptr_t)out) % 16) return (int)hipErrorInvalidValue;

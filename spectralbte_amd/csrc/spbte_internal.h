@@ -136,6 +136,11 @@ int spbte_launch_wsum_scaled(int N, int form, const spbte_tile *tile, const spbt
                              hipStream_t s);
 /* FP32 operands: n float2 values at out, then the n sums of their parts. */
 int spbte_launch_c64_to_c32(const void *in, void *out, size_t n, hipStream_t s);
+int spbte_launch_copy_cell(const double *in, double *out, size_t n, hipStream_t s);
+/* Host arrays up to this size (bytes) are read and written by kernels through their
+ * pinned copies; larger ones are copied by the engine, whose bandwidth is then worth
+ * its start. */
+#define SPBTE_PINNED_DIRECT ((size_t)512 << 10)
 int spbte_launch_copy(const void *in, void *out, size_t bytes, hipStream_t s);
 /* n values of a fixed pseudo-random pattern in [-1, 1): float if single, else double */
 int spbte_launch_fill_pattern(void *p, size_t n, int single, hipStream_t s);
