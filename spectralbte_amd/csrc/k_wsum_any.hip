@@ -39,12 +39,6 @@ __host__ __device__ constexpr int rows_per_lane(int N) {
 }
 // Lanes of an x-plane of rows, in whole waves.
 __host__ __device__ inline int lane_pad(int N) { return (N * N / rows_per_lane(N) + 63) / 64 * 64; }
-// Summed planes of row plane rx under the column fold: m = (rx + h) mod N, cx + s
-// = m (mod N); the kept ones are first, first + 1, ... (count of them), mod N.
-__host__ __device__ inline int fold_count(int N, int m) { return N % 2 ? (N + 1) / 2 : N / 2 + 1 - (m & 1); }
-__host__ __device__ inline int fold_first(int N, int m) {
-  return N % 2 ? ((m & 1) ? (m + N) / 2 : m / 2) : (m + 1) / 2;
-}
 // Line slot -> cy: from the outermost to the middle (the large terms last).
 __host__ __device__ inline int line_cy(int N, int cl) { return (cl & 1) ? N - 1 - cl / 2 : cl / 2; }
 
@@ -65,8 +59,9 @@ k_wsum_any(int Nrt, int npl, int cfold, const double *__restrict__ Wf, const dou
   const int vid = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= per || vid >= total) return;
   const int cg = vid % ncg, r1 = vid / ncg, cs = r1 % csplit, r2 = r1 / csplit, ch = r2 % chunks, rx = r2 / chunks;
-  const int m = (rx + h) % N;
-  const int ncx = cfold ? fold_count(N, m) : N, first = cfold ? fold_first(N, m) + ncx - 1 : 0;
+  int first;
+  const int ncx = spbte_fold_planes(N, rx, npl < N, cfold, &first);
+  first += ncx - 1;  // the outermost plane first
   const int ncols = (cfold ? N / 2 + 1 : N) * n2;
   // this slice's z-lines of the kept summed planes: whole planes where there are
   // enough of them (each plane is then staged once; N = 8, 250 cells: 23.0 us against 25.3)
@@ -229,19 +224,19 @@ __global__ void __launch_bounds__(256) k_fold_any(const double *__restrict__ W, 
     const size_t q = i / RP;
     const int col = (int)(q % ncols), rx = (int)(q / ncols);
     const int j = col / n2, cl = col / N % N, cz = col % N, cy = line_cy(N, cl);
-    const int m = (rx + h) % N, ncx = cfold ? fold_count(N, m) : N;
+    int first;
+    const int ncx = spbte_fold_planes(N, rx, npl < N, cfold, &first);
     double x = 0.0;
     if (row < n2 && j < ncx) {
       const int ry = row / N, rz = row % N;
-      const int cx = cfold ? (fold_first(N, m) + ncx - 1 - j) % N : j;
+      const int cx = cfold ? (first + ncx - 1 - j) % N : j;
       const int sx = (rx + h - cx + N) % N, sy = (ry + h - cy + N) % N, sz = (rz + h - cz + N) % N;
       const bool pair = cfold && sx != cx;
       const double *Wr = W + ((size_t)rx * n2 + row) * n3;
       x = Wr[((size_t)cx * N + cy) * N + cz];
       if (pair) x += Wr[((size_t)sx * N + sy) * N + sz];
-      const int mx = (a2 - rx + N) % N;
-      if (mr.on && mx != rx) {
-        const int my = (a2 - ry + N) % N, mz = (a2 - rz + N) % N;
+      if (npl < N && spbte_fold_image(N, rx, cx, cfold)) {
+        const int mx = (a2 - rx + N) % N, my = (a2 - ry + N) % N, mz = (a2 - rz + N) % N;
         const double *Wm = W + (((size_t)mx * N + my) * N + mz) * n3;
         double y = Wm[((size_t)((a2 - cx + N) % N) * N + (a2 - cy + N) % N) * N + (a2 - cz + N) % N];
         if (pair) y += Wm[((size_t)((a2 - sx + N) % N) * N + (a2 - sy + N) % N) * N + (a2 - sz + N) % N];
@@ -255,10 +250,10 @@ __global__ void __launch_bounds__(256) k_fold_any(const double *__restrict__ W, 
 size_t lds_bytes(int N, int nprod, int tb) { return (size_t)nprod * tb * N * (2 * N + rows_per_lane(N) - 1) * sizeof(double2); }
 
 // Cells per workgroup: two share each weight where one a workgroup gives two waves
-// on every SIMD already (fewer, and the slices that make up for it cost more in
+// on every SIMD already, with one product one (N = 8, 250 cells: 46 us an evaluation against 48; fewer, and the slices that make up for it cost more in
 // staging and in the inverse transform's sum) and both cells' planes fit 64 KiB of LDS.
 int any_tb(int N, int npl, int nprod, int ncell) {
-  return ncell >= 2 && (long)npl * (lane_pad(N) / 64) * ncell >= 2048 && lds_bytes(N, nprod, 2) <= 65536 ? 2 : 1;
+  return ncell >= 2 && (long)npl * (lane_pad(N) / 64) * ncell >= (nprod == 1 ? 1024 : 2048) && lds_bytes(N, nprod, 2) <= 65536 ? 2 : 1;
 }
 
 template <int NT, int TR, int NP>

@@ -41,8 +41,8 @@
 // ComputeQ FP64 67.8 -> 18.0, one cell FP64 (HBM-bound) 1.25 -> 0.44; N=24 37
 // cells FP64 2.94 -> 0.74; N=16 48 cells, two different arguments, 0.60 -> 0.19.
 // Whole planes are kept because every lane of a wave shares c and its G: the
-// self-paired planes (two of cx, in half of the row planes; rx = 0 and N/2) cost
-// 6-10% more than the exact half of each.
+// self-paired planes (two of cx, in half of the row planes; rx = N/2) cost a few
+// percent more than the exact half of each.
 #include <hip/hip_runtime.h>
 #include <type_traits>
 #include "spbte_internal.h"
@@ -187,9 +187,9 @@ k_wsum_stream(const uint4 *__restrict__ Wp, const float *__restrict__ rowscale, 
   // summed x-planes: all N from 0, or, folded (one x-plane of rows per
   // workgroup), one of every pair cx, rx + N/2 - cx (mod N); the slice's share
   // of their z-lines is [l0, l1)
-  const int m = cfold ? (rx0 + N / 2) % N : 0;
-  const int ncx = cfold ? N / 2 + 1 - (m & 1) : N;
-  const int cxs = cfold ? (m + 1) / 2 + ncx - 1 : 0;     // the outermost first (k_fold_w)
+  int cxs;
+  const int ncx = spbte_fold_planes(N, rx0, npl < N, cfold, &cxs);
+  cxs += ncx - 1;                                        // the outermost first (k_fold_w)
   const int nl = ncx * N;
   const int l0 = (int)((long)cs * nl / csplit), l1 = (int)((long)(cs + 1) * nl / csplit);
   const size_t wt = (size_t)rt * WAVES + wave;           // wave tile of the permuted table
@@ -593,18 +593,16 @@ __global__ void __launch_bounds__(256) k_permute_w(const double *__restrict__ W,
 
 // Natural FP64 table -> folded permuted copy (form 0: FP64, else FP32), units
 // as in k_permute_w over the kept rows (x-planes rx < npl) and the kept columns.
-//  * Row fold (mr.on): the inverse transform keeps the real part, and the
+//  * Row fold (npl < N): the inverse transform keeps the real part, and the
 //    operands are transforms of real cells, X[k'] = S(k) conj X[k] with
 //    k' = (2 (N/2) - k) mod N per axis.  The rows r and r' then enter as
 //    Qhat[r] + R(r) conj Qhat[r'], whose second term is the sum over the same
 //    (c, s(r, c)) with W[r'][c'] R(r) S(c) S(s): one row of
-//    W[r][c] + R(r) S(c) S(s) W[r'][c'] serves both.  Kept are rx <= N/2; a
-//    plane that is its own mirror image keeps its rows as they are.
+//    W[r][c] + R(r) S(c) S(s) W[r'][c'] serves both.  Kept are rx <= N/2.
 //  * Column fold (cfold): where the summed products are symmetric under
-//    c <-> s(r, c), the column c carries the weight of both.  With
-//    m = (rx + N/2) mod N (even N) the kept planes are cx = ceil(m/2) to
-//    ceil(m/2) + N/2 - (m odd), mod N, the last of them first.  Planes with
-//    2 cx = m (mod N) are their own partners and stay whole.
+//    c <-> s(r, c), the column c carries the weight of both.  spbte_fold_planes has
+//    the kept planes, the last of them first.  Planes with 2 cx = rx + N/2 (mod N) are
+//    their own partners and stay whole.
 // The z-lines of a plane go from the outermost cy to the middle ones, as the
 // planes do: the operands decay away from the middle of the grid, so the large
 // terms of a plane are added last and few additions round at its full size.
@@ -622,15 +620,15 @@ __global__ void __launch_bounds__(256) k_fold_w(const double *__restrict__ W, vo
     const int rx = (int)(row / n2), ry = (int)(row / N % N), rz = (int)(row % N);
     const int j = (int)(c4 * 4 / n2), cl = (int)(c4 * 4 / N % N), cz0 = (int)(c4 * 4 % N);
     const int cy = (cl & 1) ? N - 1 - cl / 2 : cl / 2;
-    const int m = (rx + h) % N;
-    const int ncx = cfold ? N / 2 + 1 - (m & 1) : N;
+    int first;
+    const int ncx = spbte_fold_planes(N, rx, npl < N, cfold, &first);
     const bool used = j < ncx;
-    const int cx = cfold && used ? ((m + 1) / 2 + ncx - 1 - j) % N : j % N;
+    const int cx = cfold && used ? (first + ncx - 1 - j) % N : j % N;
     const int sx = (rx + h - cx + N) % N, sy = (ry + h - cy + N) % N;
     const bool pair = cfold && sx != cx;
     const int a2 = 2 * h;
     const int mx = (a2 - rx + N) % N, my = (a2 - ry + N) % N, mz = (a2 - rz + N) % N;
-    const bool mir = mr.on && mx != rx;
+    const bool mir = npl < N && spbte_fold_image(N, rx, cx, cfold);
     const size_t rowm = ((size_t)mx * N + my) * N + mz;
     const double R = mir ? mr.r[rx] * mr.r[ry] * mr.r[rz] : 0.0;
     double w[4];

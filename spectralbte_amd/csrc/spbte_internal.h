@@ -63,6 +63,34 @@ typedef struct {
                          whether its columns are folded too */
 } spbte_wsum_args;
 
+#ifdef __HIPCC__
+/* Summed x-planes of an x-plane rx of rows in a folded table (k_fold_w, k_fold_any):
+ * first, first + 1, ..., *count of them, mod N.  mirror: rows folded, cfold: columns.
+ *  - Columns folded: one of every pair cx, m - cx (mod N), m = (rx + h) mod N, h = N/2:
+ *    ceil(m/2) on for even N (h + 1 planes with the self-paired two for even m, else
+ *    h), from the self-paired one on for odd N.
+ *  - A plane that is its own mirror image (rx = 0 or h of an even N, h of an odd one)
+ *    keeps all its rows; where the mirror image of the kept planes is the kept planes
+ *    (rx = 0 under the column fold, all of them without it), each row takes half of
+ *    them, cx up to h, with the weights of its image added, and leaves the other
+ *    half to its image.  (N = 32: 9 of 17 planes at rx = 0; without the column fold
+ *    17 of 32 at rx = 0 and 16.) */
+static inline __host__ __device__ int spbte_fold_planes(int N, int rx, int mirror, int cfold, int *first) {
+  const int h = N / 2, m = (rx + h) % N;
+  const int half = mirror && (2 * h - rx + N) % N == rx && (!cfold || (N % 2 == 0 && rx == 0));
+  const int a = !cfold ? 0 : (N % 2 ? ((m & 1) ? (m + N) / 2 : m / 2) : (m + 1) / 2);
+  *first = a;
+  if (half) return h + 1 - a;
+  return !cfold ? N : (N % 2 ? h + 1 : h + 1 - (m & 1));
+}
+/* 1 if a kept entry of row plane rx and summed plane cx carries its mirror image too. */
+static inline __host__ __device__ int spbte_fold_image(int N, int rx, int cx, int cfold) {
+  const int h = N / 2;
+  if ((2 * h - rx + N) % N != rx) return 1;
+  return (!cfold || (N % 2 == 0 && rx == 0)) && (2 * h - cx + N) % N != cx;
+}
+#endif
+
 /* Mirror symmetry of the transforms of real cells on one grid: with
  * k' = (2 (N/2) - k) mod N, X[k'] = s(k) conj X[k] for the forward transform,
  * and the inverse's real part takes Qhat[k'] as r(k) conj Qhat[k'] at k (both
