@@ -843,10 +843,12 @@ static long stream_wgs(int N, int ncell, const spbte_tile *t) {
  *    (512 cells: 8390 against 8680).
  *  N=16: one row per lane, 4 waves, up to 4 cells (one cell: 40 against 46 with
  *    one wave, 47 with 4 rows); then 4 rows, with one cell per lane for two
- *    products (600 cells: 1715 against 1920) and two for one.
+ *    products (600 cells: 1715 against 1920) and two for one; from 24 cells on four
+ *    such cell groups a workgroup (48 cells, one product, two arguments: 164
+ *    against 172; 600 cells, one argument: 915 against 1042).
  * The summed lines are split into at least 8 slices (16 with FP32 products at
- * N=32 and one product at N=16, 12 with one product at N=24) and into as many as
- * give 4000 workgroups, at most 32 (N=32), 48 (N=24), 64 (N=16): a last round of
+ * N=32, 12 with one product at N=24) and into as many as give 4000 workgroups
+ * (N=16: waves), at most 32 (N=32), 48 (N=24), 64 (N=16): a last round of
  * workgroups that is nearly empty costs less, and the slices of one r-tile keep
  * nearer each other in the table (N=32, 512 cells with FP32 products: 43930 us
  * with one slice, 42060 with 4, 40000 with 16; 256 cells ComputeQ in FP64: 22770
@@ -856,7 +858,7 @@ static long stream_wgs(int N, int ncell, const spbte_tile *t) {
 static int default_stream_tile(int N, int form, int nprod, int ncell, spbte_tile *t) {
   static const spbte_tile s32[] = {{4, 4, 4, 1}, {4, 4, 2, 1}, {4, 4, 1, 1}}, s32m[] = {{4, 4, 2, 1}, {4, 4, 1, 1}};
   static const spbte_tile s24[] = {{3, 3, 2, 1}, {3, 3, 1, 1}};
-  static const spbte_tile s16[] = {{4, 1, 2, 1}, {4, 1, 1, 1}};
+  static const spbte_tile s16[] = {{4, 4, 2, 1}, {4, 1, 2, 1}, {4, 1, 1, 1}}, s16m[] = {{4, 4, 1, 1}, {4, 1, 1, 1}};
   static const spbte_tile s16few[] = {{1, 4, 1, 1}, {4, 1, 2, 1}};
   const spbte_tile *c = NULL;
   int nc = 0, kmin = 8, kmax = 0;
@@ -877,16 +879,16 @@ static int default_stream_tile(int N, int form, int nprod, int ncell, spbte_tile
     nc = 2 - one;
   } else if (N == 16) {
     kmax = 64;
-    if (nprod == 1) kmin = 16;
-    const int one = nprod == 2 && form != SPBTE_FORM_FP32A;
     if (ncell <= 4) { c = s16few; nc = 2; }
-    else { c = s16 + one; nc = 2 - one; }
+    else if (nprod == 2 && form != SPBTE_FORM_FP32A) { c = s16m; nc = 2; }
+    else { c = s16; nc = 3; }
+    if (ncell > 4 && ncell < 24) { c++; nc--; } /* too few to fill four cell groups a workgroup */
   } else return 0;
   for (int i = 0; i < nc; i++) {
     if (!spbte_stream_tile_supported(N, form, nprod, c[i].tr, c[i].lines, c[i].tb)) continue;
     if (c[i].tb > ncell && i + 1 < nc) continue;
     *t = c[i];
-    const long wgs = stream_wgs(N, ncell, t);
+    const long wgs = stream_wgs(N, ncell, t) * (N == 16 ? t->lines : 1); /* N=16: waves */
     t->kind = kmin;
     for (int k = kmin; k <= kmax && wgs * t->kind < 4000; k++)
       if (spbte_csplit_valid(N, k)) t->kind = k;

@@ -12,7 +12,8 @@ from conftest import rel_l2
 
 pytestmark = pytest.mark.gpu
 
-TILES = {16: [None, (4, 1, 1, 1), (4, 1, 2, 16), (2, 1, 1, 8), (1, 1, 1, 64), (1, 2, 1, 32), (1, 4, 1, 256)],
+TILES = {16: [None, (4, 1, 1, 1), (4, 1, 2, 16), (2, 1, 1, 8), (1, 1, 1, 64), (1, 2, 1, 32), (1, 4, 1, 256),
+           (4, 4, 2, 16), (4, 4, 1, 8)],
          24: [None, (3, 3, 1, 1), (3, 3, 2, 24), (4, 2, 1, 1)],   # the last one straddles planes: whole table
          32: [None, (8, 2, 1, 4), (4, 4, 4, 1), (4, 2, 1, 64), (4, 1, 1, 2)]}
 
