@@ -34,7 +34,7 @@
 // inverse transform is kept, so half of the output modes determine Q, and in
 // Q(f, f) the modes c and s(r, c) enter alike, so half of the summed ones do: the
 // kernel then runs over N/2 + 1 of N x-planes of rows and N/2 or N/2 + 1
-// x-planes of columns (0.274 of the table at N=32, 0.293 at N=24, 0.299 at N=16),
+// x-planes of columns (0.267 of the pairs at N=32, 0.273 at N=24, 0.285 at N=16),
 // or over the rows' half alone for two different cells.  The inner loop is the
 // same; every form gains by the smaller table (MI355X, one evaluation, before and
 // after): N=32 512 problems with FP32 products 140.7 -> 40.5 ms, 256 cells

@@ -1431,7 +1431,7 @@ int spbte_autotune(spbte_op *op, int ncell, int form, int maxpreserve, int *kind
     const spbte_tile *t = have_dt ? (i ? &k_cand[i - 1] : &dt) : &k_cand[i]; /* the default tile first */
     if (!tile_supported(op->N, form, np, t)) continue;
     if (t->tb > 2 * ncell) continue;
-    if (t->kind > 1 && stream_wgs(op->N, ncell, t) >= 2048) continue; /* the chip is full without a split */
+    if (t != &dt && t->kind > 1 && stream_wgs(op->N, ncell, t) >= 2048) continue; /* the chip is full without a split */
     /* warm-up (builds the table layout it needs); a tile whose warm-up alone
      * takes twice the best time so far is not timed further */
     HIPCHK(hipEventRecord(a, op->s));
