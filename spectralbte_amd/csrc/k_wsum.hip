@@ -297,8 +297,10 @@ k_wsum(KArgs a) {
 }
 
 // Generic form for any N (and the reference's one-row-at-a-time order): one
-// thread per (output mode, cell), FP64 throughout.  Used for grids the tiled
-// kernel is not instantiated for.
+// thread per (output mode, cell), FP64 throughout, over the whole table.  Used
+// where no tile is instantiated and k_wsum_any.hip does not serve: operands that are
+// not transforms of real cells, N > 24, and an allocation-free call before the
+// folded table is there.
 __global__ void __launch_bounds__(256)
 k_wsum_generic(int N, const double *__restrict__ W, const double2 *__restrict__ F0, const double2 *__restrict__ G0,
                const double2 *__restrict__ F1, const double2 *__restrict__ G1, int nprod, double2 *__restrict__ Qh) {

@@ -37,9 +37,9 @@
 // x-planes of columns (0.267 of the pairs at N=32, 0.273 at N=24, 0.285 at N=16),
 // or over the rows' half alone for two different cells.  The inner loop is the
 // same; every form gains by the smaller table (MI355X, one evaluation, before and
-// after): N=32 512 problems with FP32 products 140.7 -> 40.5 ms, 256 cells
-// ComputeQ FP64 67.8 -> 18.0, one cell FP64 (HBM-bound) 1.25 -> 0.44; N=24 37
-// cells FP64 2.94 -> 0.74; N=16 48 cells, two different arguments, 0.60 -> 0.19.
+// after): N=32 512 problems with FP32 products 140.7 -> 41.0 ms, 256 cells ComputeQ
+// FP64 67.8 -> 17.8, one cell FP64 (HBM-bound) 1.25 -> 0.44; N=24 37 cells FP64 2.94 ->
+// 0.63; a two-species step of 48 N=16 cells 1.06 -> 0.56.
 // Whole planes are kept because every lane of a wave shares c and its G: the
 // self-paired planes (two of cx, in half of the row planes; rx = N/2) cost a few
 // percent more than the exact half of each.
