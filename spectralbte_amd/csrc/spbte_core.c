@@ -7,6 +7,7 @@
  * The reference-compatible entry points (collisions.c, conserve.c, weights.c)
  * are thin wrappers over this file.
  */
+#include <float.h>
 #include <math.h>
 #include <stdarg.h>
 #include <stdio.h>
@@ -186,17 +187,31 @@ static void build_fft_factors(int N, const double *a, double delta, double Lstar
 /* The transforms with the mirror symmetry of real cells exact to the last bit:
  * with k' = (2h - k) mod N, h = N/2 (rounded down), conj Mf[k][j] = s(k) Mf[k'][j]
  * and conj Mi[j][k] / w_k = t(k) Mi[j][k'] / w_k', signs s, t (-1 at the mode
- * -N/2 of an even N, which is its own mirror image).  The reference's phases
- * keep it to about 1e-13 only: its factor exp(i j L_eta h_v) is (-1)^j times
- * exp(i j eps), eps the rounding of L_eta h_v.  Here the part of each phase that
- * is odd under k <-> k' is kept as it is and the even part is the exact one.
- * That turns f into f exp(i eps j), so Q by i eps times a real function, which
- * the real part drops: the results agree to eps^2.  Taken instead with the
- * reference's phases, the folded sums were 3.6e-14 off (relative, N=16) where
- * the unfolded ones are 2.8e-15.
+ * -N/2 of an even N, which is its own mirror image).  The given phases keep it to
+ * rounding only: the factor exp(i j L_eta h_v) is (-1)^j times exp(i j eps), eps
+ * the rounding of L_eta h_v.  Here the part of each phase that is odd under
+ * k <-> k' is kept as it is and the even part is the exact one.  That turns f into
+ * f exp(i eps j), so Q by i eps times the inverse transform of a spectrum with the
+ * symmetry, of which the real part is taken.  For odd N that inverse is real and
+ * the results agree to eps^2.  For even N it is not: the modes 1 and N-1 are mirror
+ * images with trapezoid weights 1 and 1/2, so eps times the share of Q in the
+ * outermost modes is lost, which grows as N falls.
+ * Measured against long double sums (lambda 0 and 1, L_v from 5 to 8.5, bimodal and
+ * shock-layer cells, Q(f, f) and Q(f, g)), relative error of the whole sum with the
+ * given phases, then of the folded one: N=8 2.4e-15, 4.0e-15 (worst ratio 7);
+ * N=10 3.7e-15, 4.9e-15 (5); N=12 4.5e-15, 4.3e-15 (5); N=14 6.4e-15, 4.9e-15 (1.3);
+ * N=16 5.3e-15, 4.7e-15 (1.9, at L_v = 8.5); N=18 7.6e-15, 4.4e-15 (1.0); N=24
+ * 9.1e-15, 5.0e-15 (1.0).  So even grids under N = 16 keep the given phases and
+ * fold their columns only, which is exact for any operands (N=8 1.8e-15, N=10
+ * 2.9e-15, N=12 2.8e-15, N=14 4.2e-15): 500 -> 544 us for ten steps of 250 N=8
+ * cells, 67 -> 77 us for 75 N=10 cells.  At N=16 the rows' fold is 12% of one
+ * cell's evaluation and a third of a two-species step.
+ * (Folded with the given phases, the rows' sums were 3.6e-14 off at N=16.)
  * out: forward p, q, twiddles, inverse p, q, twiddles (N complex each), then
- * both matrices.  Returns 1 if the grid has the symmetry: the matrices within
- * 1e-12 of the given ones (the 1D grids of odd N and a caller's own may not). */
+ * both matrices.  Returns 1 if the grid has the symmetry to rounding and folds its
+ * rows: the matrices within N^2 DBL_EPSILON of the given ones (the phases reach
+ * pi N / 2; grids by the reference's formulas stay under 0.83 of it, N = 6 to 64;
+ * the 1D grids of odd N do not have it and a caller's own may not). */
 static int build_mirror(int N, const double *eta, double Lv, double heta, const double *w, const double *Mf,
                         const double *Mi, double *out /* 2 (6N + 2N^2) */, spbte_mirror *mr) {
   const long double pi = 3.141592653589793238462643383279502884L;
@@ -251,7 +266,7 @@ static int build_mirror(int N, const double *eta, double Lv, double heta, const 
         m[1] = (double)(x * ti + y * t[0]);
         dev = fmax(dev, fmax(fabs(m[0] - g[0]), fabs(m[1] - g[1])));
       }
-  return dev <= 1e-12; /* false for NaN */
+  return dev <= N * N * DBL_EPSILON && (N % 2 || N >= 16); /* false for NaN */
 }
 
 /* ---------------------------------------------- LU (src/conserve.c:89-168) */
@@ -1003,7 +1018,7 @@ static int launch_tile(spbte_op *op, int form, const spbte_tile *t, const spbte_
     }
     return SPBTE_OK;
   }
-  if (!t && sum != SUM_ANY && spbte_any_supported(op->N) && (sum == SUM_SELF || op->mirror.on)) {
+  if (!t && sum != SUM_ANY && spbte_any_supported(op->N)) {
     void **Wa = &op->t->dWa[sum == SUM_SELF];
     b.npl = op->mirror.on ? op->N / 2 + 1 : op->N;
     b.cfold = sum == SUM_SELF;
@@ -1237,7 +1252,7 @@ int spbte_compute_q_noalloc(spbte_op *op, const double *d_f, const double *d_g, 
   spbte_tile dt;
   const int is_default = have && default_stream_tile(op->N, form, mp ? 2 : 1, ncell, &dt) && !memcmp(&dt, &t, sizeof t);
   while (is_default && kind > 1 && b_fix + al256(16 * n * (size_t)kind) > op->nac_bytes) kind--;
-  if (!have && spbte_any_supported(op->N) && (self || op->mirror.on)) { /* likewise */
+  if (!have && spbte_any_supported(op->N)) { /* likewise */
     kind = spbte_any_slices(op->N, op->mirror.on ? op->N / 2 + 1 : op->N, self, mp ? 2 : 1, ncell);
     while (kind > 1 && b_fix + al256(16 * n * (size_t)kind) > op->nac_bytes) kind--;
   }

@@ -1,0 +1,48 @@
+"""A folded sum is as near the oracle as the whole sum: the row fold takes the operands' mirror symmetry as exact, which
+the transforms have to rounding only, and on small even grids and on a caller's modes that are symmetric to less than
+that the difference would be the largest error of the result.
+
+Bound: both sums round each product and addition once, in different orders, so their errors are alike in size; twice the
+whole sum's, taken over 24 cells, leaves room for the orders.  1e-15 of Q is the projection-free transforms' own."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _layer_cells(N, v, n, seed):
+    """Cells of a Mach-1.2 layer: near equilibrium, where Q is a small difference of its gain and loss."""
+    rng = np.random.default_rng(seed)
+
+    def side(rho, ux, T):
+        g = [np.exp(-(v - u) ** 2 / (2 * T)) for u in (ux, 0.0, 0.0)]
+        return rho * (2 * np.pi * T) ** -1.5 * g[0][:, None, None] * g[1][None, :, None] * g[2][None, None, :]
+    a, b = side(1.0, 1.549, 1.0), side(1.2973, 1.194, 1.1947)
+    return np.stack([((1 - s) * a + s * b).ravel() for s in rng.uniform(0.05, 0.95, n)])
+
+
+def _errors(spb, orc, N, Lv, eta_shift, pair):
+    v, eta = orc.grid_0d(N, Lv)
+    eta = eta + eta_shift / Lv
+    W = orc.weights_iso(N, eta, Lv, 1.0)
+    op = spb.Operator(N, Lv, v, eta)
+    op.set_weights(W)
+    n = 24 if N < 16 else 6
+    f = _layer_cells(N, v, n, N)
+    g = _layer_cells(N, v, n, N + 100) if pair else f
+    ref = np.stack([orc.compute_q(N, v, eta, W, f[b], g[b]).ravel() for b in range(n)])
+    folded = op.compute_q(f, g if pair else None)
+    F, G = op.transform(f.astype(complex)), op.transform(g.astype(complex))
+    whole = op.transform(op.qhat(F, G), invert=True).real
+    op.close()
+    scale = np.linalg.norm(ref)
+    return np.linalg.norm(folded - ref) / scale, np.linalg.norm(whole - ref) / scale
+
+
+@pytest.mark.parametrize("pair", [False, True])
+@pytest.mark.parametrize("N,Lv,shift", [(6, 5.0, 0.0), (8, 5.71, 0.0), (10, 6.0, 0.0), (12, 8.0, 0.0), (14, 7.6, 0.0),
+                                        (9, 8.0, 0.0), (16, 6.0, 0.0), (18, 8.5, 0.0),
+                                        (9, 8.0, 3e-13), (16, 12.0, 3e-13), (18, 14.0, 3e-13)])
+def test_folded_sum_is_as_near_as_the_whole_one(spb, orc, N, Lv, shift, pair):
+    folded, whole = _errors(spb, orc, N, Lv, shift, pair)
+    assert folded <= 2 * whole + 1e-15, (folded, whole)
