@@ -223,7 +223,7 @@ static int build_mirror(int N, const double *eta, double Lv, double heta, const 
     a[k] = (long double)Lv * ((long double)eta[k] - (long double)eta[km]) / 2;
     c[k] = -(long double)(k - h) * (long double)Lv * heta;
     mr->s[k] = mr->r[k] = 1.0;
-    if (km == k) { /* its own image: the phase is a quarter turn's multiple */
+    if (km == k && isfinite(Lv * eta[k])) { /* its own image: the phase is a quarter turn's multiple */
       const long na = lroundl((long double)Lv * eta[k] / (pi / 2)), nc = lroundl(c[k] / (pi / 2));
       a[k] = na * (pi / 2);
       c[k] = nc * (pi / 2);
@@ -254,7 +254,8 @@ static int build_mirror(int N, const double *eta, double Lv, double heta, const 
       out[4 * N + 2 * j + z] = (double)(z ? -tw[j][1] : tw[j][0]);
     }
   }
-  double dev = 0.0;
+  const double tol = N * N * DBL_EPSILON;
+  int near = 1;
   for (int d = 0; d < 2; d++) /* M[r][s] = q[r] exp(-+2 pi i r s / N) p[s] */
     for (int r = 0; r < N; r++)
       for (int s = 0; s < N; s++) {
@@ -264,9 +265,9 @@ static int build_mirror(int N, const double *eta, double Lv, double heta, const 
         const double *g = (d ? Mi : Mf) + 2 * (r * N + s);
         m[0] = (double)(x * t[0] - y * ti);
         m[1] = (double)(x * ti + y * t[0]);
-        dev = fmax(dev, fmax(fabs(m[0] - g[0]), fabs(m[1] - g[1])));
+        near &= fabs(m[0] - g[0]) <= tol && fabs(m[1] - g[1]) <= tol; /* false for NaN */
       }
-  return dev <= N * N * DBL_EPSILON && (N % 2 || N >= 16); /* false for NaN */
+  return near && (N % 2 || N >= 16);
 }
 
 /* ---------------------------------------------- LU (src/conserve.c:89-168) */

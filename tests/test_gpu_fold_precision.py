@@ -46,3 +46,20 @@ def _errors(spb, orc, N, Lv, eta_shift, pair):
 def test_folded_sum_is_as_near_as_the_whole_one(spb, orc, N, Lv, shift, pair):
     folded, whole = _errors(spb, orc, N, Lv, shift, pair)
     assert folded <= 2 * whole + 1e-15, (folded, whole)
+
+
+@pytest.mark.parametrize("N", [9, 16, 18])
+def test_modes_or_nodes_that_are_not_numbers_are_not_taken_as_symmetric(spb, orc, N):
+    """A node that is NaN makes Q NaN on its planes (the exact transforms would not read it at all); a mode, everywhere."""
+    for which in (0, 1):
+        grid = list(orc.grid_0d(N, 6.0))
+        grid[which] = grid[which].copy()
+        grid[which][3] = np.nan
+        try:
+            op = spb.Operator(N, 6.0, *grid)
+        except spb.SpbteError:
+            continue   # refused: as good
+        op.set_weights(np.random.default_rng(N).standard_normal((N ** 3, N ** 3)))
+        q = op.compute_q(np.random.default_rng(1).uniform(size=(1, N ** 3))).reshape(N, N, N)
+        op.close()
+        assert np.isnan(q[3]).all() and np.isnan(q[:, 3]).all() and np.isnan(q[:, :, 3]).all()
