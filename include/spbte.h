@@ -171,8 +171,10 @@ int spbte_qhat(spbte_op *op, const double *d_Fhat, const double *d_Ghat, double 
  * cell, so that one workgroup's W loads serve four cells) with the summed
  * x-planes split into k slices whose partial sums are added afterwards (k > 1
  * gives small batches more workgroups; k divides N, or is N times a divisor of
- * N, cutting x-planes into y-line ranges).  set_tile pins a tile for (form,
- * maxpreserve); tr = 0 restores automatic choice.  autotune times every
+ * N, cutting x-planes into y-line ranges, or is a number that get_tile reports
+ * for one cell group, whose slices fill whole rounds of the CUs).  set_tile pins
+ * a tile for (form, maxpreserve), which then runs as it is; tr = 0 restores
+ * automatic choice.  autotune times every
  * instantiated tile on the given batch shape and pins the fastest for that
  * batch size; get_tile reports the tile a batch would use. */
 int spbte_set_tile(spbte_op *op, int form, int maxpreserve, int kind, int tr, int lines, int tb);

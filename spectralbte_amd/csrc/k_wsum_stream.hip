@@ -683,9 +683,8 @@ extern "C" int spbte_stream_tile_supported(int N, int form, int nprod, int tr, i
 }
 
 // Launch with the permuted table Wp built for the same tr (spbte_launch_permute_weights).
-// csplit: slices of the summed modes -- a divisor of N (whole x-planes) or N
-// times a divisor of N (x-planes cut into y-line ranges); csplit > 1 needs Qp
-// with room for csplit * ncell * N^3 double2.
+// csplit: slices of the summed z-lines, any number; csplit > 1 needs Qp with room
+// for csplit * ncell * N^3 double2.
 extern "C" int spbte_launch_wsum_stream(int N, int form, int tr, int waves, int tb, const spbte_wsum_args *a, const void *Wp,
                                         const float *rowscale, int csplit, void *Qp, hipStream_t s) {
   const SEntry *e = sfind(N, form, a->nprod, tr, waves, tb);

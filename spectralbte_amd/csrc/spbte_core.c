@@ -847,6 +847,23 @@ static long stream_wgs(int N, int ncell, const spbte_tile *t) {
   return rows / (64L * t->lines * t->tr) * ((ncell + t->tb - 1) / t->tb);
 }
 
+/* k slices of one cell group, or the next number that fills whole rounds of the
+ * 256 CUs. */
+static int whole_rounds(int N, const spbte_tile *t, int k) {
+  const long wgs = stream_wgs(N, t->tb, t);
+  const long r = (wgs * k + 255) / 256 * 256 / wgs;
+  return (int)(r > k ? r : k);
+}
+
+/* Slice counts a tile may have: divisors of N, N times a divisor, and where one cell
+ * group's default is rounded (N >= 24), the rounded ones. */
+static int slices_valid(int N, const spbte_tile *t) {
+  if (spbte_csplit_valid(N, t->kind)) return 1;
+  for (int k = 16; N >= 24 && k < t->kind; k++)
+    if (spbte_csplit_valid(N, k) && whole_rounds(N, t, k) == t->kind) return 1;
+  return 0;
+}
+
 /* Streaming kernel defaults on folded tables, measured on an MI355X (us per
  * evaluation, best of the tiles and splits tried):
  *  N=32 two products: 4 rows x 4 waves (FP64, one cell: 444 against 472 with 8
@@ -870,7 +887,9 @@ static long stream_wgs(int N, int ncell, const spbte_tile *t) {
  * with one slice, 42060 with 4, 40000 with 16; 256 cells ComputeQ in FP64: 22770
  * with one, 17910 with 4, 17530 with 8, 17910 with 16; N=24, 37 cells ComputeQ: 756
  * with 8, 693 with 12, 665 with 24; N=16, 48 cells, two arguments: 206 with 8, 183
- * with 16, 172 with 32).  The inverse transform adds them. */
+ * with 16, 172 with 32).  The inverse transform adds them.  Where one cell group
+ * streams a table from HBM (N >= 24), whole rounds of the CUs (one N=32 cell, 17
+ * workgroups a slice: 425 us with 32 slices, 404 with 30, 392 with 45). */
 static int default_stream_tile(int N, int form, int nprod, int ncell, spbte_tile *t) {
   static const spbte_tile s32[] = {{4, 4, 4, 1}, {4, 4, 2, 1}, {4, 4, 1, 1}}, s32m[] = {{4, 4, 2, 1}, {4, 4, 1, 1}};
   static const spbte_tile s24[] = {{3, 3, 2, 1}, {3, 3, 1, 1}};
@@ -908,19 +927,10 @@ static int default_stream_tile(int N, int form, int nprod, int ncell, spbte_tile
     t->kind = kmin;
     for (int k = kmin; k <= kmax && wgs * t->kind < 4000; k++)
       if (spbte_csplit_valid(N, k)) t->kind = k;
+    if (N >= 24 && ncell <= t->tb && t->kind >= 16) t->kind = whole_rounds(N, t, t->kind);
     return 1;
   }
   return 0;
-}
-
-/* Slices a tile's launch takes: its kind; where one cell group streams a table from
- * HBM (N >= 24), the next number that fills whole rounds of the 256 CUs (one N=32
- * cell, 17 workgroups a slice: 425 us with 32 slices, 404 with 30, 392 with 45). */
-static int tile_slices(int N, int ncell, const spbte_tile *t) {
-  const long wgs = stream_wgs(N, ncell, t);
-  if (t->kind < 16 || N < 24 || ncell > t->tb) return t->kind;
-  const long k = (wgs * t->kind + 255) / 256 * 256 / wgs;
-  return (int)(k > t->kind ? k : t->kind);
 }
 
 static int pick_tile(spbte_op *op, int ncell, int form, int nprod, spbte_tile *t) {
@@ -933,7 +943,7 @@ static int pick_tile(spbte_op *op, int ncell, int form, int nprod, spbte_tile *t
 
 static int tile_supported(int N, int form, int nprod, const spbte_tile *t) {
   if (t->kind >= 1)
-    return spbte_csplit_valid(N, t->kind) && spbte_stream_tile_supported(N, form, nprod, t->tr, t->lines, t->tb);
+    return spbte_stream_tile_supported(N, form, nprod, t->tr, t->lines, t->tb) && slices_valid(N, t);
   return spbte_wsum_tile_supported(N, form, nprod, t);
 }
 
@@ -1000,7 +1010,7 @@ static int launch_tile(spbte_op *op, int form, const spbte_tile *t, const spbte_
     if (!Wp) rc = weights_permuted(op, form, t->tr, !ss->fixed, &Wp, &rs);
     if (rc) return rc;
     void *Qp = NULL;
-    const int k = ss->fixed && ss->kind ? ss->kind : tile_slices(op->N, a->ncell, t);
+    const int k = ss->fixed && ss->kind ? ss->kind : t->kind;
     if (k > 1) {
       const size_t need = (size_t)k * a->ncell * op->n3 * 16;
       if (ss->fixed) {
@@ -1249,7 +1259,7 @@ int spbte_compute_q_noalloc(spbte_op *op, const double *d_f, const double *d_g, 
   const size_t b_xs = 16 * n * (size_t)nj, b_fix = b_mom + b_part + b_fg + b_qh;
   /* a tile that was not pinned or tuned takes fewer slices where the workspace
    * does not hold its own number (the sums then differ by rounding) */
-  int kind = have ? (t.kind > 1 ? tile_slices(op->N, ncell, &t) : t.kind) : 0;
+  int kind = have ? t.kind : 0;
   spbte_tile dt;
   const int is_default = have && default_stream_tile(op->N, form, mp ? 2 : 1, ncell, &dt) && !memcmp(&dt, &t, sizeof t);
   while (is_default && kind > 1 && b_fix + al256(16 * n * (size_t)kind) > op->nac_bytes) kind--;

@@ -1,0 +1,45 @@
+"""Tiles: what is pinned is what runs and what get_tile reports.
+
+A cell's result depends on the tile's slices and on nothing else of the batch, so the same slices give the same bits."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _op(spb, N, n):
+    from spectralbte_amd import workloads
+    v, eta = workloads.grid_0d(N, 6.0)
+    op = spb.Operator(N, 6.0, v, eta)
+    op.generate_weights_iso(1.0)
+    return op, workloads.two_maxwellian_ensemble(N, 6.0, n, seed=N)
+
+
+@pytest.mark.parametrize("N,tile", [(24, (3, 3, 1, 24)), (32, (4, 4, 2, 16)), (32, (4, 4, 1, 32))])
+def test_pinned_slices_run_as_given(spb, N, tile):
+    """One cell group takes the pinned slices like several groups do: the same bits for the same cell."""
+    op, f = _op(spb, N, 2 * tile[2] + 1)
+    op.set_tile("fp64", True, *tile[:3], kind=tile[3])
+    assert op.get_tile(1, "fp64", True) == (tile[3],) + tile[:3]
+    assert np.array_equal(op.compute_q(f[:1], maxpreserve=True)[0], op.compute_q(f, maxpreserve=True)[0])
+    op.close()
+
+
+@pytest.mark.parametrize("N,form,mp", [(16, "fp64", True), (24, "fp64", False), (24, "fp32a", True), (32, "fp64", True),
+                                       (32, "fp64", False), (32, "fp32a", True)])
+def test_reported_tile_can_be_pinned(spb, N, form, mp):
+    """The default tile of one cell, pinned, accepted and with the same bits."""
+    op, f = _op(spb, N, 1)
+    q = op.compute_q(f, form=form, maxpreserve=mp)
+    kind, tr, lines, tb = op.get_tile(1, form, mp)
+    op.set_tile(form, mp, tr, lines, tb, kind=kind)
+    assert np.array_equal(op.compute_q(f, form=form, maxpreserve=mp), q)
+    op.close()
+
+
+def test_slice_counts_that_are_refused(spb):
+    op, _ = _op(spb, 32, 1)
+    for k in (3, 31, 33, 44, 46, 1025):
+        with pytest.raises(spb.SpbteError):
+            op.set_tile("fp64", True, 4, 4, 1, kind=k)
+    op.close()
