@@ -174,9 +174,9 @@ int spbte_qhat(spbte_op *op, const double *d_Fhat, const double *d_Ghat, double 
  * N, cutting x-planes into y-line ranges, or is a number that get_tile reports
  * for one cell group, whose slices fill whole rounds of the CUs).  set_tile pins
  * a tile for (form, maxpreserve), which then runs as it is; tr = 0 restores
- * automatic choice.  autotune times every
- * instantiated tile on the given batch shape and pins the fastest for that
- * batch size; get_tile reports the tile a batch would use. */
+ * automatic choice.  autotune times every instantiated tile on the given batch
+ * shape and pins the fastest for that batch size; get_tile reports the tile a
+ * batch of Q(f, f) would use. */
 int spbte_set_tile(spbte_op *op, int form, int maxpreserve, int kind, int tr, int lines, int tb);
 int spbte_autotune(spbte_op *op, int ncell, int form, int maxpreserve, int *kind, int *tr, int *lines, int *tb);
 int spbte_get_tile(spbte_op *op, int ncell, int form, int maxpreserve, int *kind, int *tr, int *lines, int *tb);

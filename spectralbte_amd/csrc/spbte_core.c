@@ -840,17 +840,15 @@ static int default_tile(int N, int form, int nprod, int ncell, spbte_tile *t) {
   return 0;
 }
 
-/* Workgroups of a streaming tile without the split, on a folded table where the
- * tile has one (N/2 + 1 x-planes of output rows). */
-static long stream_wgs(int N, int ncell, const spbte_tile *t) {
-  const long rows = (long)(spbte_stream_tile_folds(N, t->tr, t->lines) ? N / 2 + 1 : N) * N * N;
-  return rows / (64L * t->lines * t->tr) * ((ncell + t->tb - 1) / t->tb);
+/* Workgroups of a streaming tile without the split, npl x-planes of output rows. */
+static long stream_wgs(int N, int npl, int ncell, const spbte_tile *t) {
+  return (long)npl * N * N / (64L * t->lines * t->tr) * ((ncell + t->tb - 1) / t->tb);
 }
 
-/* k slices of one cell group, or the next number that fills whole rounds of the
- * 256 CUs. */
+/* k slices of one cell group on a table of folded rows, or the next number that
+ * fills whole rounds of the 256 CUs. */
 static int whole_rounds(int N, const spbte_tile *t, int k) {
-  const long wgs = stream_wgs(N, t->tb, t);
+  const long wgs = stream_wgs(N, N / 2 + 1, t->tb, t);
   const long r = (wgs * k + 255) / 256 * 256 / wgs;
   return (int)(r > k ? r : k);
 }
@@ -889,8 +887,14 @@ static int slices_valid(int N, const spbte_tile *t) {
  * with 8, 693 with 12, 665 with 24; N=16, 48 cells, two arguments: 206 with 8, 183
  * with 16, 172 with 32).  The inverse transform adds them.  Where one cell group
  * streams a table from HBM (N >= 24), whole rounds of the CUs (one N=32 cell, 17
- * workgroups a slice: 425 us with 32 slices, 404 with 30, 392 with 45). */
-static int default_stream_tile(int N, int form, int nprod, int ncell, spbte_tile *t) {
+ * workgroups a slice: 425 us with 32 slices, 404 with 30, 392 with 45).
+ * Sums over the whole table (whole) take the same tiles with longer slices, of whole
+ * planes where one cell group streams it: 3000 waves at N=16, at most 32 slices where
+ * these give 2000 (12 cells, Qhat in FP64: 76 with 32, 88 with 64; 24: 121 with 16, 146
+ * with 64), 8000 workgroups at N >= 24, at N=32 16 slices for one cell group (one cell:
+ * FP64 1275 with 16, 1388 with 45, FP32 653 and 764).
+ * npl: x-planes of rows the table has. */
+static int default_stream_tile(int N, int form, int nprod, int ncell, int npl, int whole, spbte_tile *t) {
   static const spbte_tile s32[] = {{4, 4, 4, 1}, {4, 4, 2, 1}, {4, 4, 1, 1}}, s32m[] = {{4, 4, 2, 1}, {4, 4, 1, 1}};
   static const spbte_tile s24[] = {{3, 3, 2, 1}, {3, 3, 1, 1}};
   static const spbte_tile s16[] = {{4, 4, 2, 1}, {4, 1, 2, 1}, {4, 1, 1, 1}}, s16m[] = {{4, 4, 1, 1}, {4, 1, 1, 1}};
@@ -923,21 +927,32 @@ static int default_stream_tile(int N, int form, int nprod, int ncell, spbte_tile
     if (!spbte_stream_tile_supported(N, form, nprod, c[i].tr, c[i].lines, c[i].tb)) continue;
     if (c[i].tb > ncell && i + 1 < nc) continue;
     *t = c[i];
-    const long wgs = stream_wgs(N, ncell, t) * (N == 16 ? t->lines : 1); /* N=16: waves */
+    const long wgs = stream_wgs(N, npl, ncell, t) * (N == 16 ? t->lines : 1); /* N=16: waves */
+    if (whole) {
+      if (N == 16 && wgs * 32 >= 2000) kmax = 32;
+      if (N == 32 && ncell <= t->tb) kmax = 16;
+    }
+    const long want = !whole ? 4000 : (N == 16 ? 3000 : 8000);
     t->kind = kmin;
-    for (int k = kmin; k <= kmax && wgs * t->kind < 4000; k++)
+    for (int k = kmin; k <= kmax && wgs * t->kind < want; k++)
       if (spbte_csplit_valid(N, k)) t->kind = k;
-    if (N >= 24 && ncell <= t->tb && t->kind >= 16) t->kind = whole_rounds(N, t, t->kind);
+    if (N >= 24 && npl < N && ncell <= t->tb && t->kind >= 16) t->kind = whole_rounds(N, t, t->kind);
     return 1;
   }
   return 0;
 }
 
-static int pick_tile(spbte_op *op, int ncell, int form, int nprod, spbte_tile *t) {
+/* The default streaming tile of a sum on this grid. */
+static int op_stream_tile(const spbte_op *op, int ncell, int form, int nprod, int sum, spbte_tile *t) {
+  const int whole = sum == SUM_ANY || form == SPBTE_FORM_FP16X2 || (sum == SUM_REAL && !op->mirror.on);
+  return default_stream_tile(op->N, form, nprod, ncell, whole || !op->mirror.on ? op->N : op->N / 2 + 1, whole, t);
+}
+
+static int pick_tile(const spbte_op *op, int ncell, int form, int nprod, int sum, spbte_tile *t) {
   if (op->pin[form][nprod - 1].tr) { *t = op->pin[form][nprod - 1]; return 1; }
-  spbte_tile *tt = &op->tuned[form][nprod - 1][bucket(ncell)];
+  const spbte_tile *tt = &op->tuned[form][nprod - 1][bucket(ncell)];
   if (tt->tr) { *t = *tt; return 1; }
-  if (default_stream_tile(op->N, form, nprod, ncell, t)) return 1;
+  if (op_stream_tile(op, ncell, form, nprod, sum, t)) return 1;
   return default_tile(op->N, form, nprod, ncell, t);
 }
 
@@ -976,7 +991,7 @@ int spbte_set_tile(spbte_op *op, int form, int maxpreserve, int kind, int tr, in
 int spbte_get_tile(spbte_op *op, int ncell, int form, int maxpreserve, int *kind, int *tr, int *lines, int *tb) {
   spbte_tile t = {0, 0, 0, 0};
   if (form < 0 || form >= NFORMS) return fail(SPBTE_ERR_ARG, "bad form %d", form);
-  if (!pick_tile(op, ncell, form, maxpreserve ? 2 : 1, &t)) t.tr = t.lines = t.tb = t.kind = 0;
+  if (!pick_tile(op, ncell, form, maxpreserve ? 2 : 1, SUM_SELF, &t)) t.tr = t.lines = t.tb = t.kind = 0;
   *kind = t.kind; *tr = t.tr; *lines = t.lines; *tb = t.tb;
   return SPBTE_OK;
 }
@@ -1073,7 +1088,7 @@ static int run_wsum(spbte_op *op, int form, int nprod, const void *F0, const voi
                     int ncell, int sum, const scratch_set *ss, int keep_slices, wsum_result *res) {
   if (!op->t->have_w) return fail(SPBTE_ERR_NOWEIGHTS, "no weight table set");
   spbte_tile t;
-  int have = pick_tile(op, ncell, form, nprod, &t);
+  int have = pick_tile(op, ncell, form, nprod, sum, &t);
   if (!have && form != SPBTE_FORM_FP64)
     return fail(SPBTE_ERR_UNSUPPORTED, "no reduced-precision weighted-sum kernel for N=%d", op->N);
   spbte_wsum_args a = {NULL, F0, G0, F1, G1, ss->Qh, ncell, nprod, keep_slices, 0, 0};
@@ -1237,13 +1252,13 @@ int spbte_compute_q_noalloc(spbte_op *op, const double *d_f, const double *d_g, 
   const int mp = (flags & SPBTE_MAXPRESERVE) != 0;
   /* the tile compute_chunk will pick, and its table, which must be resident */
   spbte_tile t;
-  const int have = pick_tile(op, ncell, form, mp ? 2 : 1, &t);
+  const int sum = self ? SUM_SELF : SUM_REAL, have = pick_tile(op, ncell, form, mp ? 2 : 1, sum, &t);
   if (!have && form != SPBTE_FORM_FP64)
     return fail(SPBTE_ERR_UNSUPPORTED, "no reduced-precision weighted-sum kernel for N=%d", op->N);
   const void *W = NULL;
   const float *rs;
   int rc = SPBTE_OK, npl, cfold;
-  if (have && fold_of(op, form, &t, self ? SUM_SELF : SUM_REAL, &npl, &cfold))
+  if (have && fold_of(op, form, &t, sum, &npl, &cfold))
     rc = weights_folded(op, form, t.tr, npl, cfold, 0, &W);
   if (!rc && !W)
     rc = (have && t.kind >= 1) ? weights_permuted(op, form, t.tr, 0, &W, &rs) : weights_form(op, form, 0, &W, &rs);
@@ -1261,7 +1276,7 @@ int spbte_compute_q_noalloc(spbte_op *op, const double *d_f, const double *d_g, 
    * does not hold its own number (the sums then differ by rounding) */
   int kind = have ? t.kind : 0;
   spbte_tile dt;
-  const int is_default = have && default_stream_tile(op->N, form, mp ? 2 : 1, ncell, &dt) && !memcmp(&dt, &t, sizeof t);
+  const int is_default = have && op_stream_tile(op, ncell, form, mp ? 2 : 1, sum, &dt) && !memcmp(&dt, &t, sizeof t);
   while (is_default && kind > 1 && b_fix + al256(16 * n * (size_t)kind) > op->nac_bytes) kind--;
   if (!have && spbte_any_supported(op->N)) { /* likewise */
     kind = spbte_any_slices(op->N, op->mirror.on ? op->N / 2 + 1 : op->N, self, mp ? 2 : 1, ncell);
@@ -1452,12 +1467,13 @@ int spbte_autotune(spbte_op *op, int ncell, int form, int maxpreserve, int *kind
   HIPCHK(hipEventCreate(&a));
   HIPCHK(hipEventCreate(&b));
   spbte_tile dt = {0, 0, 0, 0};
-  const int have_dt = default_stream_tile(op->N, form, np, ncell, &dt);
+  const int have_dt = op_stream_tile(op, ncell, form, np, SUM_SELF, &dt);
+  const int npl = form == SPBTE_FORM_FP16X2 || !op->mirror.on ? op->N : op->N / 2 + 1;
   for (size_t i = 0; i < sizeof k_cand / sizeof k_cand[0] + (size_t)have_dt; i++) {
     const spbte_tile *t = have_dt ? (i ? &k_cand[i - 1] : &dt) : &k_cand[i]; /* the default tile first */
     if (!tile_supported(op->N, form, np, t)) continue;
     if (t->tb > 2 * ncell) continue;
-    if (t != &dt && t->kind > 1 && stream_wgs(op->N, ncell, t) >= 2048) continue; /* the chip is full without a split */
+    if (t != &dt && t->kind > 1 && stream_wgs(op->N, npl, ncell, t) >= 2048) continue; /* the chip is full without a split */
     /* warm-up (builds the table layout it needs); a tile whose warm-up alone
      * takes twice the best time so far is not timed further */
     HIPCHK(hipEventRecord(a, op->s));

@@ -43,3 +43,15 @@ def test_slice_counts_that_are_refused(spb):
         with pytest.raises(spb.SpbteError):
             op.set_tile("fp64", True, 4, 4, 1, kind=k)
     op.close()
+
+
+@pytest.mark.parametrize("N,n,tile", [(16, 1, (1, 4, 1, 32)), (16, 12, (4, 1, 2, 32)), (32, 1, (4, 4, 1, 16)), (32, 2, (4, 4, 2, 16))])
+def test_sum_over_the_whole_table_has_its_own_slices(spb, N, n, tile):
+    """spbte_qhat runs over all rows and columns: its slices are counted from those, not from a folded table's."""
+    op, _ = _op(spb, N, 1)
+    rng = np.random.default_rng(N)
+    F, G = (rng.standard_normal((n, N ** 3)) + 1j * rng.standard_normal((n, N ** 3)) for _ in range(2))
+    q = op.qhat(F, G)
+    op.set_tile("fp64", False, *tile[:3], kind=tile[3])
+    assert np.array_equal(op.qhat(F, G), q)
+    op.close()
