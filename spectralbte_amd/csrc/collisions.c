@@ -110,6 +110,25 @@ void dealloc_coll(void) {
   N = 0;
 }
 
+/* Drops the least recently used operator other than keep; 0 if there is none. */
+static int evict_lru(const spbte_op *keep) {
+  int lru = -1, used = 0;
+  for (int i = 0; i < CACHE_SLOTS; i++) {
+    used += ops[i] != NULL;
+    if (ops[i] && ops[i] != keep && (lru < 0 || ages[i] < ages[lru])) lru = i;
+  }
+  if (lru < 0) return 0;
+  static int warned;
+  if (!warned)
+    fprintf(stderr, "spectralbte_amd: device memory holds %d weight tables of N=%d; evicting the least recently "
+            "used one (each eviction re-uploads a table on its next use)\n", used, N);
+  warned = 1;
+  spbte_op_destroy(ops[lru]);
+  ops[lru] = NULL;
+  keys[lru] = NULL;
+  return 1;
+}
+
 static spbte_op *op_for(double **conv_weights) {
   if (!N) {
     fprintf(stderr, "spectralbte_amd: ComputeQ called before initialize_coll\n");
@@ -121,31 +140,21 @@ static spbte_op *op_for(double **conv_weights) {
     if (ages[i] < ages[oldest]) oldest = i;
   }
   if (slot < 0) {
-    /* a free slot, unless HBM cannot hold one more operator (its FP64 table,
-     * the copy the streaming kernel reads and scratch): then evict the least
-     * recently used tables until it can */
+    /* a free slot, unless HBM cannot hold one more operator (its FP64 table, the
+     * copies the streaming kernel reads, which are no larger than it where the modes
+     * have mirror images, and scratch): then evict the least recently used tables
+     * until it can */
     const size_t n3 = (size_t)N * N * N, need = 2 * sizeof(double) * n3 * n3 + ((size_t)256 << 20);
-    slot = -1;
-    for (int i = 0; i < CACHE_SLOTS && slot < 0; i++)
-      if (!ops[i]) slot = i;
     for (;;) {
       size_t free_b = 0, total_b = 0;
       int used = 0;
-      for (int i = 0; i < CACHE_SLOTS; i++) used += ops[i] != NULL;
+      slot = -1;
+      for (int i = CACHE_SLOTS - 1; i >= 0; i--) {
+        used += ops[i] != NULL;
+        if (!ops[i]) slot = i;
+      }
       if (slot >= 0 && (used == 0 || (hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b >= need))) break;
-      int lru = -1;
-      for (int i = 0; i < CACHE_SLOTS; i++)
-        if (ops[i] && (lru < 0 || ages[i] < ages[lru])) lru = i;
-      if (lru < 0) break;
-      static int warned;
-      if (!warned)
-        fprintf(stderr, "spectralbte_amd: device memory holds %d weight tables of N=%d; evicting the least recently "
-                "used one (each eviction re-uploads a table on its next use)\n", used, N);
-      warned = 1;
-      spbte_op_destroy(ops[lru]);
-      ops[lru] = NULL;
-      keys[lru] = NULL;
-      if (slot < 0) slot = lru;
+      if (!evict_lru(NULL)) break;
     }
     if (slot < 0) slot = oldest;
     if (spbte_op_create(&ops[slot], N, L_v, v, eta) != SPBTE_OK) die("ComputeQ");
@@ -184,8 +193,10 @@ static void run_q(double *f, double *g, double *Q, double **conv_weights, int fl
     stage_in(df, h_buf, f, b, s, "ComputeQ");
     if (two) stage_in(dg, h_buf + n3, g, b, s, "ComputeQ");
   }
-  if (spbte_compute_q(op, df, g == f ? df : dg, dQ, 1, form_from_env(), flags | (g == f ? SPBTE_SELF : 0)) != SPBTE_OK)
-    die("ComputeQ");
+  /* the first Q(f, f) and the first Q(f, g) of a table build its folded copy: where
+   * that no longer fits, the other tables go first */
+  while (spbte_compute_q(op, df, two ? dg : df, dQ, 1, form_from_env(), flags | (two ? 0 : SPBTE_SELF)) != SPBTE_OK)
+    if (hipGetLastError() != hipErrorOutOfMemory || !evict_lru(op)) die("ComputeQ");
   if (direct) {
     hip_ok(hipStreamSynchronize(s), "ComputeQ");
     memcpy(Q, dQ, b);

@@ -536,11 +536,12 @@ typedef struct {
   void *Qp;    /* partial sums of the split streaming kernel (fixed sets only) */
   size_t qp_bytes;
   int fixed;   /* 1: allocate nothing */
-  int kind;    /* fixed sets: slices of the split streaming kernel (0: the tile's own) */
+  const spbte_tile *tile; /* fixed sets: the tile (NULL: none) */
+  int kind;    /* and its slices */
 } scratch_set;
 
 static scratch_set own_scratch(const spbte_op *op) {
-  scratch_set ss = {op->d_mom, op->d_part, op->d_xs, op->d_FG, op->d_Qh, NULL, 0, 0, 0};
+  scratch_set ss = {op->d_mom, op->d_part, op->d_xs, op->d_FG, op->d_Qh, NULL, 0, 0, NULL, 0};
   return ss;
 }
 
@@ -773,27 +774,23 @@ static int fold_of(const spbte_op *op, int form, const spbte_tile *t, int sum, i
   return 1;
 }
 
-/* The folded tables of a form for tr rows per lane.  Building makes both of them
- * resident (without the mirror symmetry the whole table in place of the
- * row-folded one) and the natural table of the form, so that what one evaluation
- * built serves every later allocation-free one with rows of that tile.  Without
- * build, *Wp is NULL where the one asked for is not resident. */
+/* The folded table of a form for tr rows per lane (columns folded too: cfold), built
+ * with the natural table of the form where it is not resident.  Without build, *Wp is
+ * NULL then. */
 static int weights_folded(spbte_op *op, int form, int tr, int npl, int cfold, int build, const void **Wp) {
   const int st = storage_of(form) == SPBTE_FORM_FP64 ? 0 : 1, N = op->N;
-  for (int c = 0; c < 2 && build; c++) {
-    void **p = &op->t->dWh[c][st][tr];
-    if (*p) continue;
+  void **p = &op->t->dWh[cfold][st][tr];
+  if (!*p && build) {
     const void *w;
     const float *rs;
-    int rc = !c && !op->mirror.on ? weights_permuted(op, form, tr, 1, &w, &rs) : weights_form(op, form, 1, &w, &rs);
+    int rc = weights_form(op, form, 1, &w, &rs);
     if (rc) return rc;
-    if (!c && !op->mirror.on) continue;
-    const size_t rows = (size_t)npl * N * N, cols = (size_t)(c ? N / 2 + 1 : N) * N * N;
+    const size_t rows = (size_t)npl * N * N, cols = (size_t)(cfold ? N / 2 + 1 : N) * N * N;
     HIPCHK(hipMalloc(p, rows * cols * (st ? 4 : 8)));
     op->gen++;
-    LCHK(spbte_launch_fold_weights(op->t->dW64, *p, st, tr, N, npl, c, &op->mirror, op->s));
+    LCHK(spbte_launch_fold_weights(op->t->dW64, *p, st, tr, N, npl, cfold, &op->mirror, op->s));
   }
-  *Wp = op->t->dWh[cfold][st][tr];
+  *Wp = *p;
   return SPBTE_OK;
 }
 
@@ -1025,7 +1022,7 @@ static int launch_tile(spbte_op *op, int form, const spbte_tile *t, const spbte_
     if (!Wp) rc = weights_permuted(op, form, t->tr, !ss->fixed, &Wp, &rs);
     if (rc) return rc;
     void *Qp = NULL;
-    const int k = ss->fixed && ss->kind ? ss->kind : t->kind;
+    const int k = ss->fixed ? ss->kind : t->kind;
     if (k > 1) {
       const size_t need = (size_t)k * a->ncell * op->n3 * 16;
       if (ss->fixed) {
@@ -1088,9 +1085,10 @@ static int run_wsum(spbte_op *op, int form, int nprod, const void *F0, const voi
                     int ncell, int sum, const scratch_set *ss, int keep_slices, wsum_result *res) {
   if (!op->t->have_w) return fail(SPBTE_ERR_NOWEIGHTS, "no weight table set");
   spbte_tile t;
-  int have = pick_tile(op, ncell, form, nprod, sum, &t);
+  int have = ss->fixed ? ss->tile != NULL : pick_tile(op, ncell, form, nprod, sum, &t);
   if (!have && form != SPBTE_FORM_FP64)
     return fail(SPBTE_ERR_UNSUPPORTED, "no reduced-precision weighted-sum kernel for N=%d", op->N);
+  if (ss->fixed && have) t = *ss->tile;
   spbte_wsum_args a = {NULL, F0, G0, F1, G1, ss->Qh, ncell, nprod, keep_slices, 0, 0};
   return launch_tile(op, form, have ? &t : NULL, &a, sum, ss, res);
 }
@@ -1250,7 +1248,9 @@ int spbte_compute_q_noalloc(spbte_op *op, const double *d_f, const double *d_g, 
   if (!d_g) flags |= SPBTE_SELF;
   const int self = (flags & SPBTE_SELF) != 0 || d_g == d_f;
   const int mp = (flags & SPBTE_MAXPRESERVE) != 0;
-  /* the tile compute_chunk will pick, and its table, which must be resident */
+  /* the tile spbte_compute_q would take, and its table, which must be resident; where
+   * only the table of the other kind of call (Q(f, f), Q(f, g)) is, with rows of that
+   * tile, the natural table on its own kernel */
   spbte_tile t;
   const int sum = self ? SUM_SELF : SUM_REAL, have = pick_tile(op, ncell, form, mp ? 2 : 1, sum, &t);
   if (!have && form != SPBTE_FORM_FP64)
@@ -1260,8 +1260,17 @@ int spbte_compute_q_noalloc(spbte_op *op, const double *d_f, const double *d_g, 
   int rc = SPBTE_OK, npl, cfold;
   if (have && fold_of(op, form, &t, sum, &npl, &cfold))
     rc = weights_folded(op, form, t.tr, npl, cfold, 0, &W);
-  if (!rc && !W)
-    rc = (have && t.kind >= 1) ? weights_permuted(op, form, t.tr, 0, &W, &rs) : weights_form(op, form, 0, &W, &rs);
+  if (!rc && !W && have && t.kind >= 1) {
+    rc = weights_permuted(op, form, t.tr, 0, &W, &rs);
+    const int st = storage_of(form) == SPBTE_FORM_FP64 ? 0 : 1;
+    spbte_tile nat;
+    if (rc && form != SPBTE_FORM_FP16X2 && (op->t->dWh[0][st][t.tr] || op->t->dWh[1][st][t.tr]) &&
+        default_tile(op->N, form, mp ? 2 : 1, ncell, &nat)) {
+      t = nat;
+      rc = SPBTE_OK;
+    }
+  }
+  if (!rc && !W) rc = weights_form(op, form, 0, &W, &rs);
   if (rc) return rc;
   /* workspace: moments | partial sums | transformed operands | Qhat | transform scratch,
    * which also holds the split sum's partial sums (they are dead by the time
@@ -1299,6 +1308,7 @@ int spbte_compute_q_noalloc(spbte_op *op, const double *d_f, const double *d_g, 
   ss.Qp = ss.xs;
   ss.qp_bytes = b_x;
   ss.fixed = 1;
+  ss.tile = have ? &t : NULL;
   ss.kind = kind;
   return compute_chunk(op, d_f, d_g, d_Q, ncell, form, flags, NULL, NULL, &ss, NULL);
 }
