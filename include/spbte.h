@@ -133,10 +133,14 @@ int spbte_compute_q(spbte_op *op, const double *d_f, const double *d_g, double *
  * d_Q lives in a fixed workspace of SPBTE_NOALLOC_SCRATCH_BYTES per GPU,
  * held by the library from the first spbte_op_create on that GPU until the
  * process ends, and the call allocates and frees nothing.  Limits: the batch
- * must fit the workspace (about 10 cells at N=32 and 80 at N=16 for
- * maxPreserve in FP64); larger batches, and tables not yet resident in the
- * layout the batch's tile streams (spbte_compute_q and spbte_autotune build
- * them on first use), return SPBTE_ERR_ARG without launching anything.  All
+ * must fit the workspace (about 18 cells at N=32 and 140 at N=16 for
+ * maxPreserve in FP64; beyond about 3 and 80 the sum goes part by part, which
+ * costs time and changes no bit); larger batches, and tables not yet resident in
+ * the layout the batch's tile streams (spbte_compute_q and spbte_autotune build
+ * them on first use), return SPBTE_ERR_ARG without launching anything.  That
+ * layout is Q(f, f)'s or Q(f, g)'s own: where a call of the other kind alone has
+ * been made with the tile, and on grids without tiles where none has, the table
+ * in its natural order is summed, more slowly and with other rounding.  All
  * operators on one GPU share its workspace and each call overwrites it, so
  * calls that overlap on one GPU (other threads, other streams) race: order
  * them on one stream or synchronise between them. */

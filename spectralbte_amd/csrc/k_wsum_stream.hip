@@ -127,7 +127,7 @@ template <int N, int TR, int WAVES, int TB, int NP, int FORM, bool NTW, int CPW>
 __global__ void __launch_bounds__(64 * WAVES * CPW) __attribute__((amdgpu_waves_per_eu(kWavesPerEU<TR, WAVES, TB, FORM>)))
 k_wsum_stream(const uint4 *__restrict__ Wp, const float *__restrict__ rowscale, const double2 *__restrict__ F0,
               const double2 *__restrict__ G0, const double2 *__restrict__ F1, const double2 *__restrict__ G1,
-              double2 *__restrict__ Qh, int ncell, int csplit, double2 *__restrict__ Qp, int npl, int fold) {
+              double2 *__restrict__ Qh, int ncell, int csplit, double2 *__restrict__ Qp, int npl, int fold, int gsum) {
   using Gm = SGeom<N, TR, WAVES>;
   constexpr int N2 = Gm::N2, P = Gm::P, RWG = Gm::RWG;
   constexpr size_t n3 = (size_t)N * N * N;
@@ -198,8 +198,8 @@ k_wsum_stream(const uint4 *__restrict__ Wp, const float *__restrict__ rowscale, 
   const C *Gp[2] = {(const C *)G0, (const C *)G1};
   const float *Gsum[2] = {nullptr, nullptr};
   if constexpr (GS) {
-    Gsum[0] = (const float *)(Gp[0] + (size_t)ncell * n3);
-    if constexpr (NP == 2) Gsum[1] = (const float *)(Gp[1] + (size_t)ncell * n3);
+    Gsum[0] = (const float *)Gp[0] + (size_t)gsum * n3;
+    if constexpr (NP == 2) Gsum[1] = (const float *)Gp[1] + (size_t)gsum * n3;
   }
   int cells[TB];
 #pragma unroll
@@ -504,12 +504,12 @@ int launch_s(const spbte_wsum_args *a, const void *Wp, const float *rowscale, in
       hipLaunchKernelGGL((k_wsum_stream<N, TR, WAVES, TB, NP, FORM, true, 1>), dim3(8 * per), dim3(64 * WAVES), 0, s,
                          (const uint4 *)Wp, rowscale, (const double2 *)a->F0, (const double2 *)a->G0,
                          (const double2 *)a->F1, (const double2 *)a->G1, (double2 *)a->Qh, a->ncell, csplit,
-                         (double2 *)Qp, npl, npl != N || cfold ? 2 + cfold : 0);
+                         (double2 *)Qp, npl, npl != N || cfold ? 2 + cfold : 0, a->gsum);
   if (!nt)
     hipLaunchKernelGGL((k_wsum_stream<N, TR, WAVES, TB, NP, FORM, false, CPW>), dim3(8 * per), dim3(64 * WAVES * CPW), 0,
                        s, (const uint4 *)Wp, rowscale, (const double2 *)a->F0, (const double2 *)a->G0,
                        (const double2 *)a->F1, (const double2 *)a->G1, (double2 *)a->Qh, a->ncell, csplit,
-                       (double2 *)Qp, npl, npl != N || cfold ? 2 + cfold : 0);
+                       (double2 *)Qp, npl, npl != N || cfold ? 2 + cfold : 0, a->gsum);
   if (csplit > 1 && !a->keep_slices) return spbte_launch_slice_sum(N, a->ncell, csplit, Qp, a->Qh, s);
   return (int)hipGetLastError();
 }

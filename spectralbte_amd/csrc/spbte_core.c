@@ -537,11 +537,10 @@ typedef struct {
   size_t qp_bytes;
   int fixed;   /* 1: allocate nothing */
   const spbte_tile *tile; /* fixed sets: the tile (NULL: none) */
-  int kind;    /* and its slices */
 } scratch_set;
 
 static scratch_set own_scratch(const spbte_op *op) {
-  scratch_set ss = {op->d_mom, op->d_part, op->d_xs, op->d_FG, op->d_Qh, NULL, 0, 0, NULL, 0};
+  scratch_set ss = {op->d_mom, op->d_part, op->d_xs, op->d_FG, op->d_Qh, NULL, 0, 0, NULL};
   return ss;
 }
 
@@ -1000,6 +999,54 @@ typedef struct {
   int npl;       /* x-planes of each cube that hold it (the others are zero, not written) */
 } wsum_result;
 
+/* A sum in k slices on a streaming tile (t) or, without one, in k_wsum_any.hip, with the
+ * partial sums of up to cap cells at a time in Qp.  Larger batches go part by part,
+ * each added into Qh: a cell's result depends on the slices alone, so it is the same
+ * to the last bit (a tile with fewer slices would round differently). */
+static int launch_split(spbte_op *op, int form, const spbte_tile *t, const spbte_wsum_args *a, const void *W,
+                        const float *rs, int k, int cap, void *Qp, wsum_result *res) {
+  const int n = a->ncell;
+  const int part = cap >= n ? n : (n + (n + cap - 1) / cap - 1) / ((n + cap - 1) / cap);
+  const size_t es = fg_bytes(form) * op->n3;
+  for (int c0 = 0; c0 < n; c0 += part) {
+    spbte_wsum_args b = *a;
+    b.ncell = n - c0 < part ? n - c0 : part;
+    b.F0 = (const char *)a->F0 + c0 * es;
+    b.G0 = (const char *)a->G0 + c0 * es;
+    if (a->nprod == 2) {
+      b.F1 = (const char *)a->F1 + c0 * es;
+      b.G1 = (const char *)a->G1 + c0 * es;
+    }
+    b.Qh = (char *)a->Qh + c0 * 16 * op->n3;
+    b.gsum = 2 * n - c0;
+    b.keep_slices = a->keep_slices && part == n;
+    if (t) LCHK(spbte_launch_wsum_stream(op->N, form, t->tr, t->lines, t->tb, &b, W, rs, k, Qp, op->s));
+    else LCHK(spbte_launch_wsum_any(op->N, &b, W, k, Qp, op->s));
+  }
+  if (a->keep_slices && part == n && k > 1) {
+    res->q = Qp;
+    res->nsl = k;
+  }
+  return SPBTE_OK;
+}
+
+/* Where the partial sums of a sum in k slices go, and those of how many cells it holds. */
+static int partials(spbte_op *op, const scratch_set *ss, int k, int ncell, void **Qp, int *cap) {
+  const size_t one = (size_t)k * op->n3 * 16;
+  *Qp = NULL;
+  *cap = ncell;
+  if (k <= 1) return SPBTE_OK;
+  if (ss->fixed) {
+    if (one > ss->qp_bytes) return fail(SPBTE_ERR_ARG, "partial sums need %zu bytes of workspace", one);
+    if (one * ncell > ss->qp_bytes) *cap = (int)(ss->qp_bytes / one);
+    *Qp = ss->Qp;
+    return SPBTE_OK;
+  }
+  int rc = ensure_partials(op, one * ncell);
+  *Qp = op->d_Qp;
+  return rc;
+}
+
 /* The weighted sum's result is left as res->nsl sets to add: Qh (one set),
  * or, with a->keep_slices, a split tile's unsummed slices in Qp. */
 static int launch_tile(spbte_op *op, int form, const spbte_tile *t, const spbte_wsum_args *a0, int sum,
@@ -1007,6 +1054,8 @@ static int launch_tile(spbte_op *op, int form, const spbte_tile *t, const spbte_
   const float *rs = NULL;
   spbte_wsum_args b = *a0;
   const spbte_wsum_args *a = &b;
+  void *Qp;
+  int cap;
   res->q = a->Qh;
   res->nsl = 1;
   res->npl = op->N;
@@ -1020,26 +1069,8 @@ static int launch_tile(spbte_op *op, int form, const spbte_tile *t, const spbte_
       else b.npl = b.cfold = 0;
     }
     if (!Wp) rc = weights_permuted(op, form, t->tr, !ss->fixed, &Wp, &rs);
-    if (rc) return rc;
-    void *Qp = NULL;
-    const int k = ss->fixed ? ss->kind : t->kind;
-    if (k > 1) {
-      const size_t need = (size_t)k * a->ncell * op->n3 * 16;
-      if (ss->fixed) {
-        if (need > ss->qp_bytes) return fail(SPBTE_ERR_ARG, "partial sums need %zu bytes of workspace", need);
-        Qp = ss->Qp;
-      } else {
-        rc = ensure_partials(op, need);
-        if (rc) return rc;
-        Qp = op->d_Qp;
-      }
-    }
-    LCHK(spbte_launch_wsum_stream(op->N, form, t->tr, t->lines, t->tb, a, Wp, rs, k, Qp, op->s));
-    if (a->keep_slices && k > 1) {
-      res->q = Qp;
-      res->nsl = k;
-    }
-    return SPBTE_OK;
+    if (!rc) rc = partials(op, ss, t->kind, a->ncell, &Qp, &cap);
+    return rc ? rc : launch_split(op, form, t, a, Wp, rs, t->kind, cap, Qp, res);
   }
   if (!t && sum != SUM_ANY && spbte_any_supported(op->N)) {
     void **Wa = &op->t->dWa[sum == SUM_SELF];
@@ -1051,24 +1082,11 @@ static int launch_tile(spbte_op *op, int form, const spbte_tile *t, const spbte_
       LCHK(spbte_launch_fold_any(op->t->dW64, *Wa, op->N, b.npl, b.cfold, &op->mirror, op->s));
     }
     if (*Wa) { /* else an allocation-free call before the first of its kind: the whole table, which is always there */
-      int k = spbte_any_slices(op->N, b.npl, b.cfold, a->nprod, a->ncell);
-      void *Qp = NULL;
-      const size_t one = (size_t)a->ncell * op->n3 * 16;
-      if (ss->fixed) {
-        k = ss->kind;
-        Qp = ss->Qp;
-      } else if (k > 1) {
-        int rc = ensure_partials(op, one * k);
-        if (rc) return rc;
-        Qp = op->d_Qp;
-      }
-      LCHK(spbte_launch_wsum_any(op->N, a, *Wa, k, Qp, op->s));
+      const int k = spbte_any_slices(op->N, b.npl, b.cfold, a->nprod, a->ncell);
+      int rc = partials(op, ss, k, a->ncell, &Qp, &cap);
+      if (rc) return rc;
       res->npl = b.npl;
-      if (a->keep_slices && k > 1) {
-        res->q = Qp;
-        res->nsl = k;
-      }
-      return SPBTE_OK;
+      return launch_split(op, form, NULL, a, *Wa, NULL, k, cap, Qp, res);
     }
     b.npl = b.cfold = 0;
   }
@@ -1089,7 +1107,7 @@ static int run_wsum(spbte_op *op, int form, int nprod, const void *F0, const voi
   if (!have && form != SPBTE_FORM_FP64)
     return fail(SPBTE_ERR_UNSUPPORTED, "no reduced-precision weighted-sum kernel for N=%d", op->N);
   if (ss->fixed && have) t = *ss->tile;
-  spbte_wsum_args a = {NULL, F0, G0, F1, G1, ss->Qh, ncell, nprod, keep_slices, 0, 0};
+  spbte_wsum_args a = {NULL, F0, G0, F1, G1, ss->Qh, ncell, nprod, keep_slices, 0, 0, 0};
   return launch_tile(op, form, have ? &t : NULL, &a, sum, ss, res);
 }
 
@@ -1272,28 +1290,21 @@ int spbte_compute_q_noalloc(spbte_op *op, const double *d_f, const double *d_g, 
   }
   if (!rc && !W) rc = weights_form(op, form, 0, &W, &rs);
   if (rc) return rc;
-  /* workspace: moments | partial sums | transformed operands | Qhat | transform scratch,
-   * which also holds the split sum's partial sums (they are dead by the time
-   * the inverse transform writes it) */
+  /* workspace: moments | partial sums | transformed operands | Qhat | transform scratch.
+   * The last one is all the rest: it also holds the split sum's partial sums, of as
+   * many cells at a time as it has room for (they are dead by the time the inverse
+   * transform writes it) */
   const int nj = mp ? (self ? 3 : 4) : (self ? 1 : 2);
   const size_t n = (size_t)ncell * op->n3;
   const size_t b_mom = al256(sizeof(double) * 2 * (size_t)ncell * SPBTE_MOM_STRIDE);
   const size_t b_part = al256(sizeof(double) * 10 * (size_t)op->N * ncell);
   const size_t b_fg = al256((size_t)nj * fg_stride(form, n)), b_qh = al256(16 * n);
   const size_t b_xs = 16 * n * (size_t)nj, b_fix = b_mom + b_part + b_fg + b_qh;
-  /* a tile that was not pinned or tuned takes fewer slices where the workspace
-   * does not hold its own number (the sums then differ by rounding) */
   int kind = have ? t.kind : 0;
-  spbte_tile dt;
-  const int is_default = have && op_stream_tile(op, ncell, form, mp ? 2 : 1, sum, &dt) && !memcmp(&dt, &t, sizeof t);
-  while (is_default && kind > 1 && b_fix + al256(16 * n * (size_t)kind) > op->nac_bytes) kind--;
-  if (!have && spbte_any_supported(op->N)) { /* likewise */
+  if (!have && op->t->dWa[sum == SUM_SELF])
     kind = spbte_any_slices(op->N, op->mirror.on ? op->N / 2 + 1 : op->N, self, mp ? 2 : 1, ncell);
-    while (kind > 1 && b_fix + al256(16 * n * (size_t)kind) > op->nac_bytes) kind--;
-  }
-  const size_t b_qp = kind > 1 ? 16 * n * (size_t)kind : 0;
-  const size_t b_x = al256(b_xs > b_qp ? b_xs : b_qp);
-  const size_t need = b_fix + b_x;
+  const size_t b_qp = kind > 1 ? 16 * op->n3 * (size_t)kind : 0; /* one cell's */
+  const size_t need = b_fix + al256(b_xs > b_qp ? b_xs : b_qp);
   if (need > op->nac_bytes)
     return fail(SPBTE_ERR_ARG, "a batch of %d cells at N=%d needs %zu bytes of workspace, more than the %zu of the "
                 "fixed workspace (SPBTE_NOALLOC_SCRATCH_BYTES)", ncell, op->N, need, op->nac_bytes);
@@ -1306,10 +1317,9 @@ int spbte_compute_q_noalloc(spbte_op *op, const double *d_f, const double *d_g, 
   ss.Qh = base + b_fg;
   ss.xs = base + b_fg + b_qh;
   ss.Qp = ss.xs;
-  ss.qp_bytes = b_x;
+  ss.qp_bytes = op->nac_bytes - b_fix;
   ss.fixed = 1;
   ss.tile = have ? &t : NULL;
-  ss.kind = kind;
   return compute_chunk(op, d_f, d_g, d_Q, ncell, form, flags, NULL, NULL, &ss, NULL);
 }
 
@@ -1468,7 +1478,7 @@ int spbte_autotune(spbte_op *op, int ncell, int form, int maxpreserve, int *kind
   char *FG = (char *)op->d_FG;
   LCHK(spbte_launch_fill_pattern(FG, 4 * stride / (single ? 4 : 8), single, op->s));
   spbte_wsum_args args = {NULL, FG, FG + stride, np == 2 ? FG + 2 * stride : NULL, np == 2 ? FG + 3 * stride : NULL,
-                          op->d_Qh, ncell, np, 0, 0, 0};
+                          op->d_Qh, ncell, np, 0, 0, 0, 0};
   const scratch_set ss = own_scratch(op);
   spbte_tile best = {0, 0, 0, 0};
   float best_ms = 1e30f;

@@ -61,6 +61,9 @@ typedef struct {
   int npl, cfold;     /* streaming kernel on a folded table: x-planes of output rows
                          it holds (0: all N; the others of Qh are not written), and
                          whether its columns are folded too */
+  int gsum;           /* streaming kernel, FP32-product form: where the sums of G's values
+                         are, in units of N^3 floats from G (2 * ncell, but for a part
+                         of a batch) */
 } spbte_wsum_args;
 
 #ifdef __HIPCC__
