@@ -325,6 +325,6 @@ extern "C" int spbte_launch_wsum_any(int N, const spbte_wsum_args *a, const void
       else launch_np<0, 1>(N, npl, cf, tb, a, Wf, csplit, Qp, s);
       break;
   }
-  if (csplit > 1 && !a->keep_slices) return spbte_launch_slice_sum(N, a->ncell, csplit, Qp, a->Qh, s);
+  if (csplit > 1 && !a->keep_slices) return spbte_launch_slice_sum(N, npl, a->ncell, csplit, Qp, a->Qh, s);
   return (int)hipGetLastError();
 }

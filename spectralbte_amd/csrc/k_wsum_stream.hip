@@ -474,12 +474,15 @@ k_wsum_stream(const uint4 *__restrict__ Wp, const float *__restrict__ rowscale, 
 }
 
 // Qh[b][r] = sum over the csplit slices of Qp[s][b][r].
-__global__ void __launch_bounds__(256) k_slice_sum(size_t n, int csplit, const double2 *__restrict__ Qp,
+// Only the first m of each cube's n3 values are there and wanted (the kept planes).
+__global__ void __launch_bounds__(256) k_slice_sum(size_t m, size_t n3, int ncell, int csplit, const double2 *__restrict__ Qp,
                                                    double2 *__restrict__ Qh) {
-  for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)gridDim.x * 256) {
+  const size_t n = m * ncell, set = n3 * ncell;
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+    const size_t e = i / m * n3 + i % m;
     double2 v = Qp[e];
     for (int s = 1; s < csplit; ++s) {
-      const double2 w = Qp[(size_t)s * n + e];
+      const double2 w = Qp[(size_t)s * set + e];
       v.x += w.x;
       v.y += w.y;
     }
@@ -510,7 +513,7 @@ int launch_s(const spbte_wsum_args *a, const void *Wp, const float *rowscale, in
                        s, (const uint4 *)Wp, rowscale, (const double2 *)a->F0, (const double2 *)a->G0,
                        (const double2 *)a->F1, (const double2 *)a->G1, (double2 *)a->Qh, a->ncell, csplit,
                        (double2 *)Qp, npl, npl != N || cfold ? 2 + cfold : 0, a->gsum);
-  if (csplit > 1 && !a->keep_slices) return spbte_launch_slice_sum(N, a->ncell, csplit, Qp, a->Qh, s);
+  if (csplit > 1 && !a->keep_slices) return spbte_launch_slice_sum(N, npl, a->ncell, csplit, Qp, a->Qh, s);
   return (int)hipGetLastError();
 }
 
@@ -671,10 +674,10 @@ extern "C" int spbte_csplit_valid(int N, int csplit) {
   return csplit % N == 0 && N % (csplit / N) == 0;
 }
 
-extern "C" int spbte_launch_slice_sum(int N, int ncell, int csplit, const void *Qp, void *Qh, hipStream_t s) {
-  const size_t n = (size_t)ncell * N * N * N;
-  hipLaunchKernelGGL(k_slice_sum, dim3((unsigned)((n + 255) / 256 < 16384 ? (n + 255) / 256 : 16384)), dim3(256), 0, s, n,
-                     csplit, (const double2 *)Qp, (double2 *)Qh);
+extern "C" int spbte_launch_slice_sum(int N, int npl, int ncell, int csplit, const void *Qp, void *Qh, hipStream_t s) {
+  const size_t m = (size_t)npl * N * N, n = m * ncell;
+  hipLaunchKernelGGL(k_slice_sum, dim3((unsigned)((n + 255) / 256 < 16384 ? (n + 255) / 256 : 16384)), dim3(256), 0, s, m,
+                     (size_t)N * N * N, ncell, csplit, (const double2 *)Qp, (double2 *)Qh);
   return (int)hipGetLastError();
 }
 

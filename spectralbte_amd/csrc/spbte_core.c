@@ -57,6 +57,11 @@ int spbte_fail(int code, const char *fmt, ...) {
 #define NFORMS 4
 #define MAXJOBS 4
 
+/* Bytes of scratch for one pass over a batch, and as many for the partial sums of its
+ * split sum, which takes more cells than that hold part by part (N=32 with FP32
+ * products: 768 of a pass's 1365). */
+#define SCRATCH_BUDGET ((size_t)6 << 30)
+
 struct spbte_op {
   spbte_grid_dev g;
   int N;
@@ -91,7 +96,7 @@ struct spbte_op {
   spbte_tile tuned[NFORMS][2][16];
   /* partial sums of the split streaming kernel */
   void *d_Qp;
-  size_t qp_bytes;
+  size_t qp_bytes, qp_limit;
   /* the fixed workspace of spbte_compute_q_noalloc on this operator's GPU */
   void *nac;
   size_t nac_bytes;
@@ -368,6 +373,7 @@ int spbte_op_create(spbte_op **out, int N, double L_v, const double *v, const do
   op->t = &op->tab[0];
   op->N = N;
   op->n3 = (size_t)N * N * N;
+  op->qp_limit = SCRATCH_BUDGET;
   op->v = malloc(sizeof(double) * N);
   op->eta = malloc(sizeof(double) * N);
   if (!op->v || !op->eta) {
@@ -499,8 +505,7 @@ void spbte_op_destroy(spbte_op *op) {
 /* Largest batch evaluated in one pass; bigger batches are processed in chunks. */
 static int chunk_cells(const spbte_op *op) {
   size_t per_cell = op->n3 * 16 * (2 * MAXJOBS + 1);
-  size_t budget = (size_t)6 << 30; /* 6 GiB of scratch */
-  size_t c = budget / per_cell;
+  size_t c = SCRATCH_BUDGET / per_cell;
   if (c > 4096) c = 4096;
   if (c < 1) c = 1;
   return (int)c;
@@ -959,16 +964,29 @@ static int tile_supported(int N, int form, int nprod, const spbte_tile *t) {
 }
 
 
-/* Partial sums of the split streaming kernel: csplit * ncell * N^3 double2. */
-static int ensure_partials(spbte_op *op, size_t bytes) {
-  if (bytes <= op->qp_bytes) return SPBTE_OK;
-  HIPCHK(hipStreamSynchronize(op->s));
-  if (op->d_Qp) hipFree(op->d_Qp);
-  op->d_Qp = NULL;
-  op->qp_bytes = 0;
-  HIPCHK(hipMalloc(&op->d_Qp, bytes));
-  op->qp_bytes = bytes;
-  op->gen++;
+/* Room for the partial sums (one bytes a cell) of up to ncell cells, *cap of them: as
+ * many as op->qp_limit allows, which a failed allocation lowers for good, so that a
+ * sequence captured in a graph finds what its eager run got.  0: not even one's. */
+static int ensure_partials(spbte_op *op, size_t one, int ncell, int *cap) {
+  const size_t most = op->qp_limit / one;
+  *cap = most < (size_t)ncell ? (int)most : ncell;
+  while (*cap > 0 && *cap * one > op->qp_bytes) {
+    HIPCHK(hipStreamSynchronize(op->s));
+    if (op->d_Qp) hipFree(op->d_Qp);
+    op->d_Qp = NULL;
+    op->qp_bytes = 0;
+    op->gen++;
+    const hipError_t e = hipMalloc(&op->d_Qp, *cap * one);
+    if (e == hipSuccess) {
+      op->qp_bytes = *cap * one;
+      break;
+    }
+    op->d_Qp = NULL;
+    if (e != hipErrorOutOfMemory) return fail(SPBTE_ERR_HIP, "partial sums: %s", hipGetErrorString(e));
+    (void)hipGetLastError();
+    *cap /= 2;
+    op->qp_limit = *cap * one;
+  }
   return SPBTE_OK;
 }
 
@@ -1030,20 +1048,26 @@ static int launch_split(spbte_op *op, int form, const spbte_tile *t, const spbte
   return SPBTE_OK;
 }
 
-/* Where the partial sums of a sum in k slices go, and those of how many cells it holds. */
-static int partials(spbte_op *op, const scratch_set *ss, int k, int ncell, void **Qp, int *cap) {
-  const size_t one = (size_t)k * op->n3 * 16;
+/* Where the partial sums of a sum in *k slices go, and those of how many cells it
+ * holds.  Without room for one cell's the sum is not split (and rounds differently). */
+static int partials(spbte_op *op, const scratch_set *ss, int *k, int ncell, void **Qp, int *cap) {
+  const size_t one = (size_t)*k * op->n3 * 16;
   *Qp = NULL;
   *cap = ncell;
-  if (k <= 1) return SPBTE_OK;
+  if (*k <= 1) return SPBTE_OK;
   if (ss->fixed) {
     if (one > ss->qp_bytes) return fail(SPBTE_ERR_ARG, "partial sums need %zu bytes of workspace", one);
     if (one * ncell > ss->qp_bytes) *cap = (int)(ss->qp_bytes / one);
     *Qp = ss->Qp;
     return SPBTE_OK;
   }
-  int rc = ensure_partials(op, one * ncell);
+  int rc = ensure_partials(op, one, ncell, cap);
   *Qp = op->d_Qp;
+  if (!rc && *cap == 0) {
+    *k = 1;
+    *cap = ncell;
+    *Qp = NULL;
+  }
   return rc;
 }
 
@@ -1069,8 +1093,9 @@ static int launch_tile(spbte_op *op, int form, const spbte_tile *t, const spbte_
       else b.npl = b.cfold = 0;
     }
     if (!Wp) rc = weights_permuted(op, form, t->tr, !ss->fixed, &Wp, &rs);
-    if (!rc) rc = partials(op, ss, t->kind, a->ncell, &Qp, &cap);
-    return rc ? rc : launch_split(op, form, t, a, Wp, rs, t->kind, cap, Qp, res);
+    int k = t->kind;
+    if (!rc) rc = partials(op, ss, &k, a->ncell, &Qp, &cap);
+    return rc ? rc : launch_split(op, form, t, a, Wp, rs, k, cap, Qp, res);
   }
   if (!t && sum != SUM_ANY && spbte_any_supported(op->N)) {
     void **Wa = &op->t->dWa[sum == SUM_SELF];
@@ -1082,8 +1107,8 @@ static int launch_tile(spbte_op *op, int form, const spbte_tile *t, const spbte_
       LCHK(spbte_launch_fold_any(op->t->dW64, *Wa, op->N, b.npl, b.cfold, &op->mirror, op->s));
     }
     if (*Wa) { /* else an allocation-free call before the first of its kind: the whole table, which is always there */
-      const int k = spbte_any_slices(op->N, b.npl, b.cfold, a->nprod, a->ncell);
-      int rc = partials(op, ss, k, a->ncell, &Qp, &cap);
+      int k = spbte_any_slices(op->N, b.npl, b.cfold, a->nprod, a->ncell);
+      int rc = partials(op, ss, &k, a->ncell, &Qp, &cap);
       if (rc) return rc;
       res->npl = b.npl;
       return launch_split(op, form, NULL, a, *Wa, NULL, k, cap, Qp, res);

@@ -182,8 +182,9 @@ int spbte_stream_tile_supported(int N, int form, int nprod, int tr, int waves, i
 int spbte_csplit_valid(int N, int csplit);
 int spbte_launch_wsum_stream(int N, int form, int tr, int waves, int tb, const spbte_wsum_args *a, const void *Wp,
                              const float *rowscale, int csplit, void *Qp, hipStream_t s);
-/* Qh = the sum of csplit sets of ncell * N^3 double2 at Qp. */
-int spbte_launch_slice_sum(int N, int ncell, int csplit, const void *Qp, void *Qh, hipStream_t s);
+/* Qh = the sum of csplit sets of ncell * N^3 double2 at Qp, the first npl x-planes of
+ * each cube. */
+int spbte_launch_slice_sum(int N, int npl, int ncell, int csplit, const void *Qp, void *Qh, hipStream_t s);
 /* k_wsum_any.hip: folded FP64 sums on grids without streaming tiles (a->npl and
  * a->cfold as for those; slices of its own choice, or fewer). */
 int spbte_any_supported(int N);

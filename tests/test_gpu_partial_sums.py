@@ -1,5 +1,7 @@
 """Split sums whose partial sums do not fit their buffer go part of the batch by part, with the same slices: the results
 are those of one launch, bit for bit."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -41,4 +43,62 @@ def test_noalloc_part_by_part(spb, N, n, form, mp, how):
     assert L.spbte_compute_q_noalloc(op.h, d_f.ptr, None, d_Q.ptr, n, FORMS[form], flags) == 0, L.spbte_last_error()
     op.sync()
     assert np.array_equal(d_Q.download(), ref)
+    op.close()
+
+
+def _free(spb):
+    a, b = ctypes.c_size_t(), ctypes.c_size_t()
+    assert spb.lib().hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0   # from the runtime the library is linked to
+    return a.value
+
+
+def _growth(spb, op, d_f, d_Q, n, form, flags):
+    free = _free(spb)
+    assert spb.lib().spbte_compute_q(op.h, d_f.ptr, None, d_Q.ptr, n, FORMS[form], flags) == 0, spb.lib().spbte_last_error()
+    op.sync()
+    return free - _free(spb)
+
+
+def _unsplit_first(spb, op, d_f, d_Q, n, form, flags):
+    """Scratch and tables of a batch without partial sums; leaves the batch's own tile, which it returns, to be split."""
+    tile = op.get_tile(n, form, True)
+    op.set_tile(form, True, *tile[1:], kind=1)
+    _growth(spb, op, d_f, d_Q, n, form, flags)
+    op.set_tile(form, True, 0, 0, 0)
+    return tile
+
+
+def test_partial_sums_of_a_large_batch_are_bounded(spb):
+    """1000 problems at N = 32 with FP32 products, 16 slices: 7.8 GiB of partial sums at once, 6 GiB at most are kept."""
+    N, n, form, flags = 32, 1000, "fp32a", spb.SELF | spb.MAXPRESERVE
+    op, workloads = _op(spb, N)
+    f = np.resize(workloads.two_maxwellian_ensemble(N, 6.0, 50, seed=1), (n, N ** 3)) * (1 + np.arange(n)[:, None] / n)
+    d_f, d_Q = spb.DeviceArray.from_host(f), spb.DeviceArray(f.shape)
+    tile = _unsplit_first(spb, op, d_f, d_Q, n, form, flags)
+    assert tile[0] == 16
+    assert _growth(spb, op, d_f, d_Q, n, form, flags) <= (6 << 30) + (64 << 20)
+    q = d_Q.download()
+    op.set_tile(form, True, *tile[1:], kind=tile[0])
+    some = [0, 1, 499, 500, 501, 998, 999]   # on both sides of the parts
+    assert np.array_equal(op.compute_q(f[some], form=form, maxpreserve=True), q[some])
+    op.close()
+
+
+def test_partial_sums_without_room(spb):
+    """Memory short of the partial sums (64 cells at N = 32: 256 MiB): the batch goes in smaller parts."""
+    N, n, form, flags = 32, 64, "fp64", spb.SELF | spb.MAXPRESERVE
+    op, workloads = _op(spb, N)
+    f = workloads.two_maxwellian_ensemble(N, 6.0, n, seed=2)
+    d_f, d_Q = spb.DeviceArray.from_host(f), spb.DeviceArray(f.shape)
+    tile = _unsplit_first(spb, op, d_f, d_Q, n, form, flags)
+    hold = []
+    while _free(spb) > 180 << 20 and len(hold) < 100:
+        hold.append(spb.DeviceArray((min(_free(spb) - (160 << 20), 8 << 30) // 8,)))
+    grown = _growth(spb, op, d_f, d_Q, n, form, flags)
+    q = d_Q.download()
+    hold.clear()
+    assert grown <= 160 << 20 < tile[0] * n * 16 * N ** 3
+    op.set_tile(form, True, *tile[1:], kind=tile[0])
+    assert np.array_equal(op.compute_q(f[:3], form=form, maxpreserve=True), q[:3])
+    assert np.array_equal(op.compute_q(f[-3:], form=form, maxpreserve=True), q[-3:])
     op.close()
