@@ -25,10 +25,7 @@
 //    wave-wide load reads 1 KiB of contiguous HBM, in consumption order.
 // Precision forms: 0 FP64 W, 1 FP32 W, 2 FP16x2 W with FP64 arithmetic; 3 FP32 W
 // with FP32 F, G (8-byte LDS entries, half the LDS), FP32 products and FP32
-// partial sums added into FP64 accumulators every 8 steps.  Over 3 Heun steps of
-// 48 N=32 problems (lambda=1, L_v=8.5) the state is 1.30e-9 off the FP64 form's,
-// 1.64e-9 with 32-step partial sums, for 2% of the time (512 problems: 38650 us
-// against 37870); the sum over the whole table with 32 steps was 1.36e-9 off.
+// partial sums added into FP64 accumulators every 4 steps (kSteps32).
 //
 // Folded tables (k_fold_w below).  Cells are real and only the real part of the
 // inverse transform is kept, so half of the output modes determine Q, and in
@@ -122,6 +119,19 @@ __device__ __forceinline__ auto wget(const u32x4 &u, const u32x4 &u2, int j) {
 // slower: it runs at 141 VGPRs, three waves per SIMD.)
 template <int TR, int WAVES, int TB, int FORM>
 constexpr int kWavesPerEU = (TB >= 4 && FORM != 3) ? 2 : 1;
+
+// Steps per FP32 partial sum.  On a folded table a product's rounding counts with the
+// weights of its partner and its images as well, where the whole table's terms round
+// independently; shorter partial sums make up for it.  Error against the FP64 form
+// (1e-7 of Q, geometric mean over L_v = 5 to 8.5 and lambda 0, 1; bimodal cells): the
+// whole table's sum with 32 steps (N=24: 8), then the folded one's with 8, 4 and 2:
+//   maxPreserve  N=16 1.17; 1.25, 1.05, 0.94   N=24 1.14; 1.26, 1.18, 1.05   N=32 1.50; 1.57, 1.37
+//   Q(f, f)      N=16 2.97; 2.90, 2.52         N=24 3.34; 2.88, 2.74         N=32 3.75; 3.61, 3.16
+//   Q(f, g)      N=16 0.95; 1.03, 0.89         N=24 0.89; 0.84, 0.79         N=32 1.04; 1.09, 0.92
+// Time, 8, 4 and 2 steps: 512 N=32 cells maxPreserve 41.2, 42.5 ms, Q(f, f) 24.1, 25.5;
+// 512 N=24 cells maxPreserve 8.24, 8.54, 9.17; 600 N=16 cells maxPreserve 1.31, 1.35, 1.42.
+template <int N, int NP>
+constexpr int kSteps32 = N == 24 ? (NP == 2 ? 2 : 8) : 4;
 
 template <int N, int TR, int WAVES, int TB, int NP, int FORM, bool NTW, int CPW>
 __global__ void __launch_bounds__(64 * WAVES * CPW) __attribute__((amdgpu_waves_per_eu(kWavesPerEU<TR, WAVES, TB, FORM>)))
@@ -413,18 +423,18 @@ k_wsum_stream(const uint4 *__restrict__ Wp, const float *__restrict__ rowscale, 
                 }
             }
           }
-        }
-        if constexpr (FORM == 3) {
-          if ((jb + 4) % 8 != 0) return;  // 8 steps per FP32 partial sum
-          // fold the FP32 partial sums into FP64
+          if constexpr (FORM == 3) {
+            if ((j + 1) % kSteps32<N, NP> != 0) continue;
+            // fold the FP32 partial sums into FP64
 #pragma unroll
-          for (int b = 0; b < TB; ++b)
+            for (int b = 0; b < TB; ++b)
 #pragma unroll
-            for (int t = 0; t < TR; ++t) {
-              acc[b][t].x += (double)a32[b][t].x;
-              acc[b][t].y += (double)a32[b][t].y;
-              a32[b][t] = make_float2(0.f, 0.f);
-            }
+              for (int t = 0; t < TR; ++t) {
+                acc[b][t].x += (double)a32[b][t].x;
+                acc[b][t].y += (double)a32[b][t].y;
+                a32[b][t] = make_float2(0.f, 0.f);
+              }
+          }
         }
       };
       // The body is a whole number of window periods (TR) and of chunk pairs,

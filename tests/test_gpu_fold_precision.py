@@ -63,3 +63,37 @@ def test_modes_or_nodes_that_are_not_numbers_are_not_taken_as_symmetric(spb, orc
         q = op.compute_q(np.random.default_rng(1).uniform(size=(1, N ** 3))).reshape(N, N, N)
         op.close()
         assert np.isnan(q[3]).all() and np.isnan(q[:, 3]).all() and np.isnan(q[:, :, 3]).all()
+
+
+# The whole table's sum in the FP32-product form (every pair summed for itself, FP32 partial sums of 32 terms, N = 24: of
+# 8), before tables were folded: its error against the FP64 form on the cells below.
+WHOLE_FP32A = {16: {"mp": 1.2498e-7, "self": 2.8476e-7, "pair": 9.050e-8},
+               24: {"mp": 1.0690e-7, "self": 3.1365e-7, "pair": 1.0222e-7},
+               32: {"mp": 1.3538e-7, "self": 3.1936e-7, "pair": 9.084e-8}}
+
+
+def _fp32a_errors(spb, N):
+    from spectralbte_amd import workloads
+    err = {"mp": [], "self": [], "pair": []}
+    for Lv in (5.0, 6.5, 8.0):
+        v, eta = workloads.grid_0d(N, Lv)
+        op = spb.Operator(N, Lv, v, eta)
+        f = workloads.two_maxwellian_ensemble(N, Lv, 64, seed=N)
+        for lam in (0.0, 1.0):
+            op.generate_weights_iso(lam)
+            for name, e in err.items():
+                n = 32 if name == "pair" else 64
+                args = (f[:n], f[n:] if name == "pair" else None)
+                q, ref = (op.compute_q(*args, form=form, maxpreserve=name == "mp") for form in ("fp32a", "fp64"))
+                e.append(np.linalg.norm(q - ref) / np.linalg.norm(ref))
+        op.close()
+    return {name: float(np.exp(np.mean(np.log(e)))) for name, e in err.items()}
+
+
+@pytest.mark.parametrize("N", [16, 24, 32])
+def test_folded_sum_with_fp32_products_is_as_near_as_the_whole_one(spb, N):
+    """A folded product's rounding counts with the weights of all its images; the partial sums are short enough for that."""
+    got = _fp32a_errors(spb, N)
+    print(N, got)
+    for name, e in got.items():
+        assert e <= WHOLE_FP32A[N][name], (name, e)
