@@ -55,3 +55,25 @@ def test_sum_over_the_whole_table_has_its_own_slices(spb, N, n, tile):
     op.set_tile("fp64", False, *tile[:3], kind=tile[3])
     assert np.array_equal(op.qhat(F, G), q)
     op.close()
+
+
+BOTH = [(form, mp) for form in ("fp64", "fp32", "fp16x2") for mp in (False, True)]
+ALL = BOTH + [("fp32a", False), ("fp32a", True)]
+ONE = [(form, False) for form in ("fp64", "fp32", "fp16x2")]
+
+
+@pytest.mark.parametrize("N,tiles", [
+    (16, {(4, 1, 1): BOTH, (4, 1, 2): ALL, (2, 1, 1): BOTH, (1, 1, 1): BOTH, (1, 2, 1): BOTH, (1, 4, 1): BOTH,
+          (4, 4, 2): [("fp64", False)], (4, 4, 1): [("fp64", True)]}),
+    (24, {(3, 3, 1): ALL, (3, 3, 2): ONE + [("fp32a", False), ("fp32a", True)], (4, 2, 1): ALL}),
+    (32, {(8, 2, 1): BOTH, (4, 4, 4): ONE + [("fp32a", False)], (4, 2, 1): BOTH, (4, 1, 1): ONE})])
+def test_streaming_tiles_that_are_there(spb, N, tiles):
+    """The tiles that the folded sums are tested with, for each (form, two products): a test that passes over a refused
+    tile must not do so for one of these."""
+    op, _ = _op(spb, N, 1)
+    for tile, pairs in tiles.items():
+        for form, mp in pairs:
+            op.set_tile(form, mp, *tile, kind=2)
+            assert op.get_tile(1, form, mp) == (2,) + tile
+            op.set_tile(form, mp, 0, 0, 0)
+    op.close()
