@@ -13,6 +13,7 @@
 // of the integral (gain - loss), one thread per entry; any other lam uses a
 // composite 64-panel x 20-point Gauss-Legendre rule per distinct entry.
 #include <hip/hip_runtime.h>
+#include <float.h>
 #include <math.h>
 
 #include <algorithm>
@@ -35,8 +36,10 @@ namespace {
 // entries at N = 16, 1/31 at N = 32.  Generation on an MI355X, before and after:
 // Landau N = 16 160.7 -> 9.1 ms, N = 32 10.67 -> 0.356 s; glance 69.2 -> 11.9 ms, 4.61
 // -> 0.190 s; isotropic with lambda = 0.5 247.5 -> 13.0 ms, 15.8 -> 0.522 s.  (A table
-// of lambda = 0 or 1 in closed form takes 0.4 ms and 19 ms either way and stays as it is.)  Modes of equal absolute value to 1e-12 of the
-// largest count as equal (they differ by the rounding of -L_eta + i h_eta).
+// of lambda = 0 or 1 in closed form takes 0.4 ms and 19 ms either way and stays as it is.)
+// Modes whose absolute values are equal to 8 roundings of the largest count as equal
+// and are computed at their mean (they differ by the rounding of -L_eta + i h_eta, at
+// most 3 roundings on the package's grids).
 struct AxisClasses {
   int na, zero;                       // absolute values; 1 if zero is the first
   int E;                              // signed values
@@ -112,16 +115,22 @@ int with_entries(int N, const double *eta, bool iso, double dfac, double P, doub
     }
     for (int i = 0; i < N && finite; ++i) ex.push_back(fabs(eta[i]));
     std::sort(ex.begin(), ex.end());
+    const double tol = 8 * DBL_EPSILON * emax;
     for (double x : ex)
-      if (A.empty() || x - A.back() > 1e-12 * emax) A.push_back(x);
+      if (A.empty() || x - A.back() > tol) A.push_back(x);  // the smallest of each class
     ax.na = (int)A.size();
-    ax.zero = finite && A[0] <= 1e-12 * emax;
+    ax.zero = finite && A[0] <= tol;
+    std::vector<double> sum(A.size(), 0.0);
+    std::vector<int> members(A.size(), 0);
     for (int i = 0; i < N && finite; ++i) {
       int k = 0;
-      while (k + 1 < ax.na && fabs(eta[i]) - A[k] > 1e-12 * emax) ++k;
+      while (k + 1 < ax.na && fabs(eta[i]) - A[k] > tol) ++k;
       ax.cls[i] = (unsigned char)k;
       ax.sgn[i] = eta[i] < 0 && !(ax.zero && k == 0) ? -1 : 1;
+      sum[k] += fabs(eta[i]) - A[k];
+      ++members[k];
     }
+    for (int k = 0; k < ax.na; ++k) A[k] += sum[k] / members[k];
     ax.E = 2 * ax.na - ax.zero;
     en = {(long)ax.na * (ax.na + 1) * (ax.na + 2) / 6, ax.E, nullptr, nullptr, nullptr, !finite};
     en.direct = en.direct || (double)en.R * ax.E * ax.E * ax.E >= (double)n3 * n3;
