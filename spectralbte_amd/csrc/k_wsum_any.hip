@@ -11,8 +11,8 @@
 //  * Per summed plane the shifted F x-plane of every cell and product is staged
 //    in LDS with every z-line twice in a row: the operand of step cz is at a fixed
 //    offset -cz from the lane's base and never wraps; a lane's TR operands slide by
-//    one entry a step, so they cost one read (N = 18, 160 cells maxPreserve: 1329 us an
-//    evaluation with 3 rows a lane, 3244 with one; N = 10, 75 cells: 76 and 94).
+//    one entry a step, so they cost one read (N = 18, 160 cells maxPreserve: 1376 us an
+//    evaluation with 3 rows a lane, 2357 with one; N = 10, 75 cells: 76 and 83).
 //  * W is column-major over the rows of a plane, padded to whole waves: a wave
 //    reads 64 TR contiguous doubles per column, each value feeding TB cells.  With
 //    N known at compile time a z-line's weights are all loaded before the first is
@@ -20,9 +20,10 @@
 // Measured on an MI355X, the sum alone, against one thread per (row, cell) over the
 // whole table (k_wsum_generic, which still serves operands that are not
 // transforms of real cells, and N > 24, whose staged planes outgrow LDS):
-//   N = 8, 250 cells ComputeQ     209 -> 25 us     N = 12, 300 cells maxPr.   8055 -> 279 us
-//   N = 10, 75 cells maxPreserve  539 -> 30 us     N = 18, 160 cells maxPr.  101.4 -> 1.33 ms
-//   N = 10, one cell maxPreserve  355 -> 11 us     N = 20, 120 cells maxPr.  126.4 -> 2.47 ms
+//   N = 8, 250 cells ComputeQ     209 -> 25 us     N = 12, 300 cells maxPr.   8055 -> 381 us
+//   N = 10, 75 cells maxPreserve  539 -> 36 us     N = 18, 160 cells maxPr.  101.4 -> 1.27 ms
+//   N = 10, one cell maxPreserve  355 -> 12 us     N = 20, 120 cells maxPr.  126.4 -> 2.41 ms
+// (even N under 16 sum all rows, see build_mirror: N = 12 252 and N = 10 27 us with half of them).
 // N = 18 and 160 cells is 21 TFLOP/s of FP64 (64 measured on FMA chains).
 #include <hip/hip_runtime.h>
 #include "spbte_internal.h"
@@ -249,11 +250,12 @@ __global__ void __launch_bounds__(256) k_fold_any(const double *__restrict__ W, 
 
 size_t lds_bytes(int N, int nprod, int tb) { return (size_t)nprod * tb * N * (2 * N + rows_per_lane(N) - 1) * sizeof(double2); }
 
-// Cells per workgroup: two share each weight where one a workgroup gives two waves
-// on every SIMD already, with one product one (N = 8, 250 cells: 46 us an evaluation against 48; fewer, and the slices that make up for it cost more in
-// staging and in the inverse transform's sum) and both cells' planes fit 64 KiB of LDS.
-int any_tb(int N, int npl, int nprod, int ncell) {
-  return ncell >= 2 && (long)npl * (lane_pad(N) / 64) * ncell >= (nprod == 1 ? 1024 : 2048) && lds_bytes(N, nprod, 2) <= 65536 ? 2 : 1;
+// Cells per workgroup: two share each weight where one a workgroup would give a folded
+// table two waves on every SIMD already, with one product one (N = 8, 250 cells: 42 us an
+// evaluation against 47; fewer, and the slices that make up for it cost more in staging
+// and in the inverse transform's sum), and both cells' planes fit 64 KiB of LDS.
+int any_tb(int N, int nprod, int ncell) {
+  return ncell >= 2 && (long)(N / 2 + 1) * (lane_pad(N) / 64) * ncell >= (nprod == 1 ? 1024 : 2048) && lds_bytes(N, nprod, 2) <= 65536 ? 2 : 1;
 }
 
 template <int NT, int TR, int NP>
@@ -291,10 +293,10 @@ extern "C" size_t spbte_any_table_bytes(int N, int npl, int cfold) {
 
 // Slices of the summed z-lines: as many as give 4096 waves (four on every SIMD),
 // each of two lines or more, and at most 48 (the inverse transform adds them).
-// Waves wanted 1024, 2048, 4096, 8192: N = 18, 160 cells maxPreserve 2029, 1586, 1437,
-// 1329 us an evaluation; N = 10, 75 cells 87, 81, 76, 78; N = 8, 250 cells 61, 49, 47, 49.
+// Waves wanted 1024, 2048, 4096, 8192: N = 18, 160 cells maxPreserve 1997, 1550, 1376,
+// 1253 us an evaluation; N = 10, 75 cells 98, 86, 76, 77; N = 8, 250 cells 48, 43, 42, 46.
 extern "C" int spbte_any_slices(int N, int npl, int cfold, int nprod, int ncell) {
-  const int tb = any_tb(N, npl, nprod, ncell);
+  const int tb = any_tb(N, nprod, ncell);
   const long waves = (long)npl * (lane_pad(N) / 64) * ((ncell + tb - 1) / tb);
   const long lines = (cfold ? (N + 1) / 2 : N) * (long)N, most = lines >= 96 ? 48 : (lines >= 4 ? lines / 2 : 1);
   const long want = (4096 + waves - 1) / waves;
@@ -311,7 +313,7 @@ extern "C" int spbte_launch_fold_any(const double *W64, void *dst, int N, int np
 extern "C" int spbte_launch_wsum_any(int N, const spbte_wsum_args *a, const void *Wf, int csplit, void *Qp,
                                      hipStream_t s) {
   if (!spbte_any_supported(N) || csplit < 1 || (csplit > 1 && !Qp)) return (int)hipErrorInvalidValue;
-  const int npl = a->npl, cf = a->cfold, tb = any_tb(N, npl, a->nprod, a->ncell);
+  const int npl = a->npl, cf = a->cfold, tb = any_tb(N, a->nprod, a->ncell);
   switch (N) {
     case 6: launch_np<6, rows_per_lane(6)>(N, npl, cf, tb, a, Wf, csplit, Qp, s); break;
     case 8: launch_np<8, rows_per_lane(8)>(N, npl, cf, tb, a, Wf, csplit, Qp, s); break;
