@@ -378,7 +378,7 @@ const Entry kTable[] = {
     // N = 16: TR=4 -> 16 lanes per line
     E_ALLFORMS(16, 4, 4, 1, 1), E_ALLFORMS(16, 4, 4, 2, 1), E_ALLFORMS(16, 4, 8, 2, 1), E_ALLFORMS(16, 4, 8, 4, 1),
     E_ALLFORMS(16, 4, 4, 1, 2), E_ALLFORMS(16, 4, 4, 2, 2), E_ALLFORMS(16, 4, 8, 2, 2),
-    // N = 8: TR=2 -> 8 lanes per line (reduced forms; FP64 N=8 runs the generic kernel)
+    // N = 8: TR=2 -> 8 lanes per line (reduced forms, over the whole table; FP64 runs k_wsum_any.hip)
     E(8, 2, 8, 2, 1, 1), E(8, 2, 8, 2, 1, 2), E(8, 2, 8, 2, 1, 3), E(8, 2, 8, 2, 2, 1), E(8, 2, 8, 2, 2, 2),
     E(8, 2, 8, 2, 2, 3),
 };

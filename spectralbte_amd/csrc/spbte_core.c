@@ -864,7 +864,8 @@ static int slices_valid(int N, const spbte_tile *t) {
 }
 
 /* Streaming kernel defaults on folded tables, measured on an MI355X (us per
- * evaluation, best of the tiles and splits tried):
+ * evaluation, best of the tiles and splits tried; FP32 products with partial sums of
+ * 8 steps):
  *  N=32 two products: 4 rows x 4 waves (FP64, one cell: 444 against 472 with 8
  *    rows x 2 waves); two cells per lane from 32 cells on with FP64 arithmetic
  *    (128 cells: 16390 against 17440), never with FP32 products (512 cells:
