@@ -34,17 +34,26 @@ namespace {
 // E = 2 na less one if zero is a mode: one more than N for even N, whose mode -N/2
 // has no mirror image), and k_expand writes every entry from its image: 1/21 of the
 // entries at N = 16, 1/31 at N = 32.  Generation on an MI355X, before and after:
-// Landau N = 16 160.7 -> 9.1 ms, N = 32 10.67 -> 0.356 s; glance 69.2 -> 11.9 ms, 4.61
-// -> 0.190 s; isotropic with lambda = 0.5 247.5 -> 13.0 ms, 15.8 -> 0.522 s.  (A table
+// Landau N = 16 160.7 -> 9.9 ms, N = 32 10.67 -> 0.409 s; glance 69.2 -> 11.8 ms, 4.61
+// -> 0.188 s; isotropic with lambda = 0.5 247.5 -> 14.4 ms, 15.8 -> 0.591 s.  (A table
 // of lambda = 0 or 1 in closed form takes 0.4 ms and 19 ms either way and stays as it is.)
 // Modes whose absolute values are equal to 8 roundings of the largest count as equal
 // and are computed at their mean (they differ by the rounding of -L_eta + i h_eta, at
-// most 3 roundings on the package's grids).
+// most 3 roundings on the package's grids).  An entry's phases reach 70, so its own modes
+// matter in the last digits: without the correction the Landau table at N = 10 was
+// 1.5e-15 off where each entry for itself is 6.4e-16, the isotropic one 1.3e-15 and
+// 2.9e-16.  The Landau and isotropic kernels therefore also give the derivatives by
+// |zeta|^2, |xi|^2 and zeta.xi (FP32, for shifts of 1e-16), and k_expand takes every
+// entry to its own modes with them: 6.3e-16 and 2.9e-16, for 1.2 ms of the Landau table
+// and 1.4 ms of the isotropic one at N = 16.  (The glance table is 3e-13 off by its
+// interpolation; its entries stay as they are.)
 struct AxisClasses {
   int na, zero;                       // absolute values; 1 if zero is the first
   int E;                              // signed values
   unsigned char cls[SPBTE_MAX_N];     // class of mode i
   signed char sgn[SPBTE_MAX_N];       // its sign (+1 for zero)
+  double A[SPBTE_MAX_N];              // value of mode i's class
+  float dev[SPBTE_MAX_N];             // |mode i| - that
 };
 __host__ __device__ inline int axis_slot(const AxisClasses &a, int c, int s) {
   return a.zero ? a.na - 1 + s * c : (s > 0 ? a.na + c : a.na - 1 - c);
@@ -59,8 +68,10 @@ __device__ __forceinline__ double iso_entry(int N, int l, int m, int n, double d
 }
 
 // One row r per blockIdx.x: W[r][c] = U[image of r][image of c] (iso: times iso_entry's factors).
-__global__ void __launch_bounds__(256) k_expand(int N, AxisClasses ax, const double *__restrict__ U, bool iso, double dfac,
-                                                double P, double *__restrict__ W) {
+// D, if there: the entries' derivatives by |zeta|^2, |xi|^2 and zeta.xi, n of each.
+__global__ void __launch_bounds__(256) k_expand(int N, AxisClasses ax, const double *__restrict__ U,
+                                                const float *__restrict__ D, size_t n, bool iso, double dfac, double P,
+                                                double *__restrict__ W) {
   const int n2 = N * N, n3 = n2 * N;
   const int r = blockIdx.x, q[3] = {r / n2, r / N % N, r % N};
   int p[3] = {0, 1, 2};  // axes by descending class
@@ -68,20 +79,34 @@ __global__ void __launch_bounds__(256) k_expand(int N, AxisClasses ax, const dou
   if (ax.cls[q[p[1]]] < ax.cls[q[p[2]]]) { const int t = p[1]; p[1] = p[2]; p[2] = t; }
   if (ax.cls[q[p[0]]] < ax.cls[q[p[1]]]) { const int t = p[0]; p[0] = p[1]; p[1] = t; }
   const int E = ax.E;
-  const double *Ur = U + row_rank(ax.cls[q[p[0]]], ax.cls[q[p[1]]], ax.cls[q[p[2]]]) * E * E * E;
-  // slot of every mode on each sorted axis
+  const size_t row = row_rank(ax.cls[q[p[0]]], ax.cls[q[p[1]]], ax.cls[q[p[2]]]) * (size_t)E * E * E;
+  // slot of every mode on each sorted axis; what it adds to the shifts of |xi|^2 and zeta.xi
   __shared__ int slot[3][SPBTE_MAX_N];
+  __shared__ float dx[3][SPBTE_MAX_N], dm[3][SPBTE_MAX_N];
+  float dz = 0.0f;  // shift of |zeta|^2
+#pragma unroll
+  for (int d = 0; d < 3; ++d) dz += 2.0f * (float)ax.A[q[p[d]]] * ax.dev[q[p[d]]];
   for (int e = threadIdx.x; e < 3 * N; e += 256) {
-    const int d = e / N, i = e - d * N;
-    slot[d][i] = axis_slot(ax, ax.cls[i], ax.sgn[q[p[d]]] * ax.sgn[i]);
+    const int d = e / N, i = e - d * N, sg = ax.sgn[q[p[d]]] * ax.sgn[i];
+    slot[d][i] = axis_slot(ax, ax.cls[i], sg);
+    dx[d][i] = 2.0f * (float)ax.A[i] * ax.dev[i];
+    dm[d][i] = sg * ((float)ax.A[q[p[d]]] * ax.dev[i] + (float)ax.A[i] * ax.dev[q[p[d]]]);
   }
   __syncthreads();
   for (int c = threadIdx.x; c < n3; c += 256) {
     const int x[3] = {c / n2, c / N % N, c % N};
     int s[3];
+    float sx = 0.0f, sm = 0.0f;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) s[d] = slot[d][p[d] == 0 ? x[0] : (p[d] == 1 ? x[1] : x[2])];
-    double w = Ur[((long)s[0] * E + s[1]) * E + s[2]];
+    for (int d = 0; d < 3; ++d) {
+      const int i = p[d] == 0 ? x[0] : (p[d] == 1 ? x[1] : x[2]);
+      s[d] = slot[d][i];
+      sx += dx[d][i];
+      sm += dm[d][i];
+    }
+    const size_t u = row + ((size_t)s[0] * E + s[1]) * E + s[2];
+    double w = U[u];
+    if (D) w += (double)(D[u] * dz + D[n + u] * sx + D[2 * n + u] * sm);
     if (iso) w = iso_entry(N, x[0], x[1], x[2], dfac, P, w);
     W[(size_t)r * n3 + c] = w;
   }
@@ -94,13 +119,15 @@ struct Entries {
   int E;
   double *rows, *ex, *out;  // device
   bool direct;              // out is the table itself
+  float *D;                 // three derivatives, n each (asked for, and not direct)
+  size_t n;                 // entries
 };
 
 // Runs compute(Entries) over the distinct entries and writes the table; over the
 // whole table itself (direct: rows and columns are the modes in their order) where
 // the modes are not symmetric (no fewer entries) or there is no room for the rest.
 template <class F>
-int with_entries(int N, const double *eta, bool iso, double dfac, double P, double *W, hipStream_t s, F compute) {
+int with_entries(int N, const double *eta, bool grad, bool iso, double dfac, double P, double *W, hipStream_t s, F compute) {
   const long n3 = (long)N * N * N;
   AxisClasses ax = {};
   std::vector<double> A, ex, rows;
@@ -131,8 +158,12 @@ int with_entries(int N, const double *eta, bool iso, double dfac, double P, doub
       ++members[k];
     }
     for (int k = 0; k < ax.na; ++k) A[k] += sum[k] / members[k];
+    for (int i = 0; i < N && finite; ++i) {
+      ax.A[i] = A[ax.cls[i]];
+      ax.dev[i] = (float)(fabs(eta[i]) - ax.A[i]);
+    }
     ax.E = 2 * ax.na - ax.zero;
-    en = {(long)ax.na * (ax.na + 1) * (ax.na + 2) / 6, ax.E, nullptr, nullptr, nullptr, !finite};
+    en = {(long)ax.na * (ax.na + 1) * (ax.na + 2) / 6, ax.E, nullptr, nullptr, nullptr, !finite, nullptr, 0};
     en.direct = en.direct || (double)en.R * ax.E * ax.E * ax.E >= (double)n3 * n3;
     for (;;) {
       rows.clear();
@@ -154,8 +185,8 @@ int with_entries(int N, const double *eta, bool iso, double dfac, double P, doub
               for (int k : {a, b, c}) rows.push_back(A[k]);
       }
       rows.insert(rows.end(), ex.begin(), ex.end());
-      const size_t nu = en.direct ? 0 : (size_t)en.R * en.E * en.E * en.E;
-      const hipError_t e = hipMalloc((void **)&buf, sizeof(double) * (rows.size() + nu));
+      en.n = en.direct ? 0 : (size_t)en.R * en.E * en.E * en.E;
+      const hipError_t e = hipMalloc((void **)&buf, sizeof(double) * (rows.size() + en.n) + (grad ? 3 * sizeof(float) * en.n : 0));
       if (e == hipSuccess) break;
       if (en.direct) return (int)e;
       (void)hipGetLastError();
@@ -167,10 +198,11 @@ int with_entries(int N, const double *eta, bool iso, double dfac, double P, doub
   en.rows = buf;
   en.ex = buf + 3 * en.R;
   en.out = en.direct ? W : buf + rows.size();
+  en.D = grad && !en.direct ? (float *)(buf + rows.size() + en.n) : nullptr;
   hipError_t e = hipMemcpyAsync(buf, rows.data(), sizeof(double) * rows.size(), hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = (hipError_t)compute(en);
   if (e == hipSuccess && !en.direct) {
-    hipLaunchKernelGGL(k_expand, dim3((unsigned)n3), dim3(256), 0, s, N, ax, en.out, iso, dfac, P, W);
+    hipLaunchKernelGGL(k_expand, dim3((unsigned)n3), dim3(256), 0, s, N, ax, en.out, en.D, en.n, iso, dfac, P, W);
     e = hipGetLastError();
   }
   const hipError_t e2 = hipStreamSynchronize(s), e3 = hipFree(buf);
@@ -220,27 +252,45 @@ struct GL20 {
   double x[20], w[20];
 };
 
-__device__ double integral_gl(double a0, double a1, double a2, double L, double lam, const GL20 &q) {
+// (sin y / y)' / y, sc = sin y / y
+__device__ __forceinline__ float sinc_slope(double y, double sc) {
+  const float x = (float)y;
+  return x < 0.5f ? -1.0f / 3.0f + x * x * (1.0f / 30.0f - x * x / 840.0f) : (cosf(x) - (float)sc) / (x * x);
+}
+
+// g: derivatives by a0^2, a1^2, a2^2
+template <bool GRAD>
+__device__ double integral_gl(double a0, double a1, double a2, double L, double lam, const GL20 &q, float *g) {
   const int panels = 64;
   const double h = L / panels;
   double sum = 0.0;
+  if constexpr (GRAD) g[0] = g[1] = g[2] = 0.0f;
   for (int p = 0; p < panels; ++p) {
     const double lo = p * h;
     double ps = 0.0;
     for (int i = 0; i < 20; ++i) {
       const double r = lo + 0.5 * h * (q.x[i] + 1.0);
-      ps += q.w[i] * pow(r, lam + 2.0) * (sinc(r * a0) * sinc(r * a2) - sinc(r * a1));
+      const double rl = pow(r, lam + 2.0), s0 = sinc(r * a0), s2 = sinc(r * a2), s1 = sinc(r * a1);
+      ps += q.w[i] * rl * (s0 * s2 - s1);
+      if (GRAD && ((p + i) & 1) == 0) {  // every second node, at twice its weight
+        const float w = (float)(0.5 * h * q.w[i] * rl * r * r);
+        g[0] += w * sinc_slope(r * a0, s0) * (float)s2;
+        g[1] -= w * sinc_slope(r * a1, s1);
+        g[2] += w * sinc_slope(r * a2, s2) * (float)s0;
+      }
     }
     sum += 0.5 * h * ps;
   }
   return sum;
 }
 
-// Any other lam: the quadrature alone, over distinct entries.
+// Any other lam: the quadrature alone, over distinct entries.  GRAD: with their
+// derivatives into D (n of each).
+template <bool GRAD>
 __global__ void __launch_bounds__(256) k_weights_iso_gl(int E, const double *__restrict__ rows,
                                                         const double *__restrict__ ex, long r0, long nrows, double L,
                                                         double lam, double mu, GL20 q, bool direct, double dfac,
-                                                        double P, double *__restrict__ out) {
+                                                        double P, double *__restrict__ out, float *__restrict__ D, size_t n) {
   const long n3 = (long)E * E * E;
   const long e = (long)blockIdx.x * 256 + threadIdx.x;
   if (e >= nrows * n3) return;
@@ -249,8 +299,14 @@ __global__ void __launch_bounds__(256) k_weights_iso_gl(int E, const double *__r
   const double k1 = ex[c / ((long)E * E)], k2 = ex[(c / E) % E], k3 = ex[c % E];
   const double a0 = mu * sqrt(z1 * z1 + z2 * z2 + z3 * z3), a1 = sqrt(k1 * k1 + k2 * k2 + k3 * k3);
   const double d1 = k1 - mu * z1, d2 = k2 - mu * z2, d3 = k3 - mu * z3;
-  const double I = integral_gl(a0, a1, sqrt(d1 * d1 + d2 * d2 + d3 * d3), L, lam, q);
+  float g[3];
+  const double I = integral_gl<GRAD>(a0, a1, sqrt(d1 * d1 + d2 * d2 + d3 * d3), L, lam, q, g);
   out[e] = direct ? iso_entry(E, (int)(c / ((long)E * E)), (int)((c / E) % E), (int)(c % E), dfac, P, I) : I;
+  if constexpr (GRAD) {  // a0^2 = mu^2 |zeta|^2, a1^2 = |xi|^2, a2^2 = |xi|^2 - 2 mu zeta.xi + mu^2 |zeta|^2
+    D[e] = (float)(mu * mu) * (g[0] + g[2]);
+    D[n + e] = g[1] + g[2];
+    D[2 * n + e] = (float)(-2.0 * mu) * g[2];
+  }
 }
 
 __global__ void __launch_bounds__(256) k_weights_iso(int N, const double *__restrict__ eta, double L, double lam, double P,
@@ -324,9 +380,49 @@ __device__ __forceinline__ double landau_g(double r, double a0, double a1, doubl
   return st * j0(r * a0 * st) * (-r * r * a1 * st * st * cv + 4 * r * a3 * sv * ct);
 }
 
+// J0(x) and J1(x) / x to 1e-3: power series, and Hankel's expansion in modulus and phase.
+__device__ __forceinline__ void bessel01(float x, float &j0x, float &j1x) {
+  if (x < 3.0f) {
+    const float y = 0.25f * x * x;
+    j0x = 1 - y * (1 - y / 4 * (1 - y / 9 * (1 - y / 16 * (1 - y / 25 * (1 - y / 36)))));
+    j1x = 0.5f * (1 - y / 2 * (1 - y / 6 * (1 - y / 12 * (1 - y / 20 * (1 - y / 30 * (1 - y / 42))))));
+    return;
+  }
+  const float t = 1.0f / x, m = sqrtf(0.63661977f * t);
+  j0x = m * (1.0f - 0.0625f * t * t) * __cosf(x - 0.78539816f - t * (0.125f - 0.06510417f * t * t));
+  j1x = m * t * (1.0f + 0.1875f * t * t) * __cosf(x - 2.35619449f + t * (0.375f - 0.1640625f * t * t));
+}
+
+// Derivatives of an entry by a0^2, a1, a2 and a3, in FP32 from every fourth node of the
+// double rule at four times its weight, chequered over both (the nodes of half a Gauss
+// rule at twice their weights are a rule of half the density): for corrections of 1e-15
+// of an entry, whose error it takes to that of the entry for itself (N=16 1.5e-15, N=10
+// 6e-16, as with every node).
+__device__ void landau_grad(const LandauRule &q, float a0, float a1, float a2, float a3, float (&d)[4]) {
+  d[0] = d[1] = d[2] = d[3] = 0.0f;
+  for (int i = 0; i < 32; ++i)
+    for (int h = 0; h < 2; ++h) {
+      const float r = (float)(h ? q.r_m[i] : q.r_p[i]);
+      const float wr = (float)(16.0 * M_PI * q.Ar * q.At * q.w[i] * (h ? q.rl_m[i] : q.rl_p[i]));
+      for (int k = (2 * h - i) & 3; k < 32; k += 4) {
+        const float st = (float)q.st[k], ct = (float)q.ct[k], f = wr * (float)q.w[k] * st, rs = r * st;
+        float sv, cv, j, j1x;
+        __sincosf(r * a2 * ct, &sv, &cv);
+        bessel01(rs * a0, j, j1x);
+        // J0(rs sqrt(u))' by u = a0^2 is -rs^2 J1(x) / (2 x)
+        d[0] -= f * 0.5f * rs * rs * j1x * (-rs * rs * a1 * cv + 4.0f * r * a3 * sv * ct);
+        const float fj = f * j;
+        d[1] -= fj * rs * rs * cv;
+        d[2] += fj * r * ct * (rs * rs * a1 * sv + 4.0f * r * a3 * ct * cv);
+        d[3] += fj * 4.0f * r * ct * sv;
+      }
+    }
+}
+
+template <bool GRAD>
 __global__ void __launch_bounds__(256) k_weights_landau(int N, const double *__restrict__ rows,
                                                         const double *__restrict__ eta, long r0, long nrows,
-                                                        LandauRule q, double *__restrict__ W) {
+                                                        LandauRule q, double *__restrict__ W, float *__restrict__ D, size_t n) {
   const long n3 = (long)N * N * N;
   const long e = (long)blockIdx.x * 256 + threadIdx.x;
   if (e >= nrows * n3) return;
@@ -353,6 +449,17 @@ __global__ void __launch_bounds__(256) k_weights_landau(int N, const double *__r
     sr += q.w[i] * (f[0] + f[1]);
   }
   W[(r - r0) * n3 + c] = 2.0 * M_PI * (q.Ar * sr);
+  if constexpr (GRAD) {
+    float g[4];
+    landau_grad(q, (float)a0, (float)zetalen2, (float)a2, (float)zetalen, g);
+    // a0^2 = |xi|^2 - m^2/p, a1 = p, a2 = m / sqrt(p), a3 = sqrt(p) with p = |zeta|^2, m = zeta.xi;
+    // the row of the zero mode is zero
+    const float p = (float)zetalen2, m = (float)xizeta, z = (float)zetalen, t = p > 1e-20f ? m / p : 0.0f;
+    const float zi = p > 1e-20f ? 1.0f / z : 0.0f;
+    D[e] = g[1] + 0.5f * g[3] * zi - 0.5f * g[2] * t * zi + g[0] * t * t;
+    D[n + e] = g[0];
+    D[2 * n + e] = g[2] * zi - 2.0f * g[0] * t;
+  }
 }
 
 // n-point Gauss-Legendre rule: the n/2 positive nodes ascending and their
@@ -396,14 +503,19 @@ extern "C" int spbte_launch_weights_landau(const spbte_grid_dev *g, const double
     q.rl_p[k] = pow(q.r_p[k], lam + 2);
     q.rl_m[k] = pow(q.r_m[k], lam + 2);
   }
-  return with_entries(g->N, eta_host, false, 0.0, 0.0, W, s, [&](const Entries &en) {
+  return with_entries(g->N, eta_host, true, false, 0.0, 0.0, W, s, [&](const Entries &en) {
     const long n3 = (long)en.E * en.E * en.E;
     // rows per launch: about 8M entries
     const long rows = n3 >= (8L << 20) ? 1 : (8L << 20) / n3;
     for (long r0 = 0; r0 < en.R; r0 += rows) {
       const long nr = r0 + rows <= en.R ? rows : en.R - r0;
       const unsigned blocks = (unsigned)((nr * n3 + 255) / 256);
-      hipLaunchKernelGGL(k_weights_landau, dim3(blocks), dim3(256), 0, s, en.E, en.rows, en.ex, r0, nr, q, en.out + r0 * n3);
+      if (en.D)
+        hipLaunchKernelGGL(k_weights_landau<true>, dim3(blocks), dim3(256), 0, s, en.E, en.rows, en.ex, r0, nr, q,
+                           en.out + r0 * n3, en.D + r0 * n3, en.n);
+      else
+        hipLaunchKernelGGL(k_weights_landau<false>, dim3(blocks), dim3(256), 0, s, en.E, en.rows, en.ex, r0, nr, q,
+                           en.out + r0 * n3, nullptr, 0);
       const hipError_t e = hipGetLastError();
       if (e != hipSuccess) return (int)e;
     }
@@ -733,7 +845,7 @@ extern "C" int spbte_launch_weights_glance(const spbte_grid_dev *g, const double
   if (e != hipSuccess) return (int)e;
   e = hipMemcpy(drule, buf.data(), bytes, hipMemcpyHostToDevice);
   if (e == hipSuccess)
-    e = (hipError_t)with_entries(N, eta_host, false, 0.0, 0.0, W, s, [&](const Entries &en) {
+    e = (hipError_t)with_entries(N, eta_host, false, false, 0.0, 0.0, W, s, [&](const Entries &en) {
       // rows per launch: about 4M entries
       const long n3 = (long)en.E * en.E * en.E, rows = n3 >= (4L << 20) ? 1 : (4L << 20) / n3;
       for (long r0 = 0; r0 < en.R; r0 += rows) {
@@ -758,12 +870,17 @@ extern "C" int spbte_launch_weights_iso(const spbte_grid_dev *g, const double *e
   if (lam != 0.0 && lam != 1.0) {
     GL20 q;
     gauss_legendre20(q);
-    return with_entries(N, eta_host, true, dfac, P, W, s, [&](const Entries &en) {
+    return with_entries(N, eta_host, true, true, dfac, P, W, s, [&](const Entries &en) {
       const long m3 = (long)en.E * en.E * en.E, rows = m3 >= (8L << 20) ? 1 : (8L << 20) / m3;
       for (long r0 = 0; r0 < en.R; r0 += rows) {
         const long nr = r0 + rows <= en.R ? rows : en.R - r0;
-        hipLaunchKernelGGL(k_weights_iso_gl, dim3((unsigned)((nr * m3 + 255) / 256)), dim3(256), 0, s, en.E, en.rows,
-                           en.ex, r0, nr, g->Lv, lam, mu, q, en.direct, dfac, P, en.out + r0 * m3);
+        const dim3 blocks((unsigned)((nr * m3 + 255) / 256));
+        if (en.D)
+          hipLaunchKernelGGL(k_weights_iso_gl<true>, blocks, dim3(256), 0, s, en.E, en.rows, en.ex, r0, nr, g->Lv, lam, mu,
+                             q, en.direct, dfac, P, en.out + r0 * m3, en.D + r0 * m3, en.n);
+        else
+          hipLaunchKernelGGL(k_weights_iso_gl<false>, blocks, dim3(256), 0, s, en.E, en.rows, en.ex, r0, nr, g->Lv, lam, mu,
+                             q, en.direct, dfac, P, en.out + r0 * m3, nullptr, 0);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return (int)e;
       }
